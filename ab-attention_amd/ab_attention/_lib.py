@@ -26,6 +26,19 @@ _P = ctypes.c_void_p
 _I64 = ctypes.c_int64
 _SZ = ctypes.c_size_t
 
+
+
+PREFILL_DENSE = -1  # AB_PREFILL_DENSE
+
+
+class PrefillArgs(ctypes.Structure):
+    """ab_prefill_args of include/ab_attention.h."""
+
+    _fields_ = [("q", _P), ("k", _P), ("v", _P), ("order", _P), ("ids", _P), ("log_weights", _P), ("out", _P),
+                ("lse", _P), ("batch_heads", _I64), ("q_tokens", _I64), ("kv_tokens", _I64), ("samples", _I64),
+                ("workspace", _P), ("workspace_bytes", _SZ)]
+
+
 # name -> (restype, argtypes); mirrors include/ab_attention.h
 SIGNATURES = {
     "ab_last_error": (ctypes.c_char_p, []),
@@ -48,6 +61,8 @@ SIGNATURES = {
     "ab_ibcs_sip_exact_draws": (ctypes.c_int, [_P, _P, _P, _I64, _I64, _P, _I64, _P, _SZ, _P, _P, _P]),
     "ab_dense_prefill": (ctypes.c_int, [_P, _P, _P, _I64, _I64, _I64, _P, _P, _P]),
     "ab_prefill_launch_slots": (_I64, [_I64, _I64]),
+    "ab_prefill_workspace_bytes": (_SZ, [_I64, _I64, _I64, _I64]),
+    "ab_prefill": (ctypes.c_int, [ctypes.POINTER(PrefillArgs), _P]),
 }
 
 # name -> (restype, argtypes); mirrors include/ab_attention_static.h
@@ -55,7 +70,7 @@ STATIC_SIGNATURES = {
     "ab_ibcs_sip_static": (ctypes.c_int, [_P, _P, _P, _I64, _I64, _P, _I64, _P, _P, _P]),
 }
 
-ABI_VERSION = 4
+ABI_VERSION = 5
 _lib = None
 _static = None
 

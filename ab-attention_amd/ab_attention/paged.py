@@ -2,13 +2,13 @@
 
 ``paged_attention`` keeps the reference's signature, validation (ValueError)
 and output/LSE layout (ab_attention/flashinfer_backend.py:164-242). The
-arithmetic is ``ab_paged_prefill_kv`` in libab_attention_hip.so: a bf16 MFMA
+arithmetic is ``ab_prefill`` in libab_attention_hip.so: a bf16 MFMA
 flash-attention kernel that reads each row's KV4 blocks straight from K and
 V by their per-head ids and adds the SIP weight of each block to its logits
 (the reference's ABSipAttention variant, flashinfer_backend.py:30-59).
 ``_prefill_dense`` runs the library's dense attention kernel, which walks
 every KV4 block of K/V at weight 0 with no page list in memory
-(ab_dense_prefill; the same rings and pipeline on 16x16x32 MFMA tiles).
+(the same rings and pipeline on 16x16x32 MFMA tiles).
 
 The reference translates per-head ids into a global page table and caches it
 per descriptor (flashinfer_backend.py:62-74, :202-217); the kernel here
@@ -30,29 +30,33 @@ _QUERY_BLOCK = 128
 _PAGE_SIZE = 4
 
 
+def _run(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, ids, weights, samples: int, order, return_lse: bool):
+    """ab_prefill of row-major q, k, v (samples: _lib.PREFILL_DENSE for dense). The workspace of a
+    call that splits its rows over more workgroups lives for the call only (the
+    caching allocator keeps it on this stream)."""
+    batch, heads, tokens, _ = q.shape
+    kv_tokens, device = k.shape[2], q.device
+    output = torch.empty_like(q)
+    lse = torch.empty((batch, heads, tokens), dtype=torch.float32, device=device) if return_lse else None
+    lib = _lib.load()
+    with torch.cuda.device(device):
+        ws_bytes = lib.ab_prefill_workspace_bytes(batch * heads, tokens, kv_tokens, samples)
+        workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=device) if ws_bytes else None
+        args = _lib.PrefillArgs(_lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(order), _lib.ptr(ids),
+                                _lib.ptr(weights), _lib.ptr(output), _lib.ptr(lse), batch * heads, tokens, kv_tokens,
+                                samples, _lib.ptr(workspace), ws_bytes)
+        _lib.check(lib.ab_prefill(args, _lib.stream(device)))
+    return (output, lse) if return_lse else output
+
+
 def _prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor,
              order: torch.Tensor | None, return_lse: bool):
-    """The weighted prefill of row-major q, k, v: ab_paged_prefill_kv, or
-    ab_paged_prefill_ordered when a query token order is given; ids/weights
-    [rows, S]. Shapes are checked by the callers."""
-    batch, heads, tokens, _ = q.shape
+    """The weighted prefill, with a query token order when one is given;
+    ids/weights [rows, S]. Shapes are checked by the callers."""
     q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
     ids = ids.to(torch.int32).contiguous()
     weights = weights.to(torch.float32).contiguous()
-    output = torch.empty_like(q)
-    lse = torch.empty((batch, heads, tokens), dtype=torch.float32, device=q.device) if return_lse else None
-    lib = _lib.load()
-    with torch.cuda.device(q.device):
-        if order is None:
-            rc = lib.ab_paged_prefill_kv(
-                _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), batch * heads, tokens, k.shape[2], _lib.ptr(ids),
-                _lib.ptr(weights), ids.shape[-1], _lib.ptr(output), _lib.ptr(lse), _lib.stream(q.device))
-        else:
-            rc = lib.ab_paged_prefill_ordered(
-                _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(order), batch * heads, tokens, _lib.ptr(ids),
-                _lib.ptr(weights), ids.shape[-1], _lib.ptr(output), _lib.ptr(lse), _lib.stream(q.device))
-        _lib.check(rc)
-    return (output, lse) if return_lse else output
+    return _run(q, k, v, ids, weights, ids.shape[-1], order, return_lse)
 
 
 def check_prefill_inputs(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> None:
@@ -111,15 +115,7 @@ def _prefill_dense(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, return_
     [B,H,Nk,128] (Nk % 4 == 0) on the dense kernel (ab_dense_prefill); the
     page list is implicit, so nothing of size rows x blocks is built. Shapes
     are checked by the callers."""
-    batch, heads, tokens, _ = q.shape
-    q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
-    output = torch.empty_like(q)
-    lse = torch.empty((batch, heads, tokens), dtype=torch.float32, device=q.device) if return_lse else None
-    lib = _lib.load()
-    with torch.cuda.device(q.device):
-        _lib.check(lib.ab_dense_prefill(_lib.ptr(q), _lib.ptr(k), _lib.ptr(v), batch * heads, tokens, k.shape[2],
-                                        _lib.ptr(output), _lib.ptr(lse), _lib.stream(q.device)))
-    return (output, lse) if return_lse else output
+    return _run(q.contiguous(), k.contiguous(), v.contiguous(), None, None, _lib.PREFILL_DENSE, None, return_lse)
 
 
 def _remap_ids(ids: torch.Tensor, page_map: torch.Tensor) -> torch.Tensor:

@@ -34,7 +34,8 @@ int launch_sip_fused(const void* lse, const float* pops, const float* lse_max, c
                      float* logw, int force_exact, hipStream_t stream);
 int launch_prefill(const void* q, const void* k, const void* v, bool dense, int64_t bh, int64_t n, int64_t n_kv,
                    const int32_t* ids, const float* logw, int64_t samples, void* out, float* lse,
-                   const int32_t* order, hipStream_t stream);
+                   const int32_t* order, void* workspace, hipStream_t stream);
+size_t prefill_workspace_bytes(bool dense, int64_t bh, int64_t n, int64_t n_kv, int64_t samples);
 int64_t prefill_launch_slots(int64_t bh, int64_t n);
 int launch_remap_ids(const int32_t* ids, int64_t count, const int32_t* map, int64_t map_len, int32_t* out,
                      hipStream_t stream);
@@ -336,7 +337,8 @@ namespace {
 // K/V at weight 0 (ids and log_weights are not read; samples is derived).
 int paged_prefill_checked(const void* q, const void* k, const void* v, bool dense, const int32_t* order,
                           int64_t batch_heads, int64_t q_tokens, int64_t kv_tokens, const int32_t* ids,
-                          const float* log_weights, int64_t samples, void* out, float* lse, void* stream) {
+                          const float* log_weights, int64_t samples, void* out, float* lse, void* workspace,
+                          size_t workspace_bytes, void* stream) {
     if (batch_heads <= 0 || q_tokens <= 0 || kv_tokens <= 0)
         return set_error(AB_ERR_INVALID, "paged_prefill: batch_heads and token counts must be positive");
     if (kv_tokens % kKvBlock)
@@ -356,8 +358,16 @@ int paged_prefill_checked(const void* q, const void* k, const void* v, bool dens
         return set_error(AB_ERR_INVALID, "paged_prefill: ids and log_weights must be 16-byte aligned");
     const int64_t rows = batch_heads * qb;
     if (rows * samples > (int64_t(1) << 40)) return set_error(AB_ERR_INVALID, "paged_prefill: plan too large");
+    if (workspace) {
+        const size_t need = prefill_workspace_bytes(dense, batch_heads, q_tokens, kv_tokens, samples);
+        if (workspace_bytes < need)
+            return set_error(AB_ERR_INVALID, "paged_prefill: workspace of %zu bytes is smaller than the %zu required",
+                             workspace_bytes, need);
+        if (!aligned16(workspace))
+            return set_error(AB_ERR_INVALID, "paged_prefill: workspace must be 16-byte aligned");
+    }
     return launch_prefill(q, k, v, dense, batch_heads, q_tokens, kv_tokens, ids, log_weights, samples, out, lse,
-                          order, static_cast<hipStream_t>(stream));
+                          order, workspace, static_cast<hipStream_t>(stream));
 }
 }  // namespace
 
@@ -365,13 +375,28 @@ int ab_paged_prefill_kv(const void* q, const void* k, const void* v, int64_t bat
                         int64_t kv_tokens, const int32_t* ids, const float* log_weights, int64_t samples,
                         void* out, float* lse, void* stream) {
     return paged_prefill_checked(q, k, v, false, nullptr, batch_heads, q_tokens, kv_tokens, ids, log_weights,
-                                 samples, out, lse, stream);
+                                 samples, out, lse, nullptr, 0, stream);
 }
 
 int ab_dense_prefill(const void* q, const void* k, const void* v, int64_t batch_heads, int64_t q_tokens,
                      int64_t kv_tokens, void* out, float* lse, void* stream) {
     return paged_prefill_checked(q, k, v, true, nullptr, batch_heads, q_tokens, kv_tokens, nullptr, nullptr, 0,
-                                 out, lse, stream);
+                                 out, lse, nullptr, 0, stream);
+}
+
+size_t ab_prefill_workspace_bytes(int64_t batch_heads, int64_t q_tokens, int64_t kv_tokens, int64_t samples) {
+    const bool dense = samples == AB_PREFILL_DENSE;
+    if (dense) samples = (kv_tokens / kKvBlock + 7) / 8 * 8;
+    if (batch_heads <= 0 || q_tokens <= 0 || kv_tokens <= 0 || samples <= 0) return 0;
+    return prefill_workspace_bytes(dense, batch_heads, q_tokens, kv_tokens, samples);
+}
+
+int ab_prefill(const ab_prefill_args* a, void* stream) {
+    if (!a) return set_error(AB_ERR_INVALID, "paged_prefill: null pointer");
+    const bool dense = a->samples == AB_PREFILL_DENSE;
+    return paged_prefill_checked(a->q, a->k, a->v, dense, a->order, a->batch_heads, a->q_tokens, a->kv_tokens,
+                                 a->ids, a->log_weights, a->samples, a->out, a->lse, a->workspace,
+                                 a->workspace_bytes, stream);
 }
 
 int ab_paged_prefill_ordered(const void* q, const void* k, const void* v, const int32_t* order,
@@ -382,7 +407,7 @@ int ab_paged_prefill_ordered(const void* q, const void* k, const void* v, const 
     if (samples <= 0 || samples % kBlocksPerPage)
         return set_error(AB_ERR_INVALID, "paged_prefill: samples must be a positive multiple of 32");
     return paged_prefill_checked(q, k, v, false, order, batch_heads, tokens, tokens, ids, log_weights, samples,
-                                 out, lse, stream);
+                                 out, lse, nullptr, 0, stream);
 }
 
 int64_t ab_prefill_launch_slots(int64_t batch_heads, int64_t q_tokens) {

@@ -56,6 +56,9 @@
 // Dense attention (every KV4 block at weight 0, no page list) runs on
 // dense_kernel: the same rings, pipeline and two passes on
 // v_mfma_f32_16x16x32_bf16 tiles (see there).
+// Calls with too few rows to fill the chip split each row's tiles over several
+// workgroups (kSplit, prefill_parts), whose float32 partial results
+// combine_kernel adds up.
 #include <algorithm>
 #include <type_traits>
 
@@ -79,6 +82,12 @@ constexpr int kVoteOffset = kWeightsOffset + 2 * kBatchBytes;  // 4 words: fast-
 constexpr int kLdsBytes = kVoteOffset + 16;                    // 72 KiB + 16 B
 constexpr int kGroupOps = 4;                                   // transfers per wave per step
 constexpr int64_t kRowsPerLaunch = 11000;                      // see launch_prefill
+// Limits of a split (prefill_parts): units that give each CU one workgroup (at
+// most twice that many are made: 33 MiB of workspace), parts of a row and the
+// fewest tiles of a part.
+constexpr int64_t kPartUnits = 256;
+constexpr int64_t kMaxParts = 64;
+constexpr int64_t kMinPartTiles = 8;
 // Largest p = 2^(y) allowed before the running reference is moved.
 constexpr float kSlack = 8.0f;
 // Largest logit above the first tile's maximum that the fast pass accepts:
@@ -178,16 +187,66 @@ __device__ __forceinline__ bool row_slot(int64_t slot_base, int64_t qb, int64_t 
     return true;
 }
 
+// The same for rows split into `parts` units each: unit (bh, part, blk), blk
+// fastest, each XCD a contiguous eighth of the units. The units of one part
+// of a head read the same stretch of its K/V (dense) or sweep the same range
+// of their ascending page lists (sparse), so they share it in the XCD's L2.
+// `unit` numbers the unit's partial result.
+struct UnitSlot : RowSlot {
+    int64_t unit;
+    int part;
+};
+__device__ __forceinline__ bool unit_slot(int64_t qb, int64_t rows, int parts, UnitSlot& us) {
+    const int64_t units = rows * parts, per_xcd = (units + 7) / 8;
+    const int64_t hw = blockIdx.x;
+    us.unit = (hw & 7) * per_xcd + (hw >> 3);
+    if ((hw >> 3) >= per_xcd || us.unit >= units) return false;
+    us.blk = us.unit % qb;
+    us.part = static_cast<int>((us.unit / qb) % parts);
+    us.bh = us.unit / (qb * parts);
+    us.row = us.bh * qb + us.blk;
+    return true;
+}
+// Tiles [first, first + count) of part `part` of `parts` (parts <= tiles, so
+// none is empty).
+__device__ __forceinline__ void part_tiles(int tiles, int parts, int part, int& first, int& count) {
+    first = static_cast<int>(int64_t(tiles) * part / parts);
+    count = static_cast<int>(int64_t(tiles) * (part + 1) / parts) - first;
+}
+
+// Partial results of the split kernels, in the caller's workspace: per unit
+// the unnormalised O of its 128 queries as 16 fragments of four consecutive
+// dims per thread (fragment, thread), 64 KiB, so every store and load is a
+// coalesced 16 bytes per lane; then per unit and query (reference m, sum l),
+// m = -inf for a query without a finite logit in the unit.
+constexpr int kFragments = 16;
+constexpr int kCombineFragments = 2;  // fragments per workgroup of combine_kernel
+struct Partials {
+    f32x4* o;      // [units][kFragments][kPfThreads]
+    float2* stat;  // [units][kQueryBlock]
+    int parts;
+};
+
 // The sparse prefill: the row's listed KV4 blocks, with their log weights.
+// kSplit: one part of the row's tiles, its result left in `partials`.
+template <bool kSplit>
 __global__ __launch_bounds__(kPfThreads, 2) void prefill_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
     const int32_t* __restrict__ ids, const float* __restrict__ logw, uint16_t* __restrict__ out,
-    float* __restrict__ lse, int64_t n, int64_t n_kv, int64_t qb, int64_t rows, int fb, int samples,
-    float scale_log2, const int32_t* __restrict__ order, int64_t slot_base) {
+    float* __restrict__ lse, int64_t n, int64_t n_kv, int64_t qb, int64_t rows, int fb, int row_samples,
+    float scale_log2, const int32_t* __restrict__ order, int64_t slot_base, Partials partials) {
     extern __shared__ __align__(16) unsigned char smem[];
 
-    RowSlot rs;
-    if (!row_slot(slot_base, qb, rows, rs)) return;
+    UnitSlot rs;
+    int tile0 = 0, samples = row_samples;
+    if constexpr (kSplit) {
+        if (!unit_slot(qb, rows, partials.parts, rs)) return;
+        int count;
+        part_tiles(row_samples / kTilePages, partials.parts, rs.part, tile0, count);
+        samples = count * kTilePages;
+    } else {
+        if (!row_slot(slot_base, qb, rows, rs)) return;
+    }
     const int64_t bh = rs.bh, blk = rs.blk, row = rs.row;
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -213,8 +272,8 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_kernel(
     }
 
     const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_u8*)smem));
-    const int32_t* row_ids = ids + row * int64_t(samples);
-    const float* row_w = logw + row * int64_t(samples);
+    const int32_t* row_ids = ids + row * int64_t(row_samples) + tile0 * kTilePages;
+    const float* row_w = logw + row * int64_t(row_samples) + tile0 * kTilePages;
     const uint16_t* kbase = k + bh * n_kv * kHeadDim;
     const uint16_t* vbase = v + bh * n_kv * kHeadDim;
 
@@ -520,6 +579,18 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_kernel(
 
     const auto lsw = __builtin_amdgcn_permlane32_swap(__float_as_uint(l_run), __float_as_uint(l_run), false, false);
     const float l_tot = __uint_as_float(lsw[0]) + __uint_as_float(lsw[1]);
+    if constexpr (kSplit) {
+        f32x4* dst = partials.o + rs.unit * (kFragments * kPfThreads) + tid;
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+                dst[(4 * dt + g) * kPfThreads] = f32x4{o_acc[dt][4 * g], o_acc[dt][4 * g + 1], o_acc[dt][4 * g + 2],
+                                                       o_acc[dt][4 * g + 3]};
+        if (half == 0)
+            partials.stat[rs.unit * kQueryBlock + wave * 32 + qi] = float2{started ? m_run : -INFINITY, l_tot};
+        return;
+    }
     if (valid_q) {
         // A query whose every listed block has weight -inf gets o = 0 and
         // lse = -inf.
@@ -563,19 +634,25 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_kernel(
 // addresses): the four 16-lane groups of a transposing read fetch the same
 // dim block of four different pages, which then fall in opposite halves of
 // the banks.
+template <bool kSplit>
 __global__ __launch_bounds__(kPfThreads, 2) void dense_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
     uint16_t* __restrict__ out, float* __restrict__ lse, int64_t n, int64_t n_kv, int64_t qb, int64_t rows, int fb,
-    int samples, float scale_log2, int64_t slot_base) {
+    int samples, float scale_log2, int64_t slot_base, Partials partials) {
     extern __shared__ __align__(16) unsigned char smem[];
-    RowSlot rs;
-    if (!row_slot(slot_base, qb, rows, rs)) return;
+    UnitSlot rs;
+    int tile0 = 0, tiles = samples / kTilePages;
+    if constexpr (kSplit) {
+        if (!unit_slot(qb, rows, partials.parts, rs)) return;
+        part_tiles(samples / kTilePages, partials.parts, rs.part, tile0, tiles);
+    } else {
+        if (!row_slot(slot_base, qb, rows, rs)) return;
+    }
     const int64_t bh = rs.bh, blk = rs.blk;
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, lg = lane >> 4;
-    const int tiles = samples / kTilePages;
     auto token_of = [&](int j) { return blk * kQueryBlock + wave * 32 + 16 * j + li; };
 
     // Q as the B operand of S^T = K Q^T: query 16j + li, dims 32ks + 8lg .. +8.
@@ -614,7 +691,7 @@ __global__ __launch_bounds__(kPfThreads, 2) void dense_kernel(
     // row's end read its last tile (their transfers only keep the per-step
     // count uniform).
     auto load_ids = [&](int u) {
-        const int id = min(u, tiles - 1) * kTilePages + 2 * wave;
+        const int id = (tile0 + min(u, tiles - 1)) * kTilePages + 2 * wave;
         const u32x2 c = {uint32_t(min(id, fb - 1)), uint32_t(min(id + 1, fb - 1))};
         return c;
     };
@@ -627,7 +704,7 @@ __global__ __launch_bounds__(kPfThreads, 2) void dense_kernel(
     // The weights of this lane's keys in tile u: pages lg and 4 + lg, 0 inside
     // K/V and -inf past its end.
     auto load_weights = [&](int u, float (&wv)[2]) {
-        const int uc = min(u, tiles - 1);
+        const int uc = tile0 + min(u, tiles - 1);
 #pragma unroll
         for (int kt = 0; kt < 2; ++kt) wv[kt] = uc * kTilePages + 4 * kt + lg < fb ? 0.f : -INFINITY;
     };
@@ -892,6 +969,15 @@ __global__ __launch_bounds__(kPfThreads, 2) void dense_kernel(
         const auto s32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(l16), __float_as_uint(l16), false, false);
         const float l_tot = __uint_as_float(s32[0]) + __uint_as_float(s32[1]);
         const int64_t token = token_of(j);
+        if constexpr (kSplit) {
+            f32x4* dst = partials.o + rs.unit * (kFragments * kPfThreads) + tid;
+#pragma unroll
+            for (int dt = 0; dt < 8; ++dt) dst[(2 * dt + j) * kPfThreads] = o_acc[dt][j];
+            if (lg == 0)
+                partials.stat[rs.unit * kQueryBlock + wave * 32 + 16 * j + li] =
+                    float2{thr[j] == kSlack ? m_run[j] : -INFINITY, l_tot};
+            continue;
+        }
         if (token < n) {
             // A query whose every block has weight -inf (none here while K/V
             // is not empty) gets o = 0 and lse = -inf.
@@ -905,6 +991,77 @@ __global__ __launch_bounds__(kPfThreads, 2) void dense_kernel(
             }
             if (lse != nullptr && lg == 0) lse[bh * n + token] = thr[j] == kSlack ? m_run[j] + log2f(l_tot) : -INFINITY;
         }
+    }
+}
+
+// Sum of a row's partial results: m = max over its parts, w_p = 2^(m_p - m),
+// o = sum w_p o_p / sum w_p l_p, in float32, rounded to bf16 once. Bound by
+// reading the partials (64 KiB per unit) or, for few rows, by the latency of
+// its loads: workgroup (row, y) takes fragments 2y and 2y + 1, so one row
+// spreads over eight workgroups, and the loads of eight parts are in flight
+// together. Thread t holds the fragments thread t of the split kernel stored
+// (kDense: its layout).
+template <bool kDense>
+__global__ __launch_bounds__(kPfThreads) void combine_kernel(Partials partials, int64_t qb, int64_t n,
+                                                             uint16_t* __restrict__ out, float* __restrict__ lse,
+                                                             const int32_t* __restrict__ order) {
+    constexpr int kQueries = kDense ? 2 : 1;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int64_t row = blockIdx.x, bh = row / qb, blk = row % qb;
+    const int64_t unit0 = bh * partials.parts * qb + blk;  // part p: unit0 + p * qb
+    const int f0 = blockIdx.y * kCombineFragments;
+    // Query of the thread's fragment f: 16 (f % 2) + lane % 16 (dense) or lane % 32 of the wave's 32.
+    int query[kQueries];
+    float m[kQueries], total[kQueries];
+#pragma unroll
+    for (int j = 0; j < kQueries; ++j) {
+        query[j] = wave * 32 + (kDense ? 16 * j + (lane & 15) : lane & 31);
+        m[j] = -INFINITY;
+        total[j] = 0.f;
+    }
+#pragma unroll 8
+    for (int p = 0; p < partials.parts; ++p)
+#pragma unroll
+        for (int j = 0; j < kQueries; ++j)
+            m[j] = fmaxf(m[j], partials.stat[(unit0 + p * qb) * kQueryBlock + query[j]].x);
+    f32x4 acc[kCombineFragments];
+#pragma unroll
+    for (int e = 0; e < kCombineFragments; ++e) acc[e] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+    for (int p = 0; p < partials.parts; ++p) {
+        const int64_t unit = unit0 + p * qb;
+        const f32x4* src = partials.o + unit * (kFragments * kPfThreads) + f0 * kPfThreads + tid;
+        f32x4 part[kCombineFragments];
+#pragma unroll
+        for (int e = 0; e < kCombineFragments; ++e) part[e] = src[e * kPfThreads];
+        float w[kQueries];
+#pragma unroll
+        for (int j = 0; j < kQueries; ++j) {
+            const float2 st = partials.stat[unit * kQueryBlock + query[j]];
+            // A part without a finite logit for the query adds nothing.
+            w[j] = st.x > -INFINITY ? fast_exp2(st.x - m[j]) : 0.f;
+            total[j] = __builtin_fmaf(w[j], st.y, total[j]);
+        }
+#pragma unroll
+        for (int e = 0; e < kCombineFragments; ++e)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[e][r] = __builtin_fmaf(w[kDense ? e & 1 : 0], part[e][r], acc[e][r]);
+    }
+#pragma unroll
+    for (int j = 0; j < kQueries; ++j) {
+        const int64_t token = blk * kQueryBlock + query[j];
+        if (token >= n) continue;
+        const int64_t at = bh * n + (order ? min<int64_t>(max(order[token], 0), n - 1) : token);
+        const float inv = total[j] > 0.f ? 1.0f / total[j] : 0.f;
+#pragma unroll
+        for (int e = j; e < kCombineFragments; e += kQueries) {
+            const int f = f0 + e;
+            const int dim = kDense ? 16 * (f >> 1) + 4 * (lane >> 4) : 32 * (f >> 2) + 8 * (f & 3) + 4 * (lane >> 5);
+            const u32x2 pk = {pack_bf16(acc[e][0] * inv, acc[e][1] * inv), pack_bf16(acc[e][2] * inv, acc[e][3] * inv)};
+            *reinterpret_cast<u32x2*>(out + at * kHeadDim + dim) = pk;
+        }
+        if (lse != nullptr && f0 == 0 && lane < (kDense ? 16 : 32))
+            lse[at] = m[j] > -INFINITY ? m[j] + log2f(total[j]) : -INFINITY;
     }
 }
 
@@ -981,9 +1138,54 @@ int64_t prefill_launch_slots(int64_t bh, int64_t n) {
     return (generations + launches - 1) / launches * 64;
 }
 
+// Parts each row's tiles are split into: 1 unless the rows leave much of the
+// chip idle. A call's units (rows * parts) run at once while there are at most
+// 512 (two workgroups per CU); the time of a tile step then grows from 0.49 us
+// (a few lone workgroups) over 0.58 (one on every CU) to 0.88 (two), measured
+// on dense calls of 24 to 3,072 rows, and a unit costs its tiles plus a
+// prologue and epilogue worth about 8. Splitting adds combine_kernel (6 us)
+// and its 128 KiB of traffic per unit (0.03 us); dense units cannot run faster
+// than their K/V arrive (5.5 TB/s). More units than 512 lose: their rounds do
+// not start together and share less of what they read (640 dense rows of 512
+// tiles: 680 us, in 2 parts 618, but 640 sparse rows of 128: 211 and 238), so
+// calls of more than 256 rows never split. Measured, unsplit and at the parts
+// this picks: dense 24 rows x 3,715 tiles 1,866 -> 269 us, 48 x 3,721 1,855 ->
+// 376, 4 x 1,024 498 -> 35, 256 x 512 275 -> 240; sparse 64 x 64 42 -> 26.
+int prefill_parts(int64_t rows, int64_t tiles, int64_t kv_bytes) {
+    constexpr double kSetupSteps = 8, kCombine = 6, kUnitTraffic = 0.03, kBytesPerUs = 5.5e6, kGain = 0.95;
+    auto cost = [&](int64_t parts) {
+        const double units = double(rows * parts), wide = double(kPartUnits);
+        const double step = units <= wide ? 0.49 + 0.09 * units / wide : 0.58 + 0.30 * (units / wide - 1.0);
+        const double run = step * (double((tiles + parts - 1) / parts) + kSetupSteps);
+        return std::max(run, double(kv_bytes) / kBytesPerUs) + (parts > 1 ? kCombine + kUnitTraffic * units : 0.0);
+    };
+    int best = 1;
+    if (rows > kPartUnits) return best;
+    double best_cost = kGain * cost(1);
+    for (int64_t parts = 2; parts <= kMaxParts && parts * kMinPartTiles <= tiles && rows * parts <= 2 * kPartUnits; ++parts)
+        if (cost(parts) < best_cost) {
+            best = static_cast<int>(parts);
+            best_cost = cost(parts);
+        }
+    return best;
+}
+
+namespace {
+int call_parts(bool dense, int64_t bh, int64_t n, int64_t n_kv, int64_t samples) {
+    return prefill_parts(bh * ((n + kQueryBlock - 1) / kQueryBlock), samples / kTilePages,
+                         dense ? bh * n_kv * kHeadDim * 4 : 0);
+}
+}  // namespace
+
+size_t prefill_workspace_bytes(bool dense, int64_t bh, int64_t n, int64_t n_kv, int64_t samples) {
+    const int parts = call_parts(dense, bh, n, n_kv, samples);
+    const size_t units = size_t(bh) * ((n + kQueryBlock - 1) / kQueryBlock) * parts;
+    return parts == 1 ? 0 : units * (kFragments * kPfThreads * sizeof(f32x4) + kQueryBlock * sizeof(float2));
+}
+
 int launch_prefill(const void* q, const void* k, const void* v, bool dense, int64_t bh, int64_t n, int64_t n_kv,
                    const int32_t* ids, const float* logw, int64_t samples, void* out, float* lse,
-                   const int32_t* order, hipStream_t stream) {
+                   const int32_t* order, void* workspace, hipStream_t stream) {
     const int64_t qb = (n + kQueryBlock - 1) / kQueryBlock;
     const int64_t rows = bh * qb;
     if (samples % kTilePages != 0)
@@ -995,9 +1197,44 @@ int launch_prefill(const void* q, const void* k, const void* v, bool dense, int6
     const float scale_log2 = static_cast<float>(1.4426950408889634 / 11.313708498984761);  // log2(e)/sqrt(128)
     const int64_t per_xcd = (qb + 7) / 8;
     if (rows == 0) return 0;
-    const void* kernel = dense ? reinterpret_cast<const void*>(dense_kernel) : reinterpret_cast<const void*>(prefill_kernel);
+    const int parts = workspace ? call_parts(dense, bh, n, n_kv, samples) : 1;
     const int lds_bytes = dense ? kDenseLdsBytes : kLdsBytes;
-    if (int rc = ensure_lds_limit(kernel, lds_bytes)) return rc;
+    const int fb = static_cast<int>(n_kv / kKvBlock), s = static_cast<int>(samples);
+    const dim3 block(kPfThreads);
+    auto launch = [&](auto split, int64_t workgroups, int64_t slot_base, Partials partials) -> int {
+        constexpr bool kSplit = decltype(split)::value;
+        const void* kernel = dense ? reinterpret_cast<const void*>(dense_kernel<kSplit>)
+                                   : reinterpret_cast<const void*>(prefill_kernel<kSplit>);
+        if (int rc = ensure_lds_limit(kernel, lds_bytes)) return rc;
+        const dim3 grid(static_cast<unsigned>(workgroups));
+        if (dense)
+            hipLaunchKernelGGL(dense_kernel<kSplit>, grid, block, lds_bytes, stream, static_cast<const uint16_t*>(q),
+                               static_cast<const uint16_t*>(k), static_cast<const uint16_t*>(v),
+                               static_cast<uint16_t*>(out), lse, n, n_kv, qb, rows, fb, s, scale_log2, slot_base,
+                               partials);
+        else
+            hipLaunchKernelGGL(prefill_kernel<kSplit>, grid, block, lds_bytes, stream, static_cast<const uint16_t*>(q),
+                               static_cast<const uint16_t*>(k), static_cast<const uint16_t*>(v), ids, logw,
+                               static_cast<uint16_t*>(out), lse, n, n_kv, qb, rows, fb, s, scale_log2, order,
+                               slot_base, partials);
+        return check_launch(dense ? "dense_kernel" : "prefill_kernel");
+    };
+    if (parts > 1) {
+        const int64_t units = rows * parts;
+        Partials partials;
+        partials.o = static_cast<f32x4*>(workspace);
+        partials.stat = reinterpret_cast<float2*>(partials.o + units * kFragments * kPfThreads);
+        partials.parts = parts;
+        if (int rc = launch(std::true_type{}, (units + 7) / 8 * 8, 0, partials)) return rc;
+        const dim3 grid(static_cast<unsigned>(rows), kFragments / kCombineFragments);
+        if (dense)
+            hipLaunchKernelGGL(combine_kernel<true>, grid, block, 0, stream, partials, qb, n,
+                               static_cast<uint16_t*>(out), lse, order);
+        else
+            hipLaunchKernelGGL(combine_kernel<false>, grid, block, 0, stream, partials, qb, n,
+                               static_cast<uint16_t*>(out), lse, order);
+        return check_launch("combine_kernel");
+    }
     // The rows are launched in chunks of about kRowsPerLaunch, each a whole
     // number of generations (64 row slots per XCD; a generation is what the
     // chip holds at once, two workgroups per CU). The rows resident on an XCD
@@ -1011,20 +1248,7 @@ int launch_prefill(const void* q, const void* k, const void* v, bool dense, int6
     const int64_t per_launch = prefill_launch_slots(bh, n);
     for (int64_t slot_base = 0; slot_base < slots; slot_base += per_launch) {
         const int64_t count = std::min(per_launch, slots - slot_base);
-        const dim3 grid(static_cast<unsigned>(count * 8)), block(kPfThreads);
-        const int fb = static_cast<int>(n_kv / kKvBlock), s = static_cast<int>(samples);
-        if (dense) {
-            hipLaunchKernelGGL(dense_kernel, grid, block, lds_bytes, stream, static_cast<const uint16_t*>(q),
-                               static_cast<const uint16_t*>(k), static_cast<const uint16_t*>(v),
-                               static_cast<uint16_t*>(out), lse, n, n_kv, qb, rows, fb, s, scale_log2, slot_base);
-            if (int rc = check_launch("dense_kernel")) return rc;
-        } else {
-            hipLaunchKernelGGL(prefill_kernel, grid, block, lds_bytes, stream, static_cast<const uint16_t*>(q),
-                               static_cast<const uint16_t*>(k), static_cast<const uint16_t*>(v), ids, logw,
-                               static_cast<uint16_t*>(out), lse, n, n_kv, qb, rows, fb, s, scale_log2, order,
-                               slot_base);
-            if (int rc = check_launch("prefill_kernel")) return rc;
-        }
+        if (int rc = launch(std::false_type{}, count * 8, slot_base, Partials{nullptr, nullptr, 1})) return rc;
     }
     return 0;
 }

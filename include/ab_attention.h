@@ -30,7 +30,7 @@
 extern "C" {
 #endif
 
-#define AB_ABI_VERSION 4
+#define AB_ABI_VERSION 5
 
 enum ab_status {
     AB_OK = 0,
@@ -132,7 +132,32 @@ int ab_paged_prefill_kv(const void *q, const void *k, const void *v, int64_t bat
 int ab_dense_prefill(const void *q, const void *k, const void *v, int64_t batch_heads, int64_t q_tokens,
                      int64_t kv_tokens, void *out, float *lse, void *stream);
 
-/* How the prefill entry points split a call's rows into launches; no
+/* Every prefill above through one entry point, with an optional workspace.
+ * samples > 0: the listed blocks, as ab_paged_prefill_kv (order NULL) or with
+ * the query rows read and written through `order` int32 [q_tokens] (see
+ * ab_paged_prefill_ordered); samples == AB_PREFILL_DENSE: as ab_dense_prefill
+ * (ids, log_weights and order unused). With a workspace, a call whose rows would
+ * leave much of the GPU idle (a prompt's few query blocks over a whole video,
+ * a short clip) splits each row's keys over several workgroups and adds up
+ * their float32 partial results; the result is the same up to float32
+ * rounding. ab_prefill_workspace_bytes gives the bytes (0: this size is not
+ * split and needs none), 16-byte aligned. workspace NULL never splits. */
+#define AB_PREFILL_DENSE (-1)
+typedef struct ab_prefill_args {
+    const void *q, *k, *v;
+    const int32_t *order;
+    const int32_t *ids;
+    const float *log_weights;
+    void *out;
+    float *lse;
+    int64_t batch_heads, q_tokens, kv_tokens, samples;
+    void *workspace;
+    size_t workspace_bytes;
+} ab_prefill_args;
+size_t ab_prefill_workspace_bytes(int64_t batch_heads, int64_t q_tokens, int64_t kv_tokens, int64_t samples);
+int ab_prefill(const ab_prefill_args *args, void *stream);
+
+/* How the unsplit prefill entry points split a call's rows into launches; no
  * counterpart in the reference (FlashInfer runs one kernel). The rows of
  * head h, query block b are dealt to 8 groups (one per XCD) of
  * ceil(q_blocks / 8) consecutive blocks: group b / ceil(q_blocks / 8), row

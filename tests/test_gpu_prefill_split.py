@@ -1,0 +1,96 @@
+"""The prefill with each row's keys split over several workgroups (ab_prefill
+with a workspace) and without (workspace NULL), both against the exact oracle
+within the bf16 bars of the unsplit tests: splitting only reorders float32
+sums."""
+import numpy as np
+import pytest
+import torch
+
+from ab_attention import _lib
+
+MAX_ABS, REL_L2, LSE_ABS = 2e-2, 1e-2, 1e-3
+UNIT_BYTES = 16 * 256 * 16 + 128 * 8
+
+
+def _run(q, k, v, ids, w, order, split):
+    bh, nq, nk = q.shape[1], q.shape[2], k.shape[2]
+    samples = _lib.PREFILL_DENSE if ids is None else ids.shape[1]
+    lib = _lib.load()
+    size = lib.ab_prefill_workspace_bytes(bh, nq, nk, samples)
+    assert size > 0 and size % UNIT_BYTES == 0
+    ws = torch.empty(size, dtype=torch.uint8, device="cuda") if split else None
+    out = torch.full_like(q, float("nan"))
+    lse = torch.full(q.shape[:3], float("nan"), device="cuda")
+    args = _lib.PrefillArgs(*(_lib.ptr(t) for t in (q, k, v, order, ids, w, out, lse)), bh, nq, nk, samples,
+                            _lib.ptr(ws), size if split else 0)
+    _lib.check(lib.ab_prefill(args, _lib.stream(q.device)))
+    torch.cuda.synchronize()
+    return out.float().cpu().numpy()[0], lse.cpu().numpy()[0]
+
+
+# (heads, queries, keys, listed blocks or None, logit scale, order): one query
+# block and several, ragged queries and keys, part counts that do and do not
+# divide the tiles, a first tile whose maximum later parts exceed by far
+# (their safe pass), and a token order.
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,nq,nk,samples,scale,ordered", [
+    (1, 4, 1024, None, 1, False), (2, 200, 4100, None, 1, False), (3, 130, 9000, None, 1, False),
+    (1, 128, 8192, None, 40, False), (1, 1000, 4096, 520, 1, False), (2, 2048, 2048, 264, 1, True),
+    (2, 2048, 2048, 256, 40, False),
+])
+def test_split_rows(oracle_mod, heads, nq, nk, samples, scale, ordered):
+    torch.manual_seed(nq + nk)
+    print(f"split prefill heads={heads} nq={nq} nk={nk} samples={samples} scale={scale}", flush=True)
+    q = (torch.randn(1, heads, nq, 128) * scale).to(torch.bfloat16)
+    k, v = (torch.randn(1, heads, nk, 128).to(torch.bfloat16) for _ in range(2))
+    rows, fb = heads * -(-nq // 128), nk // 4
+    ids = w = order = None
+    listed = np.tile(np.arange(fb, dtype=np.int32), (rows, 1)), np.zeros((rows, fb), np.float32)
+    if samples is not None:
+        rng = np.random.default_rng(nq)
+        listed = (np.stack([np.sort(rng.choice(fb, samples, replace=False)) for _ in range(rows)]).astype(np.int32),
+                  rng.random((rows, samples)).astype(np.float32) * 3)
+        # Row 0: its first 96 blocks removed (every block of its first part);
+        # row 1: all of them (no output).
+        listed[1][0, :96] = -np.inf
+        listed[1][1] = -np.inf
+        ids, w = (torch.from_numpy(t).cuda() for t in listed)
+    if ordered:
+        order = torch.randperm(nq, generator=torch.Generator().manual_seed(1))
+    f32 = lambda t: t.float().numpy()[0]
+    q_seen = q if order is None else q[:, :, order]
+    ref_o, ref_l = oracle_mod.prefill(f32(q_seen), f32(k), f32(v), *listed)
+    order_d = None if order is None else order.to(torch.int32).cuda()
+    for split in (False, True):
+        got, lse = _run(q.cuda(), k.cuda(), v.cuda(), ids, w, order_d, split)
+        if order is not None:
+            got, lse = got[:, order], lse[:, order]
+        assert np.abs(got - ref_o).max() <= MAX_ABS, split
+        assert np.linalg.norm(got - ref_o) / np.linalg.norm(ref_o) <= REL_L2, split
+        finite = np.isfinite(ref_l)
+        assert np.array_equal(finite, np.isfinite(lse)), split
+        # float32 logits of magnitude L carry about 2^-22 L.
+        assert np.abs(lse[finite] - ref_l[finite]).max() <= LSE_ABS * max(1, scale / 4), split
+
+
+def test_split_rule():
+    """Calls with a row per CU or more are not split; the units of a split
+    call stay within two per CU and within a row's tiles."""
+    size = _lib.load().ab_prefill_workspace_bytes
+    dense = _lib.PREFILL_DENSE
+    assert size(12, 32760, 32760, dense) == size(80, 75600, 75600, 2048) == size(1, 257 * 128, 8192, dense) == 0
+    assert size(0, 128, 128, dense) == size(1, 128, 128, 0) == 0
+    assert size(1, 128, 32, dense) == 0  # a single tile
+    for bh, nq, nk, samples in [(24, 256, 119056, dense), (1, 4, 119056, dense), (2, 2048, 2048, 256), (2, 16384, 16384, dense)]:
+        rows, tiles = bh * -(-nq // 128), -(-(nk // 4 if samples == dense else samples) // 8)
+        units, rest = divmod(size(bh, nq, nk, samples), UNIT_BYTES)
+        assert rest == 0 and units % rows == 0 and rows < units <= 512 and units // rows * 8 <= tiles
+
+
+def test_split_rejects_a_bad_workspace():
+    lib, a = _lib.load(), 4096  # a stand-in address: rejected before any launch
+    for ws, size, message in ((a, 64, b"smaller than"), (a + 8, 1 << 30, b"16-byte aligned")):
+        args = _lib.PrefillArgs(a, a, a, None, None, None, a, None, 24, 256, 119056, _lib.PREFILL_DENSE, ws, size)
+        assert lib.ab_prefill(args, None) == 1 and message in lib.ab_last_error()
+    args = _lib.PrefillArgs(a, a, a, None, None, None, a, None, 1, 128, 128, 0, None, 0)
+    assert lib.ab_prefill(args, None) == 1 and b"multiple of 8" in lib.ab_last_error()
