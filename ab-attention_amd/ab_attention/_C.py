@@ -43,7 +43,7 @@ def ibcs(q: torch.Tensor, k: torch.Tensor) -> torch.Tensor:
     batch_heads = batch * heads
     rows = batch_heads * -(-tokens // QUERY_BLOCK)
     lib = _lib.load()
-    with torch.cuda.device(q.device):
+    with _lib.on(q.device):
         ws_bytes = lib.ab_ibcs_workspace_bytes(batch_heads, tokens)
         workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
         scores = torch.empty((rows, fine_blocks), dtype=torch.float32, device=q.device)
@@ -64,7 +64,7 @@ def ibcs_ordered(q: torch.Tensor, k: torch.Tensor, order: torch.Tensor) -> torch
     batch_heads = batch * heads
     rows = batch_heads * -(-tokens // QUERY_BLOCK)
     lib = _lib.load()
-    with torch.cuda.device(q.device):
+    with _lib.on(q.device):
         ws_bytes = lib.ab_ibcs_workspace_bytes(batch_heads, tokens)
         workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
         scores = torch.empty((rows, tokens // KV_BLOCK), dtype=torch.float32, device=q.device)
@@ -89,7 +89,7 @@ def sip(scores: torch.Tensor, offsets: torch.Tensor, ids: torch.Tensor, logs: to
     samples = ids.shape[1]
     _require(0 < samples < scores.shape[1], "sample count must be inside the population")
     lib = _lib.load()
-    with torch.cuda.device(scores.device):
+    with _lib.on(scores.device):
         _lib.check(lib.ab_sip(_lib.ptr(scores), _lib.ptr(offsets), scores.shape[0], scores.shape[1],
                               samples, _lib.ptr(ids), _lib.ptr(logs), _lib.stream(scores.device)))
 
@@ -129,9 +129,35 @@ def ibcs_sip(q: torch.Tensor, k: torch.Tensor, offsets: torch.Tensor, ids: torch
         _require(order.dtype == torch.int32 and order.is_contiguous() and order.device == q.device
                  and order.shape == (tokens,), "order must be int32 [tokens] on the q device")
     lib = _lib.load()
-    with torch.cuda.device(q.device):
+    with _lib.on(q.device):
         ws_bytes = lib.ab_ibcs_sip_workspace_bytes(batch_heads, tokens)
         workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
         _lib.check(lib.ab_ibcs_sip(_lib.ptr(q), _lib.ptr(k), _lib.ptr(order), batch_heads, tokens,
                                    _lib.ptr(offsets), samples, _lib.ptr(workspace), ws_bytes, _lib.ptr(ids),
                                    _lib.ptr(logs), _lib.stream(q.device)))
+
+
+def plan_heads(q: torch.Tensor, k: torch.Tensor, start: int, stop: int, offsets: torch.Tensor, ids: torch.Tensor,
+               logs: torch.Tensor, order: torch.Tensor | None = None) -> None:
+    """``ibcs_sip`` of heads start .. stop-1 of the flattened [batch * heads] of
+    q, k (offsets, ids and logs are those heads' rows), reading them where they
+    lie: slices of tokens and transposed projections need no copy (ab_plan)."""
+    _require(q.is_cuda and k.is_cuda, "q and k must be CUDA tensors")
+    _require(q.device == k.device, "q and k must use the same CUDA device")
+    _require(q.dtype == torch.bfloat16 and k.dtype == torch.bfloat16, "IBCS requires bfloat16 q/k")
+    _require(q.shape[3] == HEAD_DIM, "IBCS requires head_dim=128")
+    batch, heads, tokens, _ = q.shape
+    fine_blocks = tokens // KV_BLOCK
+    _require(0 < fine_blocks <= MAX_KV_BLOCKS, "KV4 block count must be in [1, 32768]")
+    if order is not None:
+        _require(order.dtype == torch.int32 and order.is_contiguous() and order.device == q.device
+                 and order.shape == (tokens,), "order must be int32 [tokens] on the q device")
+    (q, q_stride), (k, k_stride) = _lib.in_place(q), _lib.in_place(k)
+    lib, address = _lib.load(), _lib.address
+    with _lib.on(q.device):
+        ws_bytes = lib.ab_ibcs_sip_workspace_bytes(stop - start, tokens)
+        workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
+        args = _lib.PlanArgs(address(q), address(k), address(order), address(offsets), address(ids), address(logs),
+                             batch, heads, start, stop - start, tokens, ids.shape[1], q_stride, k_stride,
+                             address(workspace), ws_bytes)
+        _lib.check(lib.ab_plan(args, _lib.stream(q.device)))

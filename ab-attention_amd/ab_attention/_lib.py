@@ -12,6 +12,7 @@ load, every entry point raises.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
 
@@ -35,8 +36,18 @@ class PrefillArgs(ctypes.Structure):
     """ab_prefill_args of include/ab_attention.h."""
 
     _fields_ = [("q", _P), ("k", _P), ("v", _P), ("order", _P), ("ids", _P), ("log_weights", _P), ("out", _P),
-                ("lse", _P), ("batch_heads", _I64), ("q_tokens", _I64), ("kv_tokens", _I64), ("samples", _I64),
-                ("workspace", _P), ("workspace_bytes", _SZ)]
+                ("lse", _P), ("batch", _I64), ("heads", _I64), ("q_tokens", _I64), ("kv_tokens", _I64),
+                ("samples", _I64), ("q_stride", _I64 * 3), ("k_stride", _I64 * 3), ("v_stride", _I64 * 3),
+                ("out_stride", _I64 * 3), ("workspace", _P), ("workspace_bytes", _SZ)]
+
+
+class PlanArgs(ctypes.Structure):
+    """ab_plan_args of include/ab_attention.h."""
+
+    _fields_ = [("q", _P), ("k", _P), ("order", _P), ("offsets", _P), ("ids", _P), ("log_weights", _P),
+                ("batch", _I64), ("heads", _I64), ("first_head", _I64), ("head_count", _I64), ("tokens", _I64),
+                ("samples", _I64), ("q_stride", _I64 * 3), ("k_stride", _I64 * 3), ("workspace", _P),
+                ("workspace_bytes", _SZ)]
 
 
 # name -> (restype, argtypes); mirrors include/ab_attention.h
@@ -59,6 +70,7 @@ SIGNATURES = {
     "ab_ibcs_sip_workspace_bytes": (_SZ, [_I64, _I64]),
     "ab_ibcs_sip": (ctypes.c_int, [_P, _P, _P, _I64, _I64, _P, _I64, _P, _SZ, _P, _P, _P]),
     "ab_ibcs_sip_exact_draws": (ctypes.c_int, [_P, _P, _P, _I64, _I64, _P, _I64, _P, _SZ, _P, _P, _P]),
+    "ab_plan": (ctypes.c_int, [ctypes.POINTER(PlanArgs), _P]),
     "ab_dense_prefill": (ctypes.c_int, [_P, _P, _P, _I64, _I64, _I64, _P, _P, _P]),
     "ab_prefill_launch_slots": (_I64, [_I64, _I64]),
     "ab_prefill_workspace_bytes": (_SZ, [_I64, _I64, _I64, _I64]),
@@ -70,7 +82,7 @@ STATIC_SIGNATURES = {
     "ab_ibcs_sip_static": (ctypes.c_int, [_P, _P, _P, _I64, _I64, _P, _I64, _P, _P, _P]),
 }
 
-ABI_VERSION = 5
+ABI_VERSION = 6
 _lib = None
 _static = None
 
@@ -137,5 +149,34 @@ def ptr(t: torch.Tensor | None) -> ctypes.c_void_p:
 
 
 def stream(device: torch.device) -> ctypes.c_void_p:
-    """The current torch stream of ``device`` as a hipStream_t."""
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    """The current torch stream of ``device`` as a hipStream_t (the raw handle;
+    ``torch.cuda.current_stream`` makes a Stream object for it, 1.8 us)."""
+    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(device.index))
+
+
+_HERE = contextlib.nullcontext()
+
+
+def on(device: torch.device):
+    """``torch.cuda.device(device)``, free where it is the current device."""
+    return _HERE if torch.cuda.current_device() == device.index else torch.cuda.device(device)
+
+
+def address(t: torch.Tensor | None) -> int:
+    """``ptr`` for a field of PrefillArgs or PlanArgs."""
+    return 0 if t is None else t.data_ptr()
+
+
+def in_place(t: torch.Tensor):
+    """(tensor, its (batch, head, token) strides in elements) for t [B, H, N,
+    128]: t itself where the library can read its rows in place (contiguous
+    rows of 128 that start on 16 bytes, at any batch, head and token strides
+    with at most 24-bit page sizes and 4 GiB per head), else a contiguous copy."""
+    if not t.is_contiguous():
+        batch, head, token, dim = t.stride()
+        if (dim == 1 and not (batch | head | token) & 7 and max(batch, head) < (1 << 34) and 0 < token < (1 << 21)
+                and t.shape[2] * token < (1 << 31) and t.data_ptr() % 16 == 0):
+            return t, (batch, head, token)
+        t = t.contiguous()
+    _, heads, tokens, dim = t.shape  # not t.stride(): it may be anything where a size is 1
+    return t, (heads * tokens * dim, tokens * dim, dim)

@@ -94,33 +94,28 @@ def _build_plan(q, k, sample_pages, seed, order=None):
         raise ValueError("sample_pages must be positive")
     if sample_pages * 128 >= q.shape[2]:
         raise ValueError("sampled key count must be smaller than the sequence length")
-    from . import _C as ops
+    from . import _C as ops, _lib
 
     batch_heads = q.shape[0] * q.shape[1]
-    tokens, dim = q.shape[2:]
+    tokens = q.shape[2]
     q_blocks = math.ceil(tokens / 128)
     rows, samples = batch_heads * q_blocks, sample_pages * 32
 
     # All offsets are drawn before chunking, so chunking cannot change the plan.
     generator = torch.Generator(device=q.device).manual_seed(seed)
     offsets = torch.rand(rows, device=q.device, generator=generator)
-    flat_q = q.reshape(batch_heads, tokens, dim)
-    flat_k = k.reshape(batch_heads, tokens, dim)
 
     heads_per_chunk = _heads_per_chunk(batch_heads, q_blocks, tokens)
     sampled = torch.empty((rows, samples), dtype=torch.int32, device=q.device)
     log_weights = torch.empty((rows, samples), dtype=torch.float32, device=q.device)
 
+    q, k = _lib.in_place(q)[0], _lib.in_place(k)[0]
     for start in range(0, batch_heads, heads_per_chunk):
         stop = min(batch_heads, start + heads_per_chunk)
         first, last = start * q_blocks, stop * q_blocks
-        # IBCS scores and SIP sampling of the chunk (the reference's _C.ibcs
-        # then _C.sip) in one native call that keeps the scores on chip.
-        ops.ibcs_sip(
-            flat_q[start:stop].unsqueeze(0).contiguous(),
-            flat_k[start:stop].unsqueeze(0).contiguous(),
-            offsets[first:last], sampled[first:last], log_weights[first:last], order,
-        )
+        # IBCS scores and SIP sampling of the chunk's heads (the reference's
+        # _C.ibcs then _C.sip) in one native call that keeps the scores on chip.
+        ops.plan_heads(q, k, start, stop, offsets[first:last], sampled[first:last], log_weights[first:last], order)
 
     return SamplePlan(
         sampled.reshape(rows, sample_pages, 32),

@@ -31,20 +31,22 @@ _PAGE_SIZE = 4
 
 
 def _run(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, ids, weights, samples: int, order, return_lse: bool):
-    """ab_prefill of row-major q, k, v (samples: _lib.PREFILL_DENSE for dense). The workspace of a
+    """ab_prefill of q, k, v, read where they lie (samples: _lib.PREFILL_DENSE for dense). The workspace of a
     call that splits its rows over more workgroups lives for the call only (the
     caching allocator keeps it on this stream)."""
-    batch, heads, tokens, _ = q.shape
+    batch, heads, tokens, dim = q.shape
     kv_tokens, device = k.shape[2], q.device
-    output = torch.empty_like(q)
+    (q, q_stride), (k, k_stride), (v, v_stride) = _lib.in_place(q), _lib.in_place(k), _lib.in_place(v)
+    output = torch.empty_like(q, memory_format=torch.contiguous_format)
     lse = torch.empty((batch, heads, tokens), dtype=torch.float32, device=device) if return_lse else None
-    lib = _lib.load()
-    with torch.cuda.device(device):
+    lib, address = _lib.load(), _lib.address
+    with _lib.on(device):
         ws_bytes = lib.ab_prefill_workspace_bytes(batch * heads, tokens, kv_tokens, samples)
         workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=device) if ws_bytes else None
-        args = _lib.PrefillArgs(_lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(order), _lib.ptr(ids),
-                                _lib.ptr(weights), _lib.ptr(output), _lib.ptr(lse), batch * heads, tokens, kv_tokens,
-                                samples, _lib.ptr(workspace), ws_bytes)
+        args = _lib.PrefillArgs(address(q), address(k), address(v), address(order), address(ids), address(weights),
+                                address(output), address(lse), batch, heads, tokens, kv_tokens, samples, q_stride,
+                                k_stride, v_stride, (heads * tokens * dim, tokens * dim, dim), address(workspace),
+                                ws_bytes)
         _lib.check(lib.ab_prefill(args, _lib.stream(device)))
     return (output, lse) if return_lse else output
 
@@ -53,9 +55,10 @@ def _prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, ids: torch.Tenso
              order: torch.Tensor | None, return_lse: bool):
     """The weighted prefill, with a query token order when one is given;
     ids/weights [rows, S]. Shapes are checked by the callers."""
-    q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
-    ids = ids.to(torch.int32).contiguous()
-    weights = weights.to(torch.float32).contiguous()
+    if ids.dtype != torch.int32 or not ids.is_contiguous():
+        ids = ids.to(torch.int32).contiguous()
+    if weights.dtype != torch.float32 or not weights.is_contiguous():
+        weights = weights.to(torch.float32).contiguous()
     return _run(q, k, v, ids, weights, ids.shape[-1], order, return_lse)
 
 
@@ -115,7 +118,7 @@ def _prefill_dense(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, return_
     [B,H,Nk,128] (Nk % 4 == 0) on the dense kernel (ab_dense_prefill); the
     page list is implicit, so nothing of size rows x blocks is built. Shapes
     are checked by the callers."""
-    return _run(q.contiguous(), k.contiguous(), v.contiguous(), None, None, _lib.PREFILL_DENSE, None, return_lse)
+    return _run(q, k, v, None, None, _lib.PREFILL_DENSE, None, return_lse)
 
 
 def _remap_ids(ids: torch.Tensor, page_map: torch.Tensor) -> torch.Tensor:
@@ -123,7 +126,7 @@ def _remap_ids(ids: torch.Tensor, page_map: torch.Tensor) -> torch.Tensor:
     ids = ids.to(torch.int32).contiguous()
     out = torch.empty_like(ids)
     lib = _lib.load()
-    with torch.cuda.device(ids.device):
+    with _lib.on(ids.device):
         _lib.check(lib.ab_remap_ids(_lib.ptr(ids), ids.numel(), _lib.ptr(page_map), page_map.numel(),
                                     _lib.ptr(out), _lib.stream(ids.device)))
     return out

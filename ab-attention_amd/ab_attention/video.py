@@ -185,7 +185,7 @@ def merge_states(state_a, state_b, *, return_lse: bool = False):
     out = torch.empty_like(o_a)
     lse = torch.empty_like(s_a) if return_lse else None
     lib = _lib.load()
-    with torch.cuda.device(o_a.device):
+    with _lib.on(o_a.device):
         _lib.check(lib.ab_merge_states(_lib.ptr(o_a), _lib.ptr(s_a), _lib.ptr(o_b), _lib.ptr(s_b), s_a.numel(),
                                        _lib.ptr(out), _lib.ptr(lse), _lib.stream(o_a.device)))
     return (out, lse) if return_lse else out

@@ -15,12 +15,13 @@
 
 #include "../../include/ab_attention.h"
 #include "common.hpp"
+#include "layout.hpp"
 
 namespace ab {
 
 int64_t lse_stride(int64_t fb);
-int launch_cluster_pool(const void* q, const void* k, int64_t bh, int64_t n, void* centroids, float* pops,
-                        void* pooled, float qk_scale_log2, const int32_t* order, hipStream_t stream);
+int launch_cluster_pool(const void* q, const void* k, const QkLayout& layout, int64_t bh, int64_t n, void* centroids,
+                        float* pops, void* pooled, float qk_scale_log2, const int32_t* order, hipStream_t stream);
 int launch_lse(const void* centroids, const void* pooled, int64_t bh, int64_t n, void* lse, float* lse_max,
                float* lse_den, hipStream_t stream);
 int launch_masses(const void* lse, const float* pops, const float* lse_max, const float* lse_den, int64_t rows,
@@ -32,9 +33,7 @@ bool sip_fused_fits(int64_t population);
 int launch_sip_fused(const void* lse, const float* pops, const float* lse_max, const float* lse_den, int64_t ld,
                      const float* offsets, int64_t rows, int64_t population, int64_t samples, int32_t* ids,
                      float* logw, int force_exact, hipStream_t stream);
-int launch_prefill(const void* q, const void* k, const void* v, bool dense, int64_t bh, int64_t n, int64_t n_kv,
-                   const int32_t* ids, const float* logw, int64_t samples, void* out, float* lse,
-                   const int32_t* order, void* workspace, hipStream_t stream);
+int launch_prefill(const PrefillCall& call, hipStream_t stream);
 size_t prefill_workspace_bytes(bool dense, int64_t bh, int64_t n, int64_t n_kv, int64_t samples);
 int64_t prefill_launch_slots(int64_t bh, int64_t n);
 int launch_remap_ids(const int32_t* ids, int64_t count, const int32_t* map, int64_t map_len, int32_t* out,
@@ -86,6 +85,18 @@ int check_qk_shape(const char* what, int64_t bh, int64_t n) {
         return set_error(AB_ERR_INVALID, "%s: KV4 block count must be in [1, 32768]", what);
     const int64_t qb = (n + kQueryBlock - 1) / kQueryBlock;
     if (qb > 65535 || bh > 65535) return set_error(AB_ERR_INVALID, "%s: grid too large", what);
+    return AB_OK;
+}
+
+// Strides (batch, head, token) in elements of a tensor whose rows start at
+// multiples of `align` elements.
+int tensor_layout(const char* what, const int64_t (&stride)[3], int64_t align, TensorLayout& out) {
+    for (int64_t s : stride)
+        if (s < 0 || s % align || s / 4 > int64_t(0xffffffff))
+            return set_error(AB_ERR_INVALID, "%s: strides must be multiples of %d elements from 0 to 2^34", what,
+                             (int)align);
+    out = {static_cast<uint32_t>(stride[0] / 4), static_cast<uint32_t>(stride[1] / 4),
+           static_cast<uint32_t>(stride[2] / 4)};
     return AB_OK;
 }
 
@@ -163,8 +174,8 @@ int ab_ibcs_cluster_pool(const void* q, const void* k, int64_t batch_heads, int6
         return set_error(AB_ERR_INVALID, "ibcs: null pointer");
     if (!aligned16(q) || !aligned16(k) || !aligned16(pooled_keys))
         return set_error(AB_ERR_INVALID, "ibcs: q, k and pooled keys must be 16-byte aligned");
-    return launch_cluster_pool(q, k, batch_heads, tokens, centroids, populations, pooled_keys, qk_scale_log2(),
-                               nullptr, static_cast<hipStream_t>(stream));
+    return launch_cluster_pool(q, k, contiguous_qk(batch_heads, tokens), batch_heads, tokens, centroids, populations,
+                               pooled_keys, qk_scale_log2(), nullptr, static_cast<hipStream_t>(stream));
 }
 
 int ab_ibcs_lse(const void* centroids, const void* pooled_keys, int64_t batch_heads, int64_t tokens,
@@ -207,7 +218,7 @@ int ibcs_chain(const void* q, const void* k, const int32_t* order, int64_t batch
     if ((reinterpret_cast<uintptr_t>(workspace) & 255u) != 0)
         return set_error(AB_ERR_INVALID, "ibcs: workspace must be 256-byte aligned");
     char* ws = static_cast<char*>(workspace);
-    if (int rc = launch_cluster_pool(q, k, batch_heads, tokens, ws + L.centroids,
+    if (int rc = launch_cluster_pool(q, k, contiguous_qk(batch_heads, tokens), batch_heads, tokens, ws + L.centroids,
                                      reinterpret_cast<float*>(ws + L.pops), ws + L.pooled, qk_scale_log2(), order,
                                      static_cast<hipStream_t>(stream)))
         return rc;
@@ -264,9 +275,9 @@ int check_ibcs_sip_args(const char* what, const void* q, const void* k, int64_t 
 namespace {
 // ab_ibcs_sip; force_exact selects the reference's probe sequence for every
 // row sampled with kept prefixes (same bits, testing only).
-int ibcs_sip_impl(const void* q, const void* k, const int32_t* order, int64_t batch_heads, int64_t tokens,
-                  const float* offsets, int64_t samples, void* workspace, size_t workspace_bytes, int32_t* ids,
-                  float* log_weights, int force_exact, void* stream) {
+int ibcs_sip_impl(const void* q, const void* k, const QkLayout& layout, const int32_t* order, int64_t batch_heads,
+                  int64_t tokens, const float* offsets, int64_t samples, void* workspace, size_t workspace_bytes,
+                  int32_t* ids, float* log_weights, int force_exact, void* stream) {
     if (int rc = check_ibcs_sip_args("ibcs_sip", q, k, batch_heads, tokens, offsets, samples, ids, log_weights))
         return rc;
     const IbcsLayout L = ibcs_layout(batch_heads, tokens);
@@ -282,7 +293,7 @@ int ibcs_sip_impl(const void* q, const void* k, const int32_t* order, int64_t ba
     float* pops = reinterpret_cast<float*>(ws + L.pops);
     float* lse_max = reinterpret_cast<float*>(ws + L.lse_max);
     float* lse_den = reinterpret_cast<float*>(ws + L.lse_den);
-    if (int rc = launch_cluster_pool(q, k, batch_heads, tokens, ws + L.centroids, pops, ws + L.pooled,
+    if (int rc = launch_cluster_pool(q, k, layout, batch_heads, tokens, ws + L.centroids, pops, ws + L.pooled,
                                      qk_scale_log2(), order, st))
         return rc;
     if (int rc = launch_lse(ws + L.centroids, ws + L.pooled, batch_heads, tokens, ws + L.lse, lse_max, lse_den, st))
@@ -297,15 +308,29 @@ extern "C" {
 int ab_ibcs_sip(const void* q, const void* k, const int32_t* order, int64_t batch_heads, int64_t tokens,
                 const float* offsets, int64_t samples, void* workspace, size_t workspace_bytes, int32_t* ids,
                 float* log_weights, void* stream) {
-    return ibcs_sip_impl(q, k, order, batch_heads, tokens, offsets, samples, workspace, workspace_bytes, ids,
-                         log_weights, 0, stream);
+    return ibcs_sip_impl(q, k, contiguous_qk(batch_heads, tokens), order, batch_heads, tokens, offsets, samples,
+                         workspace, workspace_bytes, ids, log_weights, 0, stream);
 }
 
 int ab_ibcs_sip_exact_draws(const void* q, const void* k, const int32_t* order, int64_t batch_heads,
                             int64_t tokens, const float* offsets, int64_t samples, void* workspace,
                             size_t workspace_bytes, int32_t* ids, float* log_weights, void* stream) {
-    return ibcs_sip_impl(q, k, order, batch_heads, tokens, offsets, samples, workspace, workspace_bytes, ids,
-                         log_weights, 1, stream);
+    return ibcs_sip_impl(q, k, contiguous_qk(batch_heads, tokens), order, batch_heads, tokens, offsets, samples,
+                         workspace, workspace_bytes, ids, log_weights, 1, stream);
+}
+
+int ab_plan(const ab_plan_args* a, void* stream) {
+    if (!a) return set_error(AB_ERR_INVALID, "ibcs_sip: null pointer");
+    if (a->heads <= 0 || a->first_head < 0 || a->batch <= 0 || a->heads > INT32_MAX / a->batch ||
+        a->head_count > a->batch * a->heads - a->first_head)
+        return set_error(AB_ERR_INVALID, "ibcs_sip: head range outside the tensors");
+    QkLayout layout;
+    if (int rc = tensor_layout("ibcs_sip", a->q_stride, 8, layout.q)) return rc;
+    if (int rc = tensor_layout("ibcs_sip", a->k_stride, 8, layout.k)) return rc;
+    layout.heads = divisor(static_cast<uint32_t>(a->heads));
+    layout.first_head = static_cast<uint32_t>(a->first_head);
+    return ibcs_sip_impl(a->q, a->k, layout, a->order, a->head_count, a->tokens, a->offsets, a->samples, a->workspace,
+                         a->workspace_bytes, a->ids, a->log_weights, 0, stream);
 }
 
 int ab_sip(const float* scores, const float* offsets, int64_t rows, int64_t population, int64_t samples,
@@ -333,55 +358,77 @@ int ab_paged_prefill(const void* q, const void* k, const void* v, int64_t batch_
 }
 
 namespace {
-// Shared validation of the prefill entry points. dense: every KV4 block of
-// K/V at weight 0 (ids and log_weights are not read; samples is derived).
-int paged_prefill_checked(const void* q, const void* k, const void* v, bool dense, const int32_t* order,
-                          int64_t batch_heads, int64_t q_tokens, int64_t kv_tokens, const int32_t* ids,
-                          const float* log_weights, int64_t samples, void* out, float* lse, void* workspace,
-                          size_t workspace_bytes, void* stream) {
-    if (batch_heads <= 0 || q_tokens <= 0 || kv_tokens <= 0)
+// Shared validation of the prefill entry points. call.dense: every KV4 block
+// of K/V at weight 0 (ids and log_weights are not read; samples is derived).
+int prefill_checked(PrefillCall call, size_t workspace_bytes, void* stream) {
+    if (call.batch > 65535) return set_error(AB_ERR_INVALID, "paged_prefill: grid too large");
+    const int64_t batch_heads = call.batch * call.layout.heads.d;
+    if (call.batch <= 0 || call.layout.heads.d == 0 || call.q_tokens <= 0 || call.kv_tokens <= 0)
         return set_error(AB_ERR_INVALID, "paged_prefill: batch_heads and token counts must be positive");
-    if (kv_tokens % kKvBlock)
+    if (call.kv_tokens % kKvBlock)
         return set_error(AB_ERR_INVALID, "paged_prefill: key/value length must be divisible by 4");
-    if (kv_tokens * kHeadDim * 2 > int64_t(0xffffffff))
+    if (call.kv_tokens * kHeadDim * 2 > int64_t(0xffffffff))
         return set_error(AB_ERR_INVALID, "paged_prefill: one head of K/V must be under 4 GiB");
-    const int64_t qb = (q_tokens + kQueryBlock - 1) / kQueryBlock;
+    const int64_t qb = (call.q_tokens + kQueryBlock - 1) / kQueryBlock;
     if (batch_heads > 65535 || qb > 65535) return set_error(AB_ERR_INVALID, "paged_prefill: grid too large");
-    if (dense) samples = (kv_tokens / kKvBlock + 7) / 8 * 8;
-    if (samples <= 0 || samples % 8)
+    if (call.dense) call.samples = (call.kv_tokens / kKvBlock + 7) / 8 * 8;
+    if (call.samples <= 0 || call.samples % 8)
         return set_error(AB_ERR_INVALID, "paged_prefill: samples must be a positive multiple of 8");
-    if (!q || !k || !v || !out || (!dense && (!ids || !log_weights)))
+    if (!call.q || !call.k || !call.v || !call.out || (!call.dense && (!call.ids || !call.log_weights)))
         return set_error(AB_ERR_INVALID, "paged_prefill: null pointer");
-    if (!aligned16(q) || !aligned16(k) || !aligned16(v) || (reinterpret_cast<uintptr_t>(out) & 7u))
+    if (!aligned16(call.q) || !aligned16(call.k) || !aligned16(call.v) || (reinterpret_cast<uintptr_t>(call.out) & 7u))
         return set_error(AB_ERR_INVALID, "paged_prefill: q/k/v must be 16-byte and out 8-byte aligned");
-    if (!dense && (!aligned16(ids) || !aligned16(log_weights)))
+    if (!call.dense && (!aligned16(call.ids) || !aligned16(call.log_weights)))
         return set_error(AB_ERR_INVALID, "paged_prefill: ids and log_weights must be 16-byte aligned");
     const int64_t rows = batch_heads * qb;
-    if (rows * samples > (int64_t(1) << 40)) return set_error(AB_ERR_INVALID, "paged_prefill: plan too large");
-    if (workspace) {
-        const size_t need = prefill_workspace_bytes(dense, batch_heads, q_tokens, kv_tokens, samples);
+    if (rows * call.samples > (int64_t(1) << 40)) return set_error(AB_ERR_INVALID, "paged_prefill: plan too large");
+    if (call.workspace) {
+        const size_t need = prefill_workspace_bytes(call.dense, batch_heads, call.q_tokens, call.kv_tokens, call.samples);
         if (workspace_bytes < need)
             return set_error(AB_ERR_INVALID, "paged_prefill: workspace of %zu bytes is smaller than the %zu required",
                              workspace_bytes, need);
-        if (!aligned16(workspace))
+        if (!aligned16(call.workspace))
             return set_error(AB_ERR_INVALID, "paged_prefill: workspace must be 16-byte aligned");
     }
-    return launch_prefill(q, k, v, dense, batch_heads, q_tokens, kv_tokens, ids, log_weights, samples, out, lse,
-                          order, workspace, static_cast<hipStream_t>(stream));
+    return launch_prefill(call, static_cast<hipStream_t>(stream));
+}
+
+// The call of the contiguous entry points.
+PrefillCall contiguous_call(const void* q, const void* k, const void* v, const int32_t* order, int64_t batch_heads,
+                            int64_t q_tokens, int64_t kv_tokens, const int32_t* ids, const float* log_weights,
+                            int64_t samples, void* out, float* lse) {
+    PrefillCall c{};
+    c.q = q;
+    c.k = k;
+    c.v = v;
+    c.out = out;
+    c.lse = lse;
+    c.layout.q = c.layout.out = contiguous_layout(q_tokens);
+    c.layout.k = c.layout.v = contiguous_layout(kv_tokens);
+    c.layout.heads = divisor(std::clamp<int64_t>(batch_heads, 0, 65536));  // 65,536: rejected
+    c.batch = 1;
+    c.q_tokens = q_tokens;
+    c.kv_tokens = kv_tokens;
+    c.samples = samples;
+    c.ids = ids;
+    c.log_weights = log_weights;
+    c.order = order;
+    return c;
 }
 }  // namespace
 
 int ab_paged_prefill_kv(const void* q, const void* k, const void* v, int64_t batch_heads, int64_t q_tokens,
                         int64_t kv_tokens, const int32_t* ids, const float* log_weights, int64_t samples,
                         void* out, float* lse, void* stream) {
-    return paged_prefill_checked(q, k, v, false, nullptr, batch_heads, q_tokens, kv_tokens, ids, log_weights,
-                                 samples, out, lse, nullptr, 0, stream);
+    return prefill_checked(contiguous_call(q, k, v, nullptr, batch_heads, q_tokens, kv_tokens, ids, log_weights,
+                                           samples, out, lse), 0, stream);
 }
 
 int ab_dense_prefill(const void* q, const void* k, const void* v, int64_t batch_heads, int64_t q_tokens,
                      int64_t kv_tokens, void* out, float* lse, void* stream) {
-    return paged_prefill_checked(q, k, v, true, nullptr, batch_heads, q_tokens, kv_tokens, nullptr, nullptr, 0,
-                                 out, lse, nullptr, 0, stream);
+    PrefillCall c = contiguous_call(q, k, v, nullptr, batch_heads, q_tokens, kv_tokens, nullptr, nullptr, 0, out, lse);
+    c.dense = true;
+    return prefill_checked(c, 0, stream);
 }
 
 size_t ab_prefill_workspace_bytes(int64_t batch_heads, int64_t q_tokens, int64_t kv_tokens, int64_t samples) {
@@ -393,10 +440,27 @@ size_t ab_prefill_workspace_bytes(int64_t batch_heads, int64_t q_tokens, int64_t
 
 int ab_prefill(const ab_prefill_args* a, void* stream) {
     if (!a) return set_error(AB_ERR_INVALID, "paged_prefill: null pointer");
-    const bool dense = a->samples == AB_PREFILL_DENSE;
-    return paged_prefill_checked(a->q, a->k, a->v, dense, a->order, a->batch_heads, a->q_tokens, a->kv_tokens,
-                                 a->ids, a->log_weights, a->samples, a->out, a->lse, a->workspace,
-                                 a->workspace_bytes, stream);
+    PrefillCall c{};
+    if (int rc = tensor_layout("paged_prefill", a->q_stride, 8, c.layout.q)) return rc;
+    if (int rc = tensor_layout("paged_prefill", a->k_stride, 8, c.layout.k)) return rc;
+    if (int rc = tensor_layout("paged_prefill", a->v_stride, 8, c.layout.v)) return rc;
+    if (int rc = tensor_layout("paged_prefill", a->out_stride, 4, c.layout.out)) return rc;
+    c.layout.heads = divisor(std::clamp<int64_t>(a->heads, 0, 65536));  // 65,536: rejected
+    c.batch = a->batch;
+    c.q = a->q;
+    c.k = a->k;
+    c.v = a->v;
+    c.out = a->out;
+    c.lse = a->lse;
+    c.q_tokens = a->q_tokens;
+    c.kv_tokens = a->kv_tokens;
+    c.dense = a->samples == AB_PREFILL_DENSE;
+    c.samples = a->samples;
+    c.ids = a->ids;
+    c.log_weights = a->log_weights;
+    c.order = a->order;
+    c.workspace = a->workspace;
+    return prefill_checked(c, a->workspace_bytes, stream);
 }
 
 int ab_paged_prefill_ordered(const void* q, const void* k, const void* v, const int32_t* order,
@@ -406,8 +470,8 @@ int ab_paged_prefill_ordered(const void* q, const void* k, const void* v, const 
     if (int rc = check_qk_shape("paged_prefill", batch_heads, tokens)) return rc;
     if (samples <= 0 || samples % kBlocksPerPage)
         return set_error(AB_ERR_INVALID, "paged_prefill: samples must be a positive multiple of 32");
-    return paged_prefill_checked(q, k, v, false, order, batch_heads, tokens, tokens, ids, log_weights, samples,
-                                 out, lse, nullptr, 0, stream);
+    return prefill_checked(contiguous_call(q, k, v, order, batch_heads, tokens, tokens, ids, log_weights, samples,
+                                           out, lse), 0, stream);
 }
 
 int64_t ab_prefill_launch_slots(int64_t batch_heads, int64_t q_tokens) {

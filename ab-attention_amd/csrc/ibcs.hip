@@ -21,6 +21,7 @@
 #include <cfloat>
 
 #include "common.hpp"
+#include "layout.hpp"
 #include "masses.hpp"
 
 namespace ab {
@@ -113,7 +114,7 @@ __device__ __forceinline__ float block_elem_sel(const uint32_t* block, int row, 
 
 __global__ __launch_bounds__(kClusterThreads) __attribute__((amdgpu_waves_per_eu(3, 3))) void cluster_pool_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
-    uint16_t* __restrict__ centroids, float* __restrict__ pops, uint16_t* __restrict__ pooled,
+    QkLayout layout, uint16_t* __restrict__ centroids, float* __restrict__ pops, uint16_t* __restrict__ pooled,
     int64_t n, int64_t qb, float qk_scale_log2, const int32_t* __restrict__ order) {
     __shared__ uint32_t half_block[kHalfRows * kRowWords];
     __shared__ __align__(16) float center_row[kHeadDim];
@@ -132,26 +133,29 @@ __global__ __launch_bounds__(kClusterThreads) __attribute__((amdgpu_waves_per_eu
     // (256 bytes). Token t of the head is stored row t, or order[t] for a
     // permuted token layout (clamped into the head); rows past the sequence
     // end are clamped and their data discarded. Offsets are in 16-byte units
-    // from the head's base (32-bit: a head has at most 131,072 tokens).
-    const u32x4* qhead = reinterpret_cast<const u32x4*>(q + bh * n * kHeadDim);
-    const u32x4* khead = reinterpret_cast<const u32x4*>(k + bh * n * kHeadDim);
+    // from the head's base (32-bit, checked by the launcher).
+    uint32_t h;
+    const uint32_t b = layout.heads.quotient(layout.first_head + blockIdx.y, h);
+    const u32x4* qhead = reinterpret_cast<const u32x4*>(q + layout.q.at(b, h, 0));
+    const u32x4* khead = reinterpret_cast<const u32x4*>(k + layout.k.at(b, h, 0));
+    const uint32_t q_row = layout.q.token / 2u, k_row = layout.k.token / 2u;
     const int c16 = tid & 15, r0 = tid >> 4;
     const int pairs = valid / 2;
     const int nm1 = static_cast<int>(n - 1), b32 = static_cast<int>(base);
-    auto stored = [&](int t) {  // t: token index inside the block
+    auto stored = [&](int t, uint32_t row) {  // t: token index inside the block; its offset
         const int tok = b32 + min(t, valid - 1);
-        return order ? min(max(order[tok], 0), nm1) : tok;
+        return uint32_t(__umul24(order ? min(max(order[tok], 0), nm1) : tok, row));
     };
     u32x4 ka[8], kb[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         const int p = r0 + 8 * i;
-        ka[i] = khead[uint32_t(stored(2 * p)) * 16u + c16];
-        kb[i] = khead[uint32_t(stored(2 * p + 1)) * 16u + c16];
+        ka[i] = khead[stored(2 * p, k_row) + c16];
+        kb[i] = khead[stored(2 * p + 1, k_row) + c16];
     }
     f32x4 x[32];
     {
-        const uint32_t qoff = uint32_t(stored(tid)) * 16u;
+        const uint32_t qoff = stored(tid, q_row);
         u32x4 qv[16];
 #pragma unroll
         for (int j = 0; j < 16; ++j) qv[j] = qhead[qoff + j];
@@ -348,14 +352,17 @@ __global__ __launch_bounds__(kMassThreads) void masses_kernel(
 
 int64_t lse_stride(int64_t fb) { return (fb + 63) / 64 * 64; }
 
-int launch_cluster_pool(const void* q, const void* k, int64_t bh, int64_t n, void* centroids,
+int launch_cluster_pool(const void* q, const void* k, const QkLayout& layout, int64_t bh, int64_t n, void* centroids,
                         float* pops, void* pooled, float qk_scale_log2, const int32_t* order, hipStream_t stream) {
-    // The kernel addresses a head with 32-bit offsets.
+    // The kernel addresses a head with 32-bit offsets in 16-byte units, made of 24-bit factors.
     if (n <= 0 || n > kMaxKvBlocks * kKvBlock) return set_error(1, "ibcs: %lld tokens per head", (long long)n);
+    for (const TensorLayout* t : {&layout.q, &layout.k})
+        if (t->token / 2 >= (1u << 24) || n * int64_t(t->token / 2) > int64_t(0xffffffff))
+            return set_error(1, "ibcs: token stride of %lld is too large", 4 * (long long)t->token);
     const int64_t qb = (n + kQueryBlock - 1) / kQueryBlock;
     dim3 grid(static_cast<unsigned>(qb), static_cast<unsigned>(bh));
     hipLaunchKernelGGL(cluster_pool_kernel, grid, dim3(kClusterThreads), 0, stream,
-                       static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(k),
+                       static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(k), layout,
                        static_cast<uint16_t*>(centroids), pops, static_cast<uint16_t*>(pooled), n, qb,
                        qk_scale_log2, order);
     return check_launch("cluster_pool_kernel");

@@ -63,6 +63,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "layout.hpp"
 
 namespace ab {
 namespace {
@@ -159,6 +160,21 @@ __device__ __forceinline__ void max_over_rows(float& a, float& b) {
     b = __uint_as_float(u[1]);
 }
 
+// Bytes from one token's row of a head of K or V to the next. kPacked, for
+// tensors whose tokens lie 256 bytes apart (contiguous ones and token slices
+// of them), has it at compile time: with one kernel for every stride the c2
+// prefill took 24.36 instead of 23.78 ms.
+template <bool kPacked>
+__device__ __forceinline__ uint32_t token_bytes(const TensorLayout& t) {
+    return kPacked ? kHeadDim * 2u : t.token * 8u;
+}
+// Byte offset of a page. Both factors are under 2^24, so this and the lane's
+// offset added to it are one instruction at any stride.
+template <bool kPacked>
+__device__ __forceinline__ uint32_t page_offset(uint32_t id, uint32_t page_bytes) {
+    return kPacked ? id * kPageBytes : __umul24(id, page_bytes);
+}
+
 // XCD-aware row order of the prefill kernels. The hardware deals workgroups
 // round-robin over the 8 XCDs, so workgroup w runs on XCD w % 8. Slot w / 8
 // walks the heads in order: at any time all XCDs work on the same head (its
@@ -170,20 +186,31 @@ __device__ __forceinline__ void max_over_rows(float& a, float& b) {
 // the gathers into L1 hits. A launch covers the slots from slot_base (a
 // multiple of 64) on, on every XCD. False for a slot past the rows.
 struct RowSlot {
+    uint32_t b, h;  // batch item and head
     int64_t bh, blk, row;
+    __device__ __forceinline__ void set(uint32_t flat, uint32_t block, const Divisor& heads, int64_t qb) {
+        b = heads.quotient(flat, h);
+        bh = flat;
+        blk = block;
+        row = bh * qb + blk;
+    }
 };
-__device__ __forceinline__ bool row_slot(int64_t slot_base, int64_t qb, int64_t rows, RowSlot& rs) {
-    const int64_t hw = blockIdx.x;
-    const int64_t xcd = hw & 7, slot0 = slot_base + (hw >> 3);
-    const int64_t per_xcd = (qb + 7) / 8;
-    const int64_t generation = slot0 >> 6, s64 = slot0 & 63;
-    const int64_t slot = (generation + 1) * 64 <= per_xcd * (rows / qb)
-                             ? generation * 64 + 2 * (s64 & 31) + (s64 >> 5)
-                             : slot0;
-    rs.bh = slot / per_xcd;
-    rs.blk = xcd * per_xcd + slot % per_xcd;
-    if (rs.bh >= rows / qb || rs.blk >= qb) return false;
-    rs.row = rs.bh * qb + rs.blk;
+// Rows of a call: query blocks per head, the same in one of 8 groups rounded
+// up, flattened heads, first slot of the launch.
+struct RowGrid {
+    uint32_t qb;
+    Divisor per_xcd;
+    uint32_t bh, slot_base;
+};
+__device__ __forceinline__ bool row_slot(const RowGrid& g, const Divisor& heads, RowSlot& rs) {
+    const uint32_t hw = blockIdx.x;
+    const uint32_t xcd = hw & 7, slot0 = g.slot_base + (hw >> 3);
+    const uint32_t generation = slot0 >> 6, s64 = slot0 & 63;
+    const uint32_t slot = (generation + 1) * 64 <= g.per_xcd.d * g.bh ? generation * 64 + 2 * (s64 & 31) + (s64 >> 5) : slot0;
+    uint32_t rest;
+    const uint32_t flat = g.per_xcd.quotient(slot, rest), blk = xcd * g.per_xcd.d + rest;
+    if (flat >= g.bh || blk >= g.qb) return false;
+    rs.set(flat, blk, heads, g.qb);
     return true;
 }
 
@@ -196,15 +223,14 @@ struct UnitSlot : RowSlot {
     int64_t unit;
     int part;
 };
-__device__ __forceinline__ bool unit_slot(int64_t qb, int64_t rows, int parts, UnitSlot& us) {
-    const int64_t units = rows * parts, per_xcd = (units + 7) / 8;
-    const int64_t hw = blockIdx.x;
-    us.unit = (hw & 7) * per_xcd + (hw >> 3);
-    if ((hw >> 3) >= per_xcd || us.unit >= units) return false;
-    us.blk = us.unit % qb;
-    us.part = static_cast<int>((us.unit / qb) % parts);
-    us.bh = us.unit / (qb * parts);
-    us.row = us.bh * qb + us.blk;
+__device__ __forceinline__ bool unit_slot(const RowGrid& g, const Divisor& heads, uint32_t parts, UnitSlot& us) {
+    const uint32_t units = g.qb * g.bh * parts, per_xcd = (units + 7) / 8;
+    const uint32_t hw = blockIdx.x, unit = (hw & 7) * per_xcd + (hw >> 3);
+    if ((hw >> 3) >= per_xcd || unit >= units) return false;
+    const uint32_t head_part = unit / g.qb, flat = head_part / parts;
+    us.set(flat, unit - head_part * g.qb, heads, g.qb);
+    us.unit = unit;
+    us.part = static_cast<int>(head_part - flat * parts);
     return true;
 }
 // Tiles [first, first + count) of part `part` of `parts` (parts <= tiles, so
@@ -226,43 +252,46 @@ struct Partials {
     float2* stat;  // [units][kQueryBlock]
     int parts;
 };
+struct NoPartials {};
+template <bool kSplit>
+using PartialsArg = std::conditional_t<kSplit, Partials, NoPartials>;
 
 // The sparse prefill: the row's listed KV4 blocks, with their log weights.
 // kSplit: one part of the row's tiles, its result left in `partials`.
-template <bool kSplit>
+template <bool kSplit, bool kPacked>
 __global__ __launch_bounds__(kPfThreads, 2) void prefill_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
     const int32_t* __restrict__ ids, const float* __restrict__ logw, uint16_t* __restrict__ out,
-    float* __restrict__ lse, int64_t n, int64_t n_kv, int64_t qb, int64_t rows, int fb, int row_samples,
-    float scale_log2, const int32_t* __restrict__ order, int64_t slot_base, Partials partials) {
+    float* __restrict__ lse, PrefillLayout layout, int n, RowGrid grid, int fb, int row_samples, float scale_log2,
+    const int32_t* __restrict__ order, PartialsArg<kSplit> partials) {
     extern __shared__ __align__(16) unsigned char smem[];
 
     UnitSlot rs;
     int tile0 = 0, samples = row_samples;
     if constexpr (kSplit) {
-        if (!unit_slot(qb, rows, partials.parts, rs)) return;
+        if (!unit_slot(grid, layout.heads, partials.parts, rs)) return;
         int count;
         part_tiles(row_samples / kTilePages, partials.parts, rs.part, tile0, count);
         samples = count * kTilePages;
     } else {
-        if (!row_slot(slot_base, qb, rows, rs)) return;
+        if (!row_slot(grid, layout.heads, rs)) return;
     }
     const int64_t bh = rs.bh, blk = rs.blk, row = rs.row;
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int qi = lane & 31, half = lane >> 5;
-    const int64_t token = blk * kQueryBlock + wave * 32 + qi;
+    const int token = static_cast<int>(blk) * kQueryBlock + wave * 32 + qi;
     const bool valid_q = token < n;
     // Row of Q / out / lse holding this token: the token itself, or
     // order[token] for a permuted token layout (clamped into the head).
-    const int64_t qrow_index = !valid_q ? 0 : order ? min<int64_t>(max(order[token], 0), n - 1) : token;
+    const int qrow_index = !valid_q ? 0 : order ? min(max(order[token], 0), n - 1) : token;
     const int tiles = samples / kTilePages;
 
     // Q as the B operand of S^T = K Q^T: dims 16s + 8*half .. +8.
     bf16x8 bq[8];
     {
-        const uint16_t* qrow = q + (bh * n + qrow_index) * kHeadDim + 8 * half;
+        const uint16_t* qrow = q + layout.q.at(rs.b, rs.h, qrow_index) + 8 * half;
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
             u32x4 val = {0u, 0u, 0u, 0u};
@@ -274,8 +303,9 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_kernel(
     const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_u8*)smem));
     const int32_t* row_ids = ids + row * int64_t(row_samples) + tile0 * kTilePages;
     const float* row_w = logw + row * int64_t(row_samples) + tile0 * kTilePages;
-    const uint16_t* kbase = k + bh * n_kv * kHeadDim;
-    const uint16_t* vbase = v + bh * n_kv * kHeadDim;
+    const uint16_t* kbase = k + layout.k.at(rs.b, rs.h, 0);
+    const uint16_t* vbase = v + layout.v.at(rs.b, rs.h, 0);
+    const uint32_t k_token = token_bytes<kPacked>(layout.k), v_token = token_bytes<kPacked>(layout.v);
 
     // Batch b of ids and weights (tiles 64b .. 64b+63) into buffer b & 1, by
     // wave 0: two 1 KiB transfers each. Lanes past the row's end re-read its
@@ -292,7 +322,7 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_kernel(
     };
 
     // Transfers of this wave: pages 2w and 2w+1 of a K tile and of a V tile.
-    // Source offsets inside a page (1 KiB = 4 keys x 256 B) for lane j:
+    // Source offsets inside a page (4 keys x 256 B) for lane j:
     //   K: key r = j/16 at LDS chunk position j%16 holds chunk pos ^ (key & 15);
     //   V: block m = j/8, row slot (j/2)%4 holds key slot ^ ((m>>1)&3), dims 16m + 8(j%2).
     uint32_t k_src[2];
@@ -300,11 +330,11 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_kernel(
     for (int e = 0; e < 2; ++e) {
         const int r = lane >> 4, pos = lane & 15;
         const int key = 4 * (2 * wave + e) + r;
-        k_src[e] = uint32_t(r * 16 + (pos ^ (key & 15))) * 16u;
+        k_src[e] = uint32_t(r) * k_token + uint32_t(pos ^ (key & 15)) * 16u;
     }
     const uint32_t v_src = [&] {
         const int m = lane >> 3, sl = (lane >> 1) & 3, h = lane & 1;
-        return uint32_t((sl ^ ((m >> 1) & 3)) * 16 + 2 * m + h) * 16u;
+        return uint32_t(sl ^ ((m >> 1) & 3)) * v_token + uint32_t(2 * m + h) * 16u;
     }();
     // This wave's two page ids of tile u, clamped into the head (a malformed
     // plan can never address outside it); tiles past the row's end read its
@@ -317,11 +347,12 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_kernel(
                          uint32_t(min(max(static_cast<int>(raw[1]), 0), fb - 1))};
         return c;
     };
+    const uint32_t k_page = kKvBlock * k_token, v_page = kKvBlock * v_token;
     auto dma_k = [&](int u, uint32_t id, int e) {
-        dma16(kbase, id * kPageBytes + k_src[e], lds0 + kKRing + (u & (kRing - 1)) * kTileBytes + (2 * wave + e) * kPageBytes);
+        dma16(kbase, page_offset<kPacked>(id, k_page) + k_src[e], lds0 + kKRing + (u & (kRing - 1)) * kTileBytes + (2 * wave + e) * kPageBytes);
     };
     auto dma_v = [&](int u, uint32_t id, int e) {
-        dma16(vbase, id * kPageBytes + v_src, lds0 + kVRing + (u & (kRing - 1)) * kTileBytes + (2 * wave + e) * kPageBytes);
+        dma16(vbase, page_offset<kPacked>(id, v_page) + v_src, lds0 + kVRing + (u & (kRing - 1)) * kTileBytes + (2 * wave + e) * kPageBytes);
     };
     // The four block weights of this lane's keys in tile u: lane register r
     // holds key 8*(r/4) + 4*half + r%4, i.e. page 2(r/4) + half.
@@ -595,7 +626,7 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_kernel(
         // A query whose every listed block has weight -inf gets o = 0 and
         // lse = -inf.
         const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
-        uint16_t* orow = out + (bh * n + qrow_index) * kHeadDim;
+        uint16_t* orow = out + layout.out.at(rs.b, rs.h, qrow_index);
 #pragma unroll
         for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
@@ -604,7 +635,7 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_kernel(
                                   pack_bf16(o_acc[dt][4 * g + 2] * inv, o_acc[dt][4 * g + 3] * inv)};
                 *reinterpret_cast<u32x2*>(orow + 32 * dt + 8 * g + 4 * half) = pk;
             }
-        if (lse != nullptr && half == 0) lse[bh * n + qrow_index] = started ? m_run + log2f(l_tot) : -INFINITY;
+        if (lse != nullptr && half == 0) lse[bh * int64_t(n) + qrow_index] = started ? m_run + log2f(l_tot) : -INFINITY;
     }
 }
 
@@ -634,33 +665,33 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_kernel(
 // addresses): the four 16-lane groups of a transposing read fetch the same
 // dim block of four different pages, which then fall in opposite halves of
 // the banks.
-template <bool kSplit>
+template <bool kSplit, bool kPacked>
 __global__ __launch_bounds__(kPfThreads, 2) void dense_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
-    uint16_t* __restrict__ out, float* __restrict__ lse, int64_t n, int64_t n_kv, int64_t qb, int64_t rows, int fb,
-    int samples, float scale_log2, int64_t slot_base, Partials partials) {
+    uint16_t* __restrict__ out, float* __restrict__ lse, PrefillLayout layout, int n, RowGrid grid, int fb,
+    int samples, float scale_log2, PartialsArg<kSplit> partials) {
     extern __shared__ __align__(16) unsigned char smem[];
     UnitSlot rs;
     int tile0 = 0, tiles = samples / kTilePages;
     if constexpr (kSplit) {
-        if (!unit_slot(qb, rows, partials.parts, rs)) return;
+        if (!unit_slot(grid, layout.heads, partials.parts, rs)) return;
         part_tiles(samples / kTilePages, partials.parts, rs.part, tile0, tiles);
     } else {
-        if (!row_slot(slot_base, qb, rows, rs)) return;
+        if (!row_slot(grid, layout.heads, rs)) return;
     }
     const int64_t bh = rs.bh, blk = rs.blk;
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 15, lg = lane >> 4;
-    auto token_of = [&](int j) { return blk * kQueryBlock + wave * 32 + 16 * j + li; };
+    auto token_of = [&](int j) { return static_cast<int>(blk) * kQueryBlock + wave * 32 + 16 * j + li; };
 
     // Q as the B operand of S^T = K Q^T: query 16j + li, dims 32ks + 8lg .. +8.
     bf16x8 bq[2][4];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-        const int64_t token = token_of(j);
-        const uint16_t* qrow = q + (bh * n + min<int64_t>(token, n - 1)) * kHeadDim + 8 * lg;
+        const int token = token_of(j);
+        const uint16_t* qrow = q + layout.q.at(rs.b, rs.h, min(token, n - 1)) + 8 * lg;
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
             u32x4 val = {0u, 0u, 0u, 0u};
@@ -670,11 +701,12 @@ __global__ __launch_bounds__(kPfThreads, 2) void dense_kernel(
     }
 
     const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_u8*)smem));
-    const uint16_t* kbase = k + bh * n_kv * kHeadDim;
-    const uint16_t* vbase = v + bh * n_kv * kHeadDim;
+    const uint16_t* kbase = k + layout.k.at(rs.b, rs.h, 0);
+    const uint16_t* vbase = v + layout.v.at(rs.b, rs.h, 0);
+    const uint32_t k_token = token_bytes<kPacked>(layout.k), v_token = token_bytes<kPacked>(layout.v);
 
     // Transfers of this wave: pages 2w + e (e = 0, 1) of a K tile and of a V
-    // tile. Source offsets inside a page (1 KiB = 4 keys x 256 B) for lane j:
+    // tile. Source offsets inside a page (4 keys x 256 B) for lane j:
     //   K: key r = j/16 at LDS chunk position j%16 holds chunk pos ^ (key & 15);
     //   V: 128-byte position P = j/8 holds dim block m = P ^ e, key (j/2)%4,
     //      dims 16m + 8(j%2).
@@ -683,9 +715,9 @@ __global__ __launch_bounds__(kPfThreads, 2) void dense_kernel(
     for (int e = 0; e < 2; ++e) {
         const int r = lane >> 4, pos = lane & 15;
         const int key = 4 * (2 * wave + e) + r;
-        k_src[e] = uint32_t(r * 16 + (pos ^ (key & 15))) * 16u;
+        k_src[e] = uint32_t(r) * k_token + uint32_t(pos ^ (key & 15)) * 16u;
         const int P = lane >> 3, sl = (lane >> 1) & 3, h = lane & 1;
-        v_src[e] = uint32_t(sl * 256 + (2 * (P ^ e) + h) * 16);
+        v_src[e] = uint32_t(sl) * v_token + uint32_t(2 * (P ^ e) + h) * 16u;
     }
     // This wave's two pages of tile u, clamped into the head; tiles past the
     // row's end read its last tile (their transfers only keep the per-step
@@ -695,11 +727,12 @@ __global__ __launch_bounds__(kPfThreads, 2) void dense_kernel(
         const u32x2 c = {uint32_t(min(id, fb - 1)), uint32_t(min(id + 1, fb - 1))};
         return c;
     };
+    const uint32_t k_page = kKvBlock * k_token, v_page = kKvBlock * v_token;
     auto dma_k = [&](int u, uint32_t id, int e) {
-        dma16(kbase, id * kPageBytes + k_src[e], lds0 + kKRing + (u & (kRing - 1)) * kTileBytes + (2 * wave + e) * kPageBytes);
+        dma16(kbase, page_offset<kPacked>(id, k_page) + k_src[e], lds0 + kKRing + (u & (kRing - 1)) * kTileBytes + (2 * wave + e) * kPageBytes);
     };
     auto dma_v = [&](int u, uint32_t id, int e) {
-        dma16(vbase, id * kPageBytes + v_src[e], lds0 + kVRing + (u & (kRing - 1)) * kTileBytes + (2 * wave + e) * kPageBytes);
+        dma16(vbase, page_offset<kPacked>(id, v_page) + v_src[e], lds0 + kVRing + (u & (kRing - 1)) * kTileBytes + (2 * wave + e) * kPageBytes);
     };
     // The weights of this lane's keys in tile u: pages lg and 4 + lg, 0 inside
     // K/V and -inf past its end.
@@ -968,7 +1001,7 @@ __global__ __launch_bounds__(kPfThreads, 2) void dense_kernel(
         const float l16 = __uint_as_float(s16[0]) + __uint_as_float(s16[1]);
         const auto s32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(l16), __float_as_uint(l16), false, false);
         const float l_tot = __uint_as_float(s32[0]) + __uint_as_float(s32[1]);
-        const int64_t token = token_of(j);
+        const int token = token_of(j);
         if constexpr (kSplit) {
             f32x4* dst = partials.o + rs.unit * (kFragments * kPfThreads) + tid;
 #pragma unroll
@@ -982,14 +1015,14 @@ __global__ __launch_bounds__(kPfThreads, 2) void dense_kernel(
             // A query whose every block has weight -inf (none here while K/V
             // is not empty) gets o = 0 and lse = -inf.
             const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
-            uint16_t* orow = out + (bh * n + token) * kHeadDim + 4 * lg;
+            uint16_t* orow = out + layout.out.at(rs.b, rs.h, token) + 4 * lg;
 #pragma unroll
             for (int dt = 0; dt < 8; ++dt) {
                 const u32x2 pk = {pack_bf16(o_acc[dt][j][0] * inv, o_acc[dt][j][1] * inv),
                                   pack_bf16(o_acc[dt][j][2] * inv, o_acc[dt][j][3] * inv)};
                 *reinterpret_cast<u32x2*>(orow + 16 * dt) = pk;
             }
-            if (lse != nullptr && lg == 0) lse[bh * n + token] = thr[j] == kSlack ? m_run[j] + log2f(l_tot) : -INFINITY;
+            if (lse != nullptr && lg == 0) lse[bh * int64_t(n) + token] = thr[j] == kSlack ? m_run[j] + log2f(l_tot) : -INFINITY;
         }
     }
 }
@@ -1002,13 +1035,17 @@ __global__ __launch_bounds__(kPfThreads, 2) void dense_kernel(
 // together. Thread t holds the fragments thread t of the split kernel stored
 // (kDense: its layout).
 template <bool kDense>
-__global__ __launch_bounds__(kPfThreads) void combine_kernel(Partials partials, int64_t qb, int64_t n,
-                                                             uint16_t* __restrict__ out, float* __restrict__ lse,
+__global__ __launch_bounds__(kPfThreads) void combine_kernel(Partials partials, PrefillLayout layout, uint32_t qb,
+                                                             int64_t n, uint16_t* __restrict__ out,
+                                                             float* __restrict__ lse,
                                                              const int32_t* __restrict__ order) {
     constexpr int kQueries = kDense ? 2 : 1;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int64_t row = blockIdx.x, bh = row / qb, blk = row % qb;
-    const int64_t unit0 = bh * partials.parts * qb + blk;  // part p: unit0 + p * qb
+    RowSlot rs;
+    const uint32_t flat = blockIdx.x / qb;
+    rs.set(flat, blockIdx.x - flat * qb, layout.heads, qb);
+    const int64_t bh = rs.bh, blk = rs.blk;
+    const int64_t unit0 = bh * partials.parts * int64_t(qb) + blk;  // part p: unit0 + p * qb
     const int f0 = blockIdx.y * kCombineFragments;
     // Query of the thread's fragment f: 16 (f % 2) + lane % 16 (dense) or lane % 32 of the wave's 32.
     int query[kQueries];
@@ -1023,13 +1060,13 @@ __global__ __launch_bounds__(kPfThreads) void combine_kernel(Partials partials, 
     for (int p = 0; p < partials.parts; ++p)
 #pragma unroll
         for (int j = 0; j < kQueries; ++j)
-            m[j] = fmaxf(m[j], partials.stat[(unit0 + p * qb) * kQueryBlock + query[j]].x);
+            m[j] = fmaxf(m[j], partials.stat[(unit0 + p * int64_t(qb)) * kQueryBlock + query[j]].x);
     f32x4 acc[kCombineFragments];
 #pragma unroll
     for (int e = 0; e < kCombineFragments; ++e) acc[e] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 8
     for (int p = 0; p < partials.parts; ++p) {
-        const int64_t unit = unit0 + p * qb;
+        const int64_t unit = unit0 + p * int64_t(qb);
         const f32x4* src = partials.o + unit * (kFragments * kPfThreads) + f0 * kPfThreads + tid;
         f32x4 part[kCombineFragments];
 #pragma unroll
@@ -1051,17 +1088,18 @@ __global__ __launch_bounds__(kPfThreads) void combine_kernel(Partials partials, 
     for (int j = 0; j < kQueries; ++j) {
         const int64_t token = blk * kQueryBlock + query[j];
         if (token >= n) continue;
-        const int64_t at = bh * n + (order ? min<int64_t>(max(order[token], 0), n - 1) : token);
+        const int64_t at = order ? min<int64_t>(max(order[token], 0), n - 1) : token;
+        uint16_t* orow = out + layout.out.at(rs.b, rs.h, at);
         const float inv = total[j] > 0.f ? 1.0f / total[j] : 0.f;
 #pragma unroll
         for (int e = j; e < kCombineFragments; e += kQueries) {
             const int f = f0 + e;
             const int dim = kDense ? 16 * (f >> 1) + 4 * (lane >> 4) : 32 * (f >> 2) + 8 * (f & 3) + 4 * (lane >> 5);
             const u32x2 pk = {pack_bf16(acc[e][0] * inv, acc[e][1] * inv), pack_bf16(acc[e][2] * inv, acc[e][3] * inv)};
-            *reinterpret_cast<u32x2*>(out + at * kHeadDim + dim) = pk;
+            *reinterpret_cast<u32x2*>(orow + dim) = pk;
         }
         if (lse != nullptr && f0 == 0 && lane < (kDense ? 16 : 32))
-            lse[at] = m[j] > -INFINITY ? m[j] + log2f(total[j]) : -INFINITY;
+            lse[bh * n + at] = m[j] > -INFINITY ? m[j] + log2f(total[j]) : -INFINITY;
     }
 }
 
@@ -1183,56 +1221,68 @@ size_t prefill_workspace_bytes(bool dense, int64_t bh, int64_t n, int64_t n_kv, 
     return parts == 1 ? 0 : units * (kFragments * kPfThreads * sizeof(f32x4) + kQueryBlock * sizeof(float2));
 }
 
-int launch_prefill(const void* q, const void* k, const void* v, bool dense, int64_t bh, int64_t n, int64_t n_kv,
-                   const int32_t* ids, const float* logw, int64_t samples, void* out, float* lse,
-                   const int32_t* order, void* workspace, hipStream_t stream) {
+int launch_prefill(const PrefillCall& c, hipStream_t stream) {
+    const bool dense = c.dense;
+    const int64_t bh = c.batch * c.layout.heads.d, n = c.q_tokens, n_kv = c.kv_tokens, samples = c.samples;
     const int64_t qb = (n + kQueryBlock - 1) / kQueryBlock;
     const int64_t rows = bh * qb;
     if (samples % kTilePages != 0)
         return set_error(1, "prefill: samples (%lld) must be a multiple of %d", (long long)samples, kTilePages);
-    if (!dense && ((reinterpret_cast<uintptr_t>(ids) & 15u) || (reinterpret_cast<uintptr_t>(logw) & 15u)))
+    if (!dense && ((reinterpret_cast<uintptr_t>(c.ids) & 15u) || (reinterpret_cast<uintptr_t>(c.log_weights) & 15u)))
         return set_error(1, "prefill: ids and log_weights must be 16-byte aligned");
-    if (n_kv * kHeadDim * 2 > int64_t(0xffffffff))
-        return set_error(1, "prefill: one head of K/V must be under 4 GiB");
+    // The kernels address a head of K/V with 32-bit byte offsets made of 24-bit factors.
+    for (const TensorLayout* t : {&c.layout.k, &c.layout.v})
+        if (int64_t(t->token) * 8 * kKvBlock >= (1 << 24) || n_kv / kKvBlock >= (1 << 24) ||
+            n_kv * t->token * 8 > int64_t(0xffffffff))
+            return set_error(1, "prefill: one head of K/V must be under 4 GiB");
     const float scale_log2 = static_cast<float>(1.4426950408889634 / 11.313708498984761);  // log2(e)/sqrt(128)
     const int64_t per_xcd = (qb + 7) / 8;
     if (rows == 0) return 0;
-    const int parts = workspace ? call_parts(dense, bh, n, n_kv, samples) : 1;
+    const int parts = c.workspace ? call_parts(dense, bh, n, n_kv, samples) : 1;
     const int lds_bytes = dense ? kDenseLdsBytes : kLdsBytes;
     const int fb = static_cast<int>(n_kv / kKvBlock), s = static_cast<int>(samples);
     const dim3 block(kPfThreads);
-    auto launch = [&](auto split, int64_t workgroups, int64_t slot_base, Partials partials) -> int {
-        constexpr bool kSplit = decltype(split)::value;
-        const void* kernel = dense ? reinterpret_cast<const void*>(dense_kernel<kSplit>)
-                                   : reinterpret_cast<const void*>(prefill_kernel<kSplit>);
+    uint16_t* out = static_cast<uint16_t*>(c.out);
+    auto launch_as = [&](auto split, auto packed, int64_t workgroups, int64_t slot_base, auto partials) -> int {
+        const RowGrid rows_of{static_cast<uint32_t>(qb), divisor(static_cast<uint32_t>(per_xcd)),
+                              static_cast<uint32_t>(bh), static_cast<uint32_t>(slot_base)};
+        constexpr bool kSplit = decltype(split)::value, kPacked = decltype(packed)::value;
+        const auto dense_fn = dense_kernel<kSplit, kPacked>;
+        const auto sparse_fn = prefill_kernel<kSplit, kPacked>;
+        const void* kernel = dense ? reinterpret_cast<const void*>(dense_fn) : reinterpret_cast<const void*>(sparse_fn);
         if (int rc = ensure_lds_limit(kernel, lds_bytes)) return rc;
         const dim3 grid(static_cast<unsigned>(workgroups));
         if (dense)
-            hipLaunchKernelGGL(dense_kernel<kSplit>, grid, block, lds_bytes, stream, static_cast<const uint16_t*>(q),
-                               static_cast<const uint16_t*>(k), static_cast<const uint16_t*>(v),
-                               static_cast<uint16_t*>(out), lse, n, n_kv, qb, rows, fb, s, scale_log2, slot_base,
+            hipLaunchKernelGGL(dense_fn, grid, block, lds_bytes, stream,
+                               static_cast<const uint16_t*>(c.q), static_cast<const uint16_t*>(c.k),
+                               static_cast<const uint16_t*>(c.v), out, c.lse, c.layout, static_cast<int>(n), rows_of, fb, s, scale_log2,
                                partials);
         else
-            hipLaunchKernelGGL(prefill_kernel<kSplit>, grid, block, lds_bytes, stream, static_cast<const uint16_t*>(q),
-                               static_cast<const uint16_t*>(k), static_cast<const uint16_t*>(v), ids, logw,
-                               static_cast<uint16_t*>(out), lse, n, n_kv, qb, rows, fb, s, scale_log2, order,
-                               slot_base, partials);
+            hipLaunchKernelGGL(sparse_fn, grid, block, lds_bytes, stream,
+                               static_cast<const uint16_t*>(c.q), static_cast<const uint16_t*>(c.k),
+                               static_cast<const uint16_t*>(c.v), c.ids, c.log_weights, out, c.lse, c.layout,
+                               static_cast<int>(n), rows_of, fb, s, scale_log2, c.order, partials);
         return check_launch(dense ? "dense_kernel" : "prefill_kernel");
+    };
+    const bool packed = c.layout.k.token == kHeadDim / 4 && c.layout.v.token == kHeadDim / 4;
+    auto launch = [&](auto split, int64_t workgroups, int64_t slot_base, auto partials) {
+        return packed ? launch_as(split, std::true_type{}, workgroups, slot_base, partials)
+                      : launch_as(split, std::false_type{}, workgroups, slot_base, partials);
     };
     if (parts > 1) {
         const int64_t units = rows * parts;
         Partials partials;
-        partials.o = static_cast<f32x4*>(workspace);
+        partials.o = static_cast<f32x4*>(c.workspace);
         partials.stat = reinterpret_cast<float2*>(partials.o + units * kFragments * kPfThreads);
         partials.parts = parts;
         if (int rc = launch(std::true_type{}, (units + 7) / 8 * 8, 0, partials)) return rc;
         const dim3 grid(static_cast<unsigned>(rows), kFragments / kCombineFragments);
         if (dense)
-            hipLaunchKernelGGL(combine_kernel<true>, grid, block, 0, stream, partials, qb, n,
-                               static_cast<uint16_t*>(out), lse, order);
+            hipLaunchKernelGGL(combine_kernel<true>, grid, block, 0, stream, partials, c.layout, static_cast<uint32_t>(qb), n, out, c.lse,
+                               nullptr);
         else
-            hipLaunchKernelGGL(combine_kernel<false>, grid, block, 0, stream, partials, qb, n,
-                               static_cast<uint16_t*>(out), lse, order);
+            hipLaunchKernelGGL(combine_kernel<false>, grid, block, 0, stream, partials, c.layout, static_cast<uint32_t>(qb), n, out, c.lse,
+                               c.order);
         return check_launch("combine_kernel");
     }
     // The rows are launched in chunks of about kRowsPerLaunch, each a whole
@@ -1248,7 +1298,7 @@ int launch_prefill(const void* q, const void* k, const void* v, bool dense, int6
     const int64_t per_launch = prefill_launch_slots(bh, n);
     for (int64_t slot_base = 0; slot_base < slots; slot_base += per_launch) {
         const int64_t count = std::min(per_launch, slots - slot_base);
-        if (int rc = launch(std::false_type{}, count * 8, slot_base, Partials{nullptr, nullptr, 1})) return rc;
+        if (int rc = launch(std::false_type{}, count * 8, slot_base, NoPartials{})) return rc;
     }
     return 0;
 }

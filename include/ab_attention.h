@@ -30,7 +30,7 @@
 extern "C" {
 #endif
 
-#define AB_ABI_VERSION 5
+#define AB_ABI_VERSION 6
 
 enum ab_status {
     AB_OK = 0,
@@ -89,6 +89,23 @@ int ab_ibcs_sip(const void *q, const void *k, const int32_t *order, int64_t batc
                 const float *offsets, int64_t samples, void *workspace, size_t workspace_bytes, int32_t *ids,
                 float *log_weights, void *stream);
 
+/* ab_ibcs_sip of heads first_head .. first_head + head_count - 1 (of the
+ * flattened batch * heads) of q, k [batch, heads, tokens, 128] with strides of
+ * their own (batch, head, token; in elements, multiples of 8): only the heads'
+ * rows, offsets and workspace are passed. */
+typedef struct ab_plan_args {
+    const void *q, *k;
+    const int32_t *order;
+    const float *offsets;
+    int32_t *ids;
+    float *log_weights;
+    int64_t batch, heads, first_head, head_count, tokens, samples;
+    int64_t q_stride[3], k_stride[3];
+    void *workspace;
+    size_t workspace_bytes;
+} ab_plan_args;
+int ab_plan(const ab_plan_args *args, void *stream);
+
 /* Testing variant of ab_ibcs_sip; no counterpart in the reference. Every
  * row that is sampled with kept prefixes takes the reference's binary-search
  * probes (each prefix rebuilt from the kept ones), the path otherwise taken
@@ -136,7 +153,11 @@ int ab_dense_prefill(const void *q, const void *k, const void *v, int64_t batch_
  * samples > 0: the listed blocks, as ab_paged_prefill_kv (order NULL) or with
  * the query rows read and written through `order` int32 [q_tokens] (see
  * ab_paged_prefill_ordered); samples == AB_PREFILL_DENSE: as ab_dense_prefill
- * (ids, log_weights and order unused). With a workspace, a call whose rows would
+ * (ids, log_weights and order unused).
+ * Q, K, V and out are [batch, heads, tokens, 128] with strides of their own
+ * (batch, head, token; in elements, multiples of 8, of 4 for out; the 128 dims
+ * are contiguous), so slices of tokens and the transposed views of [batch,
+ * tokens, heads, 128] are read in place. lse is contiguous. With a workspace, a call whose rows would
  * leave much of the GPU idle (a prompt's few query blocks over a whole video,
  * a short clip) splits each row's keys over several workgroups and adds up
  * their float32 partial results; the result is the same up to float32
@@ -150,7 +171,8 @@ typedef struct ab_prefill_args {
     const float *log_weights;
     void *out;
     float *lse;
-    int64_t batch_heads, q_tokens, kv_tokens, samples;
+    int64_t batch, heads, q_tokens, kv_tokens, samples;
+    int64_t q_stride[3], k_stride[3], v_stride[3], out_stride[3];
     void *workspace;
     size_t workspace_bytes;
 } ab_prefill_args;

@@ -1,0 +1,69 @@
+"""Q, K and V that are not contiguous are read where they lie (or copied where
+their rows cannot be): every public call equals the same call on contiguous
+tensors bit for bit, for each form of strides the dispatch distinguishes."""
+import pytest
+import torch
+
+from ab_attention import _lib, apply_plan, attention, build_plan
+from ab_attention.video import apply_cube_plan, cube_plan, exact_attention
+
+B, H, N, GRID = 2, 3, 1920, (6, 16, 20)
+
+
+def _forms(x):
+    """Views equal to x [B, H, N, 128] in every layout; True: read in place."""
+    b, h, n, d = x.shape
+    wide = torch.zeros(b, h, n + 20, d, dtype=x.dtype, device=x.device)
+    wide[:, :, 12:12 + n] = x
+    odd = torch.zeros(b * h * n * d + 4, dtype=x.dtype, device=x.device)
+    odd[4:] = x.transpose(1, 2).reshape(-1)
+    packed = torch.zeros(b, n, h, 3, d, dtype=x.dtype, device=x.device)  # one projection of Q, K and V
+    packed[:, :, :, 1] = x.transpose(1, 2)
+    return {
+        "token major": (x.transpose(1, 2).contiguous().transpose(1, 2), True),
+        "token slice": (wide[:, :, 12:12 + n], True),
+        "batch inside": (x.permute(2, 0, 1, 3).contiguous().permute(1, 2, 0, 3), True),
+        "packed": (packed[:, :, :, 1].transpose(1, 2), True),
+        "misaligned rows": (odd[4:].view(b, n, h, d).transpose(1, 2), False),
+        "dims outside": (x.transpose(2, 3).contiguous().transpose(2, 3), False),
+    }
+
+
+def test_forms_read_in_place():
+    x = torch.randn(B, H, 64, 128).to(torch.bfloat16)
+    for name, (view, in_place) in _forms(x).items():
+        got, strides = _lib.in_place(view)
+        assert torch.equal(got, x), name
+        assert (got.data_ptr() == view.data_ptr()) == in_place, name
+        assert strides == got.stride()[:3], name
+    one = torch.zeros(1, 1, 64, 128).as_strided((1, 1, 64, 128), (5, 3, 128, 1))
+    assert _lib.in_place(one)[0] is one and _lib.in_place(one)[1] == (64 * 128, 64 * 128, 128)
+    still = torch.zeros(1, 1, 1, 128).expand(2, 2, 64, 128)
+    assert _lib.in_place(still)[0].is_contiguous()  # a token stride of 0 is copied
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("form", ["token major", "token slice", "batch inside", "packed", "misaligned rows",
+                                  "dims outside", "shared heads"])
+def test_layouts_equal_contiguous(form, monkeypatch):
+    print(f"layout {form}", flush=True)
+    torch.manual_seed(4)
+    q, k, v = (torch.randn(B, H, N, 128, device="cuda").to(torch.bfloat16) for _ in range(3))
+    if form == "shared heads":  # K/V of one head for all of them: a head stride of 0
+        ks, vs = k[:, :1].expand(B, H, N, 128), v[:, :1].expand(B, H, N, 128)
+        qs, k, v = q, ks.contiguous(), vs.contiguous()
+    else:
+        qs, ks, vs = (_forms(t)[form][0] for t in (q, k, v))
+    want = build_plan(q, k, sample_pages=4)
+    for heads in (B * H, 1, 4):  # heads per chunk; a chunk of 4 crosses the batch items
+        monkeypatch.setattr(attention, "_heads_per_chunk", lambda *_: heads)
+        plan = build_plan(qs, ks, sample_pages=4)
+        assert torch.equal(plan.descriptor, want.descriptor)
+        assert torch.equal(plan.log_weights.view(torch.int32), want.log_weights.view(torch.int32))
+    cube = cube_plan(qs, ks, GRID, sample_pages=4)
+    assert torch.equal(cube.descriptor, cube_plan(q, k, GRID, sample_pages=4).descriptor)
+    for call in (lambda *t: apply_plan(*t, want, return_lse=True), lambda *t: exact_attention(*t, return_lse=True),
+                 lambda *t: apply_cube_plan(*t, cube, GRID, return_lse=True)):
+        for got, ref in zip(call(qs, ks, vs), call(q, k, v)):
+            assert got.is_contiguous() and torch.equal(got, ref)
+    torch.cuda.synchronize()

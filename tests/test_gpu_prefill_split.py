@@ -21,7 +21,8 @@ def _run(q, k, v, ids, w, order, split):
     ws = torch.empty(size, dtype=torch.uint8, device="cuda") if split else None
     out = torch.full_like(q, float("nan"))
     lse = torch.full(q.shape[:3], float("nan"), device="cuda")
-    args = _lib.PrefillArgs(*(_lib.ptr(t) for t in (q, k, v, order, ids, w, out, lse)), bh, nq, nk, samples,
+    args = _lib.PrefillArgs(*(_lib.ptr(t) for t in (q, k, v, order, ids, w, out, lse)), 1, bh, nq, nk, samples,
+                            *(_lib.in_place(t)[1] for t in (q, k, v, out)),
                             _lib.ptr(ws), size if split else 0)
     _lib.check(lib.ab_prefill(args, _lib.stream(q.device)))
     torch.cuda.synchronize()
@@ -88,9 +89,13 @@ def test_split_rule():
 
 
 def test_split_rejects_a_bad_workspace():
-    lib, a = _lib.load(), 4096  # a stand-in address: rejected before any launch
+    lib, a, rows = _lib.load(), 4096, 4 * [(1 << 20, 1 << 14, 128)]  # a stand-in address: rejected before any launch
     for ws, size, message in ((a, 64, b"smaller than"), (a + 8, 1 << 30, b"16-byte aligned")):
-        args = _lib.PrefillArgs(a, a, a, None, None, None, a, None, 24, 256, 119056, _lib.PREFILL_DENSE, ws, size)
+        args = _lib.PrefillArgs(a, a, a, None, None, None, a, None, 1, 24, 256, 119056, _lib.PREFILL_DENSE, *rows, ws, size)
         assert lib.ab_prefill(args, None) == 1 and message in lib.ab_last_error()
-    args = _lib.PrefillArgs(a, a, a, None, None, None, a, None, 1, 128, 128, 0, None, 0)
+    args = _lib.PrefillArgs(a, a, a, None, None, None, a, None, 1, 1, 128, 128, 0, *rows, None, 0)
     assert lib.ab_prefill(args, None) == 1 and b"multiple of 8" in lib.ab_last_error()
+    for bad in ((1 << 20, 1 << 14, 132), (-8, 1 << 14, 128), (1 << 20, 1 << 14, 1 << 21)):
+        args = _lib.PrefillArgs(a, a, a, None, None, None, a, None, 1, 1, 128, 128, _lib.PREFILL_DENSE, rows[0], bad,
+                                *rows[:2], None, 0)
+        assert lib.ab_prefill(args, None) == 1
