@@ -38,7 +38,8 @@ class PrefillArgs(ctypes.Structure):
     _fields_ = [("q", _P), ("k", _P), ("v", _P), ("order", _P), ("ids", _P), ("log_weights", _P), ("out", _P),
                 ("lse", _P), ("batch", _I64), ("heads", _I64), ("q_tokens", _I64), ("kv_tokens", _I64),
                 ("samples", _I64), ("q_stride", _I64 * 3), ("k_stride", _I64 * 3), ("v_stride", _I64 * 3),
-                ("out_stride", _I64 * 3), ("workspace", _P), ("workspace_bytes", _SZ)]
+                ("out_stride", _I64 * 3), ("tail_ids", _P), ("tail_log_weights", _P), ("tail_samples", _I64),
+                ("workspace", _P), ("workspace_bytes", _SZ)]
 
 
 class PlanArgs(ctypes.Structure):
@@ -82,7 +83,7 @@ STATIC_SIGNATURES = {
     "ab_ibcs_sip_static": (ctypes.c_int, [_P, _P, _P, _I64, _I64, _P, _I64, _P, _P, _P]),
 }
 
-ABI_VERSION = 6
+ABI_VERSION = 7
 _lib = None
 _static = None
 

@@ -30,36 +30,41 @@ _QUERY_BLOCK = 128
 _PAGE_SIZE = 4
 
 
-def _run(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, ids, weights, samples: int, order, return_lse: bool):
-    """ab_prefill of q, k, v, read where they lie (samples: _lib.PREFILL_DENSE for dense). The workspace of a
-    call that splits its rows over more workgroups lives for the call only (the
+def _run(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, ids, weights, samples: int, order, return_lse: bool,
+         tail=(None, None, 0), out=None):
+    """ab_prefill of q, k, v, read where they lie (samples: _lib.PREFILL_DENSE for
+    dense; tail: ids, weights and count of the blocks every row attends to as
+    well; out: a view with rows of 128 to write to). The workspace of a call
+    that splits its rows over more workgroups lives for the call only (the
     caching allocator keeps it on this stream)."""
     batch, heads, tokens, dim = q.shape
     kv_tokens, device = k.shape[2], q.device
     (q, q_stride), (k, k_stride), (v, v_stride) = _lib.in_place(q), _lib.in_place(k), _lib.in_place(v)
-    output = torch.empty_like(q, memory_format=torch.contiguous_format)
+    out_stride = (heads * tokens * dim, tokens * dim, dim) if out is None else out.stride()[:3]
+    output = torch.empty_like(q, memory_format=torch.contiguous_format) if out is None else out
     lse = torch.empty((batch, heads, tokens), dtype=torch.float32, device=device) if return_lse else None
     lib, address = _lib.load(), _lib.address
+    tail_ids, tail_weights, tail_samples = tail
     with _lib.on(device):
-        ws_bytes = lib.ab_prefill_workspace_bytes(batch * heads, tokens, kv_tokens, samples)
+        ws_bytes = lib.ab_prefill_workspace_bytes(batch * heads, tokens, kv_tokens, samples + tail_samples)
         workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=device) if ws_bytes else None
         args = _lib.PrefillArgs(address(q), address(k), address(v), address(order), address(ids), address(weights),
                                 address(output), address(lse), batch, heads, tokens, kv_tokens, samples, q_stride,
-                                k_stride, v_stride, (heads * tokens * dim, tokens * dim, dim), address(workspace),
-                                ws_bytes)
+                                k_stride, v_stride, out_stride, address(tail_ids), address(tail_weights),
+                                tail_samples, address(workspace), ws_bytes)
         _lib.check(lib.ab_prefill(args, _lib.stream(device)))
     return (output, lse) if return_lse else output
 
 
 def _prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor,
-             order: torch.Tensor | None, return_lse: bool):
+             order: torch.Tensor | None, return_lse: bool, *, tail=(None, None, 0), out=None):
     """The weighted prefill, with a query token order when one is given;
     ids/weights [rows, S]. Shapes are checked by the callers."""
     if ids.dtype != torch.int32 or not ids.is_contiguous():
         ids = ids.to(torch.int32).contiguous()
     if weights.dtype != torch.float32 or not weights.is_contiguous():
         weights = weights.to(torch.float32).contiguous()
-    return _run(q, k, v, ids, weights, ids.shape[-1], order, return_lse)
+    return _run(q, k, v, ids, weights, ids.shape[-1], order, return_lse, tail, out)
 
 
 def check_prefill_inputs(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> None:
@@ -103,22 +108,22 @@ def paged_attention(
 
 
 def _prefill_kv(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor,
-                *, return_lse: bool = False):
-    """The weighted prefill with K/V of their own length.
+                *, return_lse: bool = False, tail=(None, None, 0), out=None):
+    """The weighted prefill with K/V of their own length (tail, out: see _run).
 
     q bf16 [B,H,Nq,128], k/v bf16 [B,H,Nk,128] with Nk % 4 == 0, ids int32 /
     weights f32 [B*H*ceil(Nq/128), S] with S % 8 == 0 (per-head KV4 ids; a -inf
     weight removes its block). Shapes are checked by the callers.
     """
-    return _prefill(q, k, v, ids, weights, None, return_lse)
+    return _prefill(q, k, v, ids, weights, None, return_lse, tail=tail, out=out)
 
 
-def _prefill_dense(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, return_lse: bool = False):
+def _prefill_dense(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, return_lse: bool = False, out=None):
     """Dense attention of q bf16 [B,H,Nq,128] over every key of k/v bf16
     [B,H,Nk,128] (Nk % 4 == 0) on the dense kernel (ab_dense_prefill); the
     page list is implicit, so nothing of size rows x blocks is built. Shapes
     are checked by the callers."""
-    return _run(q, k, v, None, None, _lib.PREFILL_DENSE, None, return_lse)
+    return _run(q, k, v, None, None, _lib.PREFILL_DENSE, None, return_lse, out=out)
 
 
 def _remap_ids(ids: torch.Tensor, page_map: torch.Tensor) -> torch.Tensor:

@@ -289,26 +289,28 @@ def hunyuan_attention(schedule: VideoAttention, layer: int, q: torch.Tensor, k: 
     prompt_end = video_tokens + prompt_tokens
     if video_tokens % _PAGE or prompt_tokens % _PAGE or (tokens - prompt_end) % _PAGE or prompt_end > tokens:
         raise ValueError("video, prompt and padding lengths must be divisible by 4 and fit in N")
+    # Every part reads its slices of Q, K and V in place and writes its slice of
+    # the output.
+    out = torch.empty_like(q, memory_format=torch.contiguous_format)
     if not schedule.is_sparse(layer):
-        outputs = [exact_attention(q[:, :, :prompt_end], k[:, :, :prompt_end], v[:, :, :prompt_end])]
+        seen = slice(0, prompt_end)
+        _prefill_dense(q[:, :, seen], k[:, :, seen], v[:, :, seen], out=out[:, :, seen])
     else:
-        q_video = q[:, :, :video_tokens].contiguous()
-        k_video = k[:, :, :video_tokens].contiguous()
-        k_prompt, v_prompt = k[:, :, :prompt_end].contiguous(), v[:, :, :prompt_end].contiguous()
+        video, text, seen = slice(0, video_tokens), slice(video_tokens, prompt_end), slice(0, prompt_end)
+        q_video, k_video = q[:, :, video], k[:, :, video]
         if fused:
             plan = schedule.plan(layer, q_video, k_video)
             rows = plan.descriptor.shape[0]
-            text_ids, text_w = _dense_pages(rows, prompt_tokens // _PAGE, q.device, offset=video_tokens // _PAGE)
-            ids = torch.cat([plan.descriptor.reshape(rows, -1), text_ids], dim=1)
-            weights = torch.cat([plan.log_weights.reshape(rows, -1), text_w], dim=1)
-            video_out = _prefill_kv(q_video, k_prompt, v_prompt, ids, weights)
+            text_ids, text_w = _dense_pages(1, prompt_tokens // _PAGE, q.device, offset=video_tokens // _PAGE)
+            _prefill_kv(q_video, k[:, :, seen], v[:, :, seen], plan.descriptor.reshape(rows, -1),
+                        plan.log_weights.reshape(rows, -1), tail=(text_ids, text_w, text_ids.shape[1]),
+                        out=out[:, :, video])
         else:
-            video_state = schedule.attend(layer, q_video, k_video, v[:, :, :video_tokens].contiguous(),
-                                          return_lse=True)
-            text_state = exact_attention(q_video, k[:, :, video_tokens:prompt_end], v[:, :, video_tokens:prompt_end],
-                                         return_lse=True)
-            video_out = merge_states(video_state, text_state)
-        outputs = [video_out, exact_attention(q[:, :, video_tokens:prompt_end], k_prompt, v_prompt)]
+            video_state = schedule.attend(layer, q_video, k_video, v[:, :, video], return_lse=True)
+            text_state = exact_attention(q_video, k[:, :, text], v[:, :, text], return_lse=True)
+            out[:, :, video] = merge_states(video_state, text_state)
+        _prefill_dense(q[:, :, text], k[:, :, seen], v[:, :, seen], out=out[:, :, text])
     if prompt_end < tokens:
-        outputs.append(exact_attention(q[:, :, prompt_end:], k[:, :, prompt_end:], v[:, :, prompt_end:]))
-    return torch.cat(outputs, dim=2)
+        rest = slice(prompt_end, tokens)
+        _prefill_dense(q[:, :, rest], k[:, :, rest], v[:, :, rest], out=out[:, :, rest])
+    return out

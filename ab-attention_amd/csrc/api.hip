@@ -374,16 +374,23 @@ int prefill_checked(PrefillCall call, size_t workspace_bytes, void* stream) {
     if (call.dense) call.samples = (call.kv_tokens / kKvBlock + 7) / 8 * 8;
     if (call.samples <= 0 || call.samples % 8)
         return set_error(AB_ERR_INVALID, "paged_prefill: samples must be a positive multiple of 8");
+    if (call.tail_samples < 0 || call.tail_samples % 8 || (call.dense && call.tail_samples) ||
+        call.samples + call.tail_samples > INT32_MAX / 4)
+        return set_error(AB_ERR_INVALID, "paged_prefill: the shared list must be a multiple of 8 blocks of a sparse call");
+    if (call.tail_samples && (!call.tail_ids || !call.tail_log_weights))
+        return set_error(AB_ERR_INVALID, "paged_prefill: null pointer");
     if (!call.q || !call.k || !call.v || !call.out || (!call.dense && (!call.ids || !call.log_weights)))
         return set_error(AB_ERR_INVALID, "paged_prefill: null pointer");
     if (!aligned16(call.q) || !aligned16(call.k) || !aligned16(call.v) || (reinterpret_cast<uintptr_t>(call.out) & 7u))
         return set_error(AB_ERR_INVALID, "paged_prefill: q/k/v must be 16-byte and out 8-byte aligned");
-    if (!call.dense && (!aligned16(call.ids) || !aligned16(call.log_weights)))
+    if (!call.dense && (!aligned16(call.ids) || !aligned16(call.log_weights) || !aligned16(call.tail_ids) ||
+                        !aligned16(call.tail_log_weights)))
         return set_error(AB_ERR_INVALID, "paged_prefill: ids and log_weights must be 16-byte aligned");
     const int64_t rows = batch_heads * qb;
     if (rows * call.samples > (int64_t(1) << 40)) return set_error(AB_ERR_INVALID, "paged_prefill: plan too large");
     if (call.workspace) {
-        const size_t need = prefill_workspace_bytes(call.dense, batch_heads, call.q_tokens, call.kv_tokens, call.samples);
+        const size_t need = prefill_workspace_bytes(call.dense, batch_heads, call.q_tokens, call.kv_tokens,
+                                                    call.samples + call.tail_samples);
         if (workspace_bytes < need)
             return set_error(AB_ERR_INVALID, "paged_prefill: workspace of %zu bytes is smaller than the %zu required",
                              workspace_bytes, need);
@@ -458,6 +465,9 @@ int ab_prefill(const ab_prefill_args* a, void* stream) {
     c.samples = a->samples;
     c.ids = a->ids;
     c.log_weights = a->log_weights;
+    c.tail_samples = a->tail_samples;
+    c.tail_ids = a->tail_ids;
+    c.tail_log_weights = a->tail_log_weights;
     c.order = a->order;
     c.workspace = a->workspace;
     return prefill_checked(c, a->workspace_bytes, stream);

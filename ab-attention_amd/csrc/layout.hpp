@@ -76,6 +76,9 @@ struct PrefillCall {
     int64_t samples;
     const int32_t* ids;
     const float* log_weights;
+    int64_t tail_samples;
+    const int32_t* tail_ids;
+    const float* tail_log_weights;
     const int32_t* order;
     void* workspace;
 };

@@ -124,6 +124,10 @@ __device__ __forceinline__ void dma16(const void* base, uint32_t voffset, uint32
     asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voffset), "s"(base)
                  : "memory", "m0");
 }
+// The same from an address of its own in each lane.
+__device__ __forceinline__ void dma16(const void* address, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(address) : "memory", "m0");
+}
 #pragma clang diagnostic pop
 
 // s_waitcnt with vmcnt(N) and lgkmcnt(0) (expcnt left open), then a workgroup
@@ -214,7 +218,18 @@ __device__ __forceinline__ bool row_slot(const RowGrid& g, const Divisor& heads,
     return true;
 }
 
-// The same for rows split into `parts` units each: unit (bh, part, blk), blk
+// The lists of a sparse call: row r's blocks, ids and log weights
+// [rows][samples], then the `tail` blocks that every row attends to as well
+// (a prompt behind the video; ids and weights [tail], tail 0 for none).
+struct BlockLists {
+    const int32_t* ids;
+    const float* logw;
+    int samples, tail;
+    const int32_t* tail_ids;
+    const float* tail_logw;
+};
+
+// row_slot for rows split into `parts` units each: unit (bh, part, blk), blk
 // fastest, each XCD a contiguous eighth of the units. The units of one part
 // of a head read the same stretch of its K/V (dense) or sweep the same range
 // of their ascending page lists (sparse), so they share it in the XCD's L2.
@@ -257,22 +272,22 @@ template <bool kSplit>
 using PartialsArg = std::conditional_t<kSplit, Partials, NoPartials>;
 
 // The sparse prefill: the row's listed KV4 blocks, with their log weights.
-// kSplit: one part of the row's tiles, its result left in `partials`.
-template <bool kSplit, bool kPacked>
+// kSplit: one part of the row's tiles, its result left in `partials`. kTail:
+// the shared blocks behind the row's own (at compile time: with the choice of
+// list in the kernel every call runs, c2 took 23.12 instead of 22.74 ms).
+template <bool kSplit, bool kPacked, bool kTail>
 __global__ __launch_bounds__(kPfThreads, 2) void prefill_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
-    const int32_t* __restrict__ ids, const float* __restrict__ logw, uint16_t* __restrict__ out,
-    float* __restrict__ lse, PrefillLayout layout, int n, RowGrid grid, int fb, int row_samples, float scale_log2,
+    BlockLists lists, uint16_t* __restrict__ out,
+    float* __restrict__ lse, PrefillLayout layout, int n, RowGrid grid, int fb, float scale_log2,
     const int32_t* __restrict__ order, PartialsArg<kSplit> partials) {
     extern __shared__ __align__(16) unsigned char smem[];
 
     UnitSlot rs;
-    int tile0 = 0, samples = row_samples;
+    int tile0 = 0, tiles = (lists.samples + (kTail ? lists.tail : 0)) / kTilePages;
     if constexpr (kSplit) {
         if (!unit_slot(grid, layout.heads, partials.parts, rs)) return;
-        int count;
-        part_tiles(row_samples / kTilePages, partials.parts, rs.part, tile0, count);
-        samples = count * kTilePages;
+        part_tiles(tiles, partials.parts, rs.part, tile0, tiles);
     } else {
         if (!row_slot(grid, layout.heads, rs)) return;
     }
@@ -286,7 +301,6 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_kernel(
     // Row of Q / out / lse holding this token: the token itself, or
     // order[token] for a permuted token layout (clamped into the head).
     const int qrow_index = !valid_q ? 0 : order ? min(max(order[token], 0), n - 1) : token;
-    const int tiles = samples / kTilePages;
 
     // Q as the B operand of S^T = K Q^T: dims 16s + 8*half .. +8.
     bf16x8 bq[8];
@@ -301,23 +315,34 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_kernel(
     }
 
     const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_u8*)smem));
-    const int32_t* row_ids = ids + row * int64_t(row_samples) + tile0 * kTilePages;
-    const float* row_w = logw + row * int64_t(row_samples) + tile0 * kTilePages;
+    const int first = kTail ? 0 : tile0 * kTilePages;
+    const int32_t* row_ids = lists.ids + row * int64_t(lists.samples) + first;
+    const float* row_w = lists.logw + row * int64_t(lists.samples) + first;
     const uint16_t* kbase = k + layout.k.at(rs.b, rs.h, 0);
     const uint16_t* vbase = v + layout.v.at(rs.b, rs.h, 0);
     const uint32_t k_token = token_bytes<kPacked>(layout.k), v_token = token_bytes<kPacked>(layout.v);
 
     // Batch b of ids and weights (tiles 64b .. 64b+63) into buffer b & 1, by
     // wave 0: two 1 KiB transfers each. Lanes past the row's end re-read its
-    // last 16 bytes (those entries are never used).
-    const uint32_t row_bytes = static_cast<uint32_t>(samples) * 4u;
+    // last 16 bytes (those entries are never used). kTail: 16 bytes per lane
+    // from the row's list or, past its end, from the tail.
+    const uint32_t unit_bytes = static_cast<uint32_t>(tiles) * (kTilePages * 4u);
     auto issue_batch = [&](int b) {
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-            const uint32_t src = min(uint32_t(b) * kBatchBytes + i * 1024u + 16u * lane, row_bytes - 16u);
+            const uint32_t src = min(uint32_t(b) * kBatchBytes + i * 1024u + 16u * lane, unit_bytes - 16u);
             const uint32_t dst = (b & 1) * kBatchBytes + i * 1024u;
-            dma16(row_ids, src, lds0 + kIdsOffset + dst);
-            dma16(row_w, src, lds0 + kWeightsOffset + dst);
+            if constexpr (kTail) {
+                const uint32_t at = src + static_cast<uint32_t>(tile0) * (kTilePages * 4u);
+                const uint32_t row_bytes = static_cast<uint32_t>(lists.samples) * 4u;
+                const bool tail = at >= row_bytes;
+                const uint32_t off = at - (tail ? row_bytes : 0u);
+                dma16(reinterpret_cast<const char*>(tail ? lists.tail_ids : row_ids) + off, lds0 + kIdsOffset + dst);
+                dma16(reinterpret_cast<const char*>(tail ? lists.tail_logw : row_w) + off, lds0 + kWeightsOffset + dst);
+            } else {
+                dma16(row_ids, src, lds0 + kIdsOffset + dst);
+                dma16(row_w, src, lds0 + kWeightsOffset + dst);
+            }
         }
     };
 
@@ -1226,10 +1251,13 @@ int launch_prefill(const PrefillCall& c, hipStream_t stream) {
     const int64_t bh = c.batch * c.layout.heads.d, n = c.q_tokens, n_kv = c.kv_tokens, samples = c.samples;
     const int64_t qb = (n + kQueryBlock - 1) / kQueryBlock;
     const int64_t rows = bh * qb;
-    if (samples % kTilePages != 0)
+    if (samples % kTilePages != 0 || c.tail_samples % kTilePages != 0)
         return set_error(1, "prefill: samples (%lld) must be a multiple of %d", (long long)samples, kTilePages);
-    if (!dense && ((reinterpret_cast<uintptr_t>(c.ids) & 15u) || (reinterpret_cast<uintptr_t>(c.log_weights) & 15u)))
-        return set_error(1, "prefill: ids and log_weights must be 16-byte aligned");
+    if (!dense)
+        for (const void* p : {static_cast<const void*>(c.ids), static_cast<const void*>(c.log_weights),
+                              static_cast<const void*>(c.tail_ids), static_cast<const void*>(c.tail_log_weights)})
+            if (reinterpret_cast<uintptr_t>(p) & 15u)
+                return set_error(1, "prefill: ids and log_weights must be 16-byte aligned");
     // The kernels address a head of K/V with 32-bit byte offsets made of 24-bit factors.
     for (const TensorLayout* t : {&c.layout.k, &c.layout.v})
         if (int64_t(t->token) * 8 * kKvBlock >= (1 << 24) || n_kv / kKvBlock >= (1 << 24) ||
@@ -1238,17 +1266,18 @@ int launch_prefill(const PrefillCall& c, hipStream_t stream) {
     const float scale_log2 = static_cast<float>(1.4426950408889634 / 11.313708498984761);  // log2(e)/sqrt(128)
     const int64_t per_xcd = (qb + 7) / 8;
     if (rows == 0) return 0;
-    const int parts = c.workspace ? call_parts(dense, bh, n, n_kv, samples) : 1;
+    const int parts = c.workspace ? call_parts(dense, bh, n, n_kv, samples + c.tail_samples) : 1;
     const int lds_bytes = dense ? kDenseLdsBytes : kLdsBytes;
     const int fb = static_cast<int>(n_kv / kKvBlock), s = static_cast<int>(samples);
     const dim3 block(kPfThreads);
     uint16_t* out = static_cast<uint16_t*>(c.out);
+    const BlockLists lists{c.ids, c.log_weights, s, static_cast<int>(c.tail_samples), c.tail_ids, c.tail_log_weights};
     auto launch_as = [&](auto split, auto packed, int64_t workgroups, int64_t slot_base, auto partials) -> int {
         const RowGrid rows_of{static_cast<uint32_t>(qb), divisor(static_cast<uint32_t>(per_xcd)),
                               static_cast<uint32_t>(bh), static_cast<uint32_t>(slot_base)};
         constexpr bool kSplit = decltype(split)::value, kPacked = decltype(packed)::value;
         const auto dense_fn = dense_kernel<kSplit, kPacked>;
-        const auto sparse_fn = prefill_kernel<kSplit, kPacked>;
+        const auto sparse_fn = c.tail_samples ? prefill_kernel<kSplit, kPacked, true> : prefill_kernel<kSplit, kPacked, false>;
         const void* kernel = dense ? reinterpret_cast<const void*>(dense_fn) : reinterpret_cast<const void*>(sparse_fn);
         if (int rc = ensure_lds_limit(kernel, lds_bytes)) return rc;
         const dim3 grid(static_cast<unsigned>(workgroups));
@@ -1260,8 +1289,8 @@ int launch_prefill(const PrefillCall& c, hipStream_t stream) {
         else
             hipLaunchKernelGGL(sparse_fn, grid, block, lds_bytes, stream,
                                static_cast<const uint16_t*>(c.q), static_cast<const uint16_t*>(c.k),
-                               static_cast<const uint16_t*>(c.v), c.ids, c.log_weights, out, c.lse, c.layout,
-                               static_cast<int>(n), rows_of, fb, s, scale_log2, c.order, partials);
+                               static_cast<const uint16_t*>(c.v), lists, out, c.lse, c.layout, static_cast<int>(n),
+                               rows_of, fb, scale_log2, c.order, partials);
         return check_launch(dense ? "dense_kernel" : "prefill_kernel");
     };
     const bool packed = c.layout.k.token == kHeadDim / 4 && c.layout.v.token == kHeadDim / 4;

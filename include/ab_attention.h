@@ -30,7 +30,7 @@
 extern "C" {
 #endif
 
-#define AB_ABI_VERSION 6
+#define AB_ABI_VERSION 7
 
 enum ab_status {
     AB_OK = 0,
@@ -157,7 +157,10 @@ int ab_dense_prefill(const void *q, const void *k, const void *v, int64_t batch_
  * Q, K, V and out are [batch, heads, tokens, 128] with strides of their own
  * (batch, head, token; in elements, multiples of 8, of 4 for out; the 128 dims
  * are contiguous), so slices of tokens and the transposed views of [batch,
- * tokens, heads, 128] are read in place. lse is contiguous. With a workspace, a call whose rows would
+ * tokens, heads, 128] are read in place. lse is contiguous. A sparse call may
+ * list tail_samples blocks (a multiple of 8) once for all rows, as if they
+ * followed every row's own list: a prompt's blocks at weight 0 behind each
+ * video row's sampled ones. ab_prefill_workspace_bytes counts them in samples. With a workspace, a call whose rows would
  * leave much of the GPU idle (a prompt's few query blocks over a whole video,
  * a short clip) splits each row's keys over several workgroups and adds up
  * their float32 partial results; the result is the same up to float32
@@ -173,6 +176,9 @@ typedef struct ab_prefill_args {
     float *lse;
     int64_t batch, heads, q_tokens, kv_tokens, samples;
     int64_t q_stride[3], k_stride[3], v_stride[3], out_stride[3];
+    const int32_t *tail_ids;
+    const float *tail_log_weights;
+    int64_t tail_samples;
     void *workspace;
     size_t workspace_bytes;
 } ab_prefill_args;

@@ -22,7 +22,7 @@ def _run(q, k, v, ids, w, order, split):
     out = torch.full_like(q, float("nan"))
     lse = torch.full(q.shape[:3], float("nan"), device="cuda")
     args = _lib.PrefillArgs(*(_lib.ptr(t) for t in (q, k, v, order, ids, w, out, lse)), 1, bh, nq, nk, samples,
-                            *(_lib.in_place(t)[1] for t in (q, k, v, out)),
+                            *(_lib.in_place(t)[1] for t in (q, k, v, out)), None, None, 0,
                             _lib.ptr(ws), size if split else 0)
     _lib.check(lib.ab_prefill(args, _lib.stream(q.device)))
     torch.cuda.synchronize()
@@ -91,11 +91,39 @@ def test_split_rule():
 def test_split_rejects_a_bad_workspace():
     lib, a, rows = _lib.load(), 4096, 4 * [(1 << 20, 1 << 14, 128)]  # a stand-in address: rejected before any launch
     for ws, size, message in ((a, 64, b"smaller than"), (a + 8, 1 << 30, b"16-byte aligned")):
-        args = _lib.PrefillArgs(a, a, a, None, None, None, a, None, 1, 24, 256, 119056, _lib.PREFILL_DENSE, *rows, ws, size)
+        args = _lib.PrefillArgs(a, a, a, None, None, None, a, None, 1, 24, 256, 119056, _lib.PREFILL_DENSE, *rows,
+                                None, None, 0, ws, size)
         assert lib.ab_prefill(args, None) == 1 and message in lib.ab_last_error()
-    args = _lib.PrefillArgs(a, a, a, None, None, None, a, None, 1, 1, 128, 128, 0, *rows, None, 0)
+    args = _lib.PrefillArgs(a, a, a, None, None, None, a, None, 1, 1, 128, 128, 0, *rows, None, None, 0,
+                            None, 0)
     assert lib.ab_prefill(args, None) == 1 and b"multiple of 8" in lib.ab_last_error()
     for bad in ((1 << 20, 1 << 14, 132), (-8, 1 << 14, 128), (1 << 20, 1 << 14, 1 << 21)):
         args = _lib.PrefillArgs(a, a, a, None, None, None, a, None, 1, 1, 128, 128, _lib.PREFILL_DENSE, rows[0], bad,
-                                *rows[:2], None, 0)
+                                *rows[:2], None, None, 0, None, 0)
         assert lib.ab_prefill(args, None) == 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,samples,tail", [(2, 8, 8), (2, 504, 24), (2, 512, 8), (3, 1016, 520), (40, 128, 16)])
+def test_shared_list(heads, samples, tail):
+    """Blocks listed once for all rows equal the same blocks appended to every
+    row's list, bit for bit: lists that end inside, at and beyond a batch of 512
+    listed blocks, on split calls and (40 heads) an unsplit one."""
+    from ab_attention.paged import _prefill_kv
+
+    print(f"shared list heads={heads} samples={samples} tail={tail}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(samples + tail)
+    n, fb = 1000, 4096
+    q = torch.randn(1, heads, n, 128, device="cuda", generator=g).to(torch.bfloat16)
+    k, v = (torch.randn(1, heads, 4 * fb, 128, device="cuda", generator=g).to(torch.bfloat16) for _ in range(2))
+    rows = heads * -(-n // 128)
+    ids = torch.randint(fb, (rows, samples), device="cuda", generator=g, dtype=torch.int32)
+    w = torch.rand(rows, samples, device="cuda", generator=g) * 3
+    tail_ids = torch.randint(fb, (1, tail), device="cuda", generator=g, dtype=torch.int32)
+    tail_w = torch.zeros(1, tail, device="cuda")
+    tail_w[:, -3:] = float("-inf")
+    got = _prefill_kv(q, k, v, ids, w, return_lse=True, tail=(tail_ids, tail_w, tail))
+    want = _prefill_kv(q, k, v, torch.cat([ids, tail_ids.expand(rows, tail)], 1),
+                       torch.cat([w, tail_w.expand(rows, tail)], 1), return_lse=True)
+    torch.cuda.synchronize()
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
