@@ -19,6 +19,7 @@
 //   - the normaliser D is accumulated tile by tile from the fp16-rounded values
 //     (online max/rescale), matching the reference up to fp32 rounding order.
 #include <cfloat>
+#include <type_traits>
 
 #include "common.hpp"
 #include "layout.hpp"
@@ -31,8 +32,16 @@ namespace {
 // Stage 1+2: clustering of one 128-query block and pooling of the same 128
 // key tokens. One workgroup of 128 threads per (query block, head): thread i
 // owns query i (its row kept in 128 VGPRs as f32); thread d owns dim d in the
-// column sums, which read the block from LDS one 64-row half at a time
-// (17 KB of LDS and 162 VGPRs: three waves per SIMD).
+// mean, which reads the block from LDS one 64-row half at a time (17 KB of LDS
+// and 150 VGPRs: three waves per SIMD).
+//
+// Bound by VALU issue on a full chip (nine distance passes of 256 sub/fma per
+// query are over half of it) and by the chain of passes, reductions and
+// barriers of one workgroup (22 us) on a small call. Centre rows come through
+// scalar loads instead of being published in LDS, the argmax stays in
+// registers (DPP), and the member sums split the slots between the waves:
+// 80 heads x 75,600 tokens 1,061 -> 887 us, 12 x 32,760 97 -> 81 us, 2 x 2,048
+// 26.8 -> 21.7 us.
 
 constexpr int kClusterThreads = 128;
 constexpr int kHalfRows = 64;
@@ -79,16 +88,63 @@ __device__ __forceinline__ float lane_distance(const f32x4 (&x)[32], const float
     return pending[5];
 }
 
+// The same to a query row that every lane shares, read through the scalar
+// cache straight into scalar registers (packed: the row's 64 bf16 pairs in
+// global memory, wave-uniform address): no LDS reads, and no store and barrier
+// to publish the row first.
+__device__ __forceinline__ float lane_distance_to_row(const f32x4 (&x)[32], const uint32_t* __restrict__ packed) {
+    float pending[6];
+#pragma unroll
+    for (int k = 0; k < 32; ++k) {
+        const int dim = leaf_chain(k);
+        float acc = 0.0f;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const uint32_t pair = packed[(dim >> 1) + 16 * r];
+            const float delta = x[k][r] - ((dim & 1) ? bf16_hi(pair) : bf16_lo(pair));
+            acc = __builtin_fmaf(delta, delta, acc);
+        }
+        float v = acc;
+        int level = 0;
+#pragma unroll
+        for (int b = 0; b < 5; ++b)
+            if (((k >> b) & 1) && level == b) {
+                v = pending[b] + v;
+                level = b + 1;
+            }
+        pending[level] = v;
+    }
+    return pending[5];
+}
+
+// Maximum over the wave's lanes, in every lane: DPP row shifts and row
+// broadcasts leave it in lane 63 (a few cycles each; a shuffle goes through the
+// LDS unit).
+__device__ __forceinline__ float wave_max(float v) {
+    // Lanes without a source take their own value.
+    auto step = [&](auto ctrl, auto rows) {
+        const int own = __float_as_int(v);
+        v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(own, own, decltype(ctrl)::value, decltype(rows)::value,
+                                                               0xf, false)));
+    };
+    using std::integral_constant;
+    step(integral_constant<int, 0x111>{}, integral_constant<int, 0xf>{});  // row_shr:1
+    step(integral_constant<int, 0x112>{}, integral_constant<int, 0xf>{});  // row_shr:2
+    step(integral_constant<int, 0x114>{}, integral_constant<int, 0xf>{});  // row_shr:4
+    step(integral_constant<int, 0x118>{}, integral_constant<int, 0xf>{});  // row_shr:8
+    step(integral_constant<int, 0x142>{}, integral_constant<int, 0xa>{});  // row_bcast:15 into rows 1 and 3
+    step(integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{});  // row_bcast:31 into rows 2 and 3
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+}
+
 // Block-wide argmax over the 128 threads' values: largest value, lowest
 // thread index on ties (cub::ArgMax semantics, csrc/ibcs.cu:94-102), valid
-// in every thread. Per wave: the maximum by an xor butterfly (exact, so every
-// lane holds the same value), then the lowest lane holding it from a ballot;
-// the two waves meet in LDS. One barrier: the caller places another barrier
-// between this call and the next (the LDS slots are reused).
+// in every thread. Per wave: the maximum (exact, whatever its order), then the
+// lowest lane holding it from a ballot; the two waves meet in LDS. One
+// barrier: the caller places another barrier between this call and the next
+// (the LDS slots are reused).
 __device__ __forceinline__ int block_argmax(float value, float* s_val, int* s_idx) {
-    float m = value;
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
+    const float m = wave_max(value);
     const uint64_t hit = __ballot(value == m);  // empty only if every value is NaN
     const int wave = threadIdx.x >> 6;
     if ((threadIdx.x & 63) == 0) {
@@ -116,7 +172,7 @@ __global__ __launch_bounds__(kClusterThreads) __attribute__((amdgpu_waves_per_eu
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
     QkLayout layout, uint16_t* __restrict__ centroids, float* __restrict__ pops, uint16_t* __restrict__ pooled,
     int64_t n, int64_t qb, float qk_scale_log2, const int32_t* __restrict__ order) {
-    __shared__ uint32_t half_block[kHalfRows * kRowWords];
+    __shared__ uint32_t half_block[(kHalfRows + 1) * kRowWords];  // 64 rows and a row of zeros
     __shared__ __align__(16) float center_row[kHeadDim];
     __shared__ float s_val[2];
     __shared__ int s_idx[2];
@@ -188,8 +244,9 @@ __global__ __launch_bounds__(kClusterThreads) __attribute__((amdgpu_waves_per_eu
             }
     }
 
-    // Thread tid owns dim tid in the column passes: its word of a packed row
-    // and the selector of its half.
+    if (tid < kRowWords) half_block[kHalfRows * kRowWords + tid] = 0u;  // read after the barriers below
+    // Thread tid owns dim tid in the mean: its word of a packed row and the
+    // selector of its half.
     const int my_word = tid >> 1;
     const uint32_t my_sel = bf16_select(tid);
     // The rows of half h (queries 64h .. 64h+63) into LDS, written by wave h
@@ -227,29 +284,25 @@ __global__ __launch_bounds__(kClusterThreads) __attribute__((amdgpu_waves_per_eu
     }
     __syncthreads();
 
-    // Farthest-first centres with nearest-centre assignment (:158-197).
+    // Farthest-first centres with nearest-centre assignment (:158-197). A
+    // centre is a query of the block: its row is read from global memory (in
+    // the caches since the block's own loads) by scalar loads.
     const bool live = tid < valid;
     float min_d = live ? lane_distance(x, center_row) : -INFINITY;
     int center = block_argmax(min_d, s_val, s_idx);
     min_d = INFINITY;
     int assign = 0;
     for (int slot = 0; slot < kCentroids; ++slot) {
-        // The centre's own thread publishes its row (every thread has read
-        // the previous centre row and the argmax slots before the argmax's
-        // barrier).
-        if (tid == center) {
-#pragma unroll
-            for (int kk = 0; kk < 32; ++kk) *reinterpret_cast<f32x4*>(center_row + 4 * kk) = x[kk];
+        const uint32_t coff = __builtin_amdgcn_readfirstlane(stored(__builtin_amdgcn_readfirstlane(center), q_row));
+        const float dist = lane_distance_to_row(x, reinterpret_cast<const uint32_t*>(qhead + coff));
+        if (live && dist < min_d) {
+            min_d = dist;
+            assign = slot;
         }
-        __syncthreads();
-        if (live) {
-            const float dist = lane_distance(x, center_row);
-            if (dist < min_d) {
-                min_d = dist;
-                assign = slot;
-            }
+        if (slot + 1 < kCentroids) {
+            __syncthreads();  // every thread has read the last argmax's slots
+            center = block_argmax(live ? min_d : -INFINITY, s_val, s_idx);
         }
-        if (slot + 1 < kCentroids) center = block_argmax(live ? min_d : -INFINITY, s_val, s_idx);
     }
 
     // Members of each slot: per wave, the ballot of the queries assigned to
@@ -267,45 +320,59 @@ __global__ __launch_bounds__(kClusterThreads) __attribute__((amdgpu_waves_per_eu
 
     // Centroid = bf16(member sum / count), then the LSE pre-scale
     // bf16(centroid * 128^-0.5 * log2 e) (csrc/ibcs.cu:213-237, :293-295).
-    // Members are added in query order (half 0, then half 1), read from the
-    // staged half that holds them, 8 loads in flight.
-    // The member masks are made wave-uniform (SGPRs), so the walk over the
-    // members (find first set bit, clear it) is scalar work.
-    float msum[kCentroids];
+    // Wave w sums slots 4w .. 4w + 3, lane l dims 2l and 2l + 1 (one word of a
+    // row), each slot's members in query order (half 0, then half 1) from the
+    // staged half that holds them. Two slots are walked together, four members
+    // of each at a time, so eight reads are in flight; a slot that has run out
+    // reads the zero row, whose +0.0 leaves a sum (never -0.0) as it is. The
+    // member masks are wave-uniform, so finding the next member is scalar work.
+    constexpr int kWaveSlots = kCentroids * 64 / kClusterThreads;
+    const int lane = tid & 63;
+    float sum_lo[kWaveSlots], sum_hi[kWaveSlots];
 #pragma unroll
-    for (int s = 0; s < kCentroids; ++s) msum[s] = 0.0f;
+    for (int i = 0; i < kWaveSlots; ++i) sum_lo[i] = sum_hi[i] = 0.0f;
     for (int h = 0; h < 2; ++h) {
         stage_half(h);
-        for (int s = 0; s < kCentroids; ++s) {
-            const uint64_t lds_m = slot_mask[h][s];
-            const uint32_t m_lo = __builtin_amdgcn_readfirstlane(uint32_t(lds_m));
-            const uint32_t m_hi = __builtin_amdgcn_readfirstlane(uint32_t(lds_m >> 32));
-            uint64_t m = (uint64_t(m_hi) << 32) | m_lo;
-            float sum = msum[s];
-            for (int left = __popcll(m); left >= 8; left -= 8) {
-                int idx[8];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    idx[e] = static_cast<int>(__builtin_ctzll(m));
-                    m &= m - 1u;
-                }
-                float v[8];
+        for (int i = 0; i < kWaveSlots; i += 2) {
+            uint64_t m[2];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) v[e] = block_elem_sel(half_block, idx[e], my_word, my_sel);
-#pragma unroll
-                for (int e = 0; e < 8; ++e) sum += v[e];
+            for (int j = 0; j < 2; ++j) {
+                const uint64_t mask = slot_mask[h][kWaveSlots * wave + i + j];
+                m[j] = (uint64_t(__builtin_amdgcn_readfirstlane(uint32_t(mask >> 32))) << 32) |
+                       uint32_t(__builtin_amdgcn_readfirstlane(uint32_t(mask)));
             }
-            for (; m != 0u; m &= m - 1u) sum += block_elem_sel(half_block, __builtin_ctzll(m), my_word, my_sel);
-            msum[s] = sum;
+            while ((m[0] | m[1]) != 0u) {
+                uint32_t w[2][4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) {
+                        const int idx = m[j] != 0u ? static_cast<int>(__builtin_ctzll(m[j])) : kHalfRows;
+                        m[j] &= m[j] - 1u;
+                        w[j][e] = half_block[idx * kRowWords + lane];
+                    }
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) {
+                        sum_lo[i + j] += bf16_lo(w[j][e]);
+                        sum_hi[i + j] += bf16_hi(w[j][e]);
+                    }
+            }
         }
         __syncthreads();
     }
-    uint16_t* dst = centroids + row * kCentroids * kHeadDim + tid;
+    uint32_t* dst = reinterpret_cast<uint32_t*>(centroids) + row * (kCentroids * kHeadDim / 2) + lane;
 #pragma unroll
-    for (int s = 0; s < kCentroids; ++s) {
+    for (int i = 0; i < kWaveSlots; ++i) {
+        const int s = kWaveSlots * wave + i;
         const int cnt = __popcll(slot_mask[0][s]) + __popcll(slot_mask[1][s]);
-        const uint32_t c = cnt > 0 ? f32_to_bf16(__fdiv_rn(msum[s], static_cast<float>(cnt))) : 0u;
-        dst[s * kHeadDim] = static_cast<uint16_t>(f32_to_bf16(__uint_as_float(c << 16) * qk_scale_log2));
+        auto scaled = [&](float sum) {
+            const uint32_t c = cnt > 0 ? f32_to_bf16(__fdiv_rn(sum, static_cast<float>(cnt))) : 0u;
+            return f32_to_bf16(__uint_as_float(c << 16) * qk_scale_log2);
+        };
+        dst[s * (kHeadDim / 2)] = scaled(sum_lo[i]) | (scaled(sum_hi[i]) << 16);
     }
 }
 
