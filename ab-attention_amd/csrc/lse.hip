@@ -16,7 +16,8 @@
 // This file is compiled with -fno-honor-nans: every input is finite, and
 // without NaNs fmaxf/fminf of MFMA results are single instructions.
 //
-// One workgroup = 4 waves = 8 query blocks (64 centroid rows) of one head.
+// One workgroup = 4 waves = 8 query blocks (64 centroid rows) of one head (4 or
+// 2 of them on calls with few query blocks: lse_qblocks).
 // The head's KV4 blocks are taken in chunks of 16; in round i wave w handles
 // chunk 4i + w, so every pooled key is read by exactly one wave. A chunk (32
 // pooled rows, 8 KiB) reaches the wave's LDS buffer by global_load_lds_dwordx4;
@@ -43,17 +44,17 @@ int64_t lse_stride(int64_t fb);  // ibcs.hip
 namespace {
 
 constexpr int kLseThreads = 256;
-constexpr int kLseQBlocks = 8;   // query blocks per workgroup
-constexpr int kLseRows = kLseQBlocks * kCentroids;
 constexpr int kLseChunk = 16;    // KV4 blocks per wave step
 constexpr int kLseChunkBytes = kLseChunk * kReps * kHeadDim * 2;  // 8 KiB
 constexpr int kLseInBytes = 4 * kLseChunkBytes;                   // one buffer per wave
-constexpr int kLseOutBytes = kLseRows * 4 * kLseChunk * 2;        // 8 KiB per round
-constexpr int kLseLdsBytes = kLseInBytes + 2 * kLseOutBytes;      // 48 KiB
+// Bytes of a round's results, and of a workgroup's LDS, for `qblocks` query blocks.
+constexpr int lse_out_bytes(int qblocks) { return qblocks * kCentroids * 4 * kLseChunk * 2; }
+constexpr int lse_lds_bytes(int qblocks) { return kLseInBytes + 2 * lse_out_bytes(qblocks); }
 // Largest 2^(l - ref) allowed before the normaliser's reference is moved.
 constexpr float kLseSlack = 8.0f;
 
-static_assert(3 * kLseLdsBytes <= 160 * 1024, "three workgroups per CU must fit in LDS");
+static_assert(3 * lse_lds_bytes(8) <= 160 * 1024, "three workgroups per CU must fit in LDS");
+static_assert(4 * lse_lds_bytes(4) <= 160 * 1024, "four smaller ones too");
 
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -89,11 +90,17 @@ __device__ __forceinline__ void combine_pair(float& m, float& d, float om, float
     m = nm;
 }
 
-__global__ __launch_bounds__(kLseThreads, 3) void lse_kernel(
+// kQBlocks: query blocks per workgroup (8, or fewer for calls with few of them:
+// lse_qblocks). A row's arithmetic and the order of its sums are the same.
+template <int kQBlocks>
+__global__ __launch_bounds__(kLseThreads, kQBlocks == 8 ? 3 : 4) void lse_kernel(
     const uint16_t* __restrict__ centroids, const uint16_t* __restrict__ pooled,
     _Float16* __restrict__ lse, float* __restrict__ lse_max, float* __restrict__ lse_den,
     int64_t qb, int fb, int64_t ld, int groups_per_head, int total_groups) {
     extern __shared__ __align__(16) unsigned char smem[];
+    constexpr int kTiles = kQBlocks / 2;  // 16-row centroid tiles
+    constexpr int kRows = kQBlocks * kCentroids;
+    constexpr int kOutBytes = lse_out_bytes(kQBlocks);
 
     // XCD-aware order: hardware deals workgroups round-robin over 8 XCDs, so
     // consecutive logical groups (same head) are given to one XCD.
@@ -110,10 +117,10 @@ __global__ __launch_bounds__(kLseThreads, 3) void lse_kernel(
 
     // B operand: centroid row 16*rt + col (query block 2rt + col/8 of the
     // group, centroid col%8), dims 32s + 8*quad .. +8.
-    bf16x8 cen[4][4];
+    bf16x8 cen[kTiles][4];
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt) {
-        const int64_t qbk = qgroup * kLseQBlocks + 2 * rt + (col >> 3);
+    for (int rt = 0; rt < kTiles; ++rt) {
+        const int64_t qbk = qgroup * kQBlocks + 2 * rt + (col >> 3);
         const int64_t crow = (bh * qb + min(qbk, qb - 1)) * kCentroids + (col & 7);
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
@@ -172,14 +179,14 @@ __global__ __launch_bounds__(kLseThreads, 3) void lse_kernel(
     for (int r = 0; r < 2; ++r)
 #pragma unroll
         for (int s = 0; s < 4; ++s) a_off[r][s] = (2 * col + r) * 256 + 16 * ((4 * s + quad) ^ col);
-    // Round output staging: fp16 [64 rows][64 blocks]; the 16-byte unit U of
+    // Round output staging: fp16 [kRows][64 blocks]; the 16-byte unit U of
     // row R sits at position U ^ ((R >> 1) & 7).
     unsigned char* out_stage = smem + kLseInBytes;
 
     // Per 16-row tile: exact maximum, normaliser and its reference.
-    float top[4], den[4], ref[4];
+    float top[kTiles], den[kTiles], ref[kTiles];
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt) {
+    for (int rt = 0; rt < kTiles; ++rt) {
         top[rt] = -FLT_MAX;
         den[rt] = 0.0f;
         ref[rt] = -FLT_MAX;
@@ -195,14 +202,14 @@ __global__ __launch_bounds__(kLseThreads, 3) void lse_kernel(
     };
     auto compute = [&](int c, int i, const bf16x8 (&a)[2][4], auto tail_tag) {
         constexpr bool kTail = decltype(tail_tag)::value;
-        unsigned char* ostage = out_stage + (i & 1) * kLseOutBytes;
+        unsigned char* ostage = out_stage + (i & 1) * kOutBytes;
         const int jq = c * kLseChunk + 4 * quad;  // first block of this lane
         // fp16 pair-LSEs of each row tile, blocks (0, 1) and (2, 3) (non-tail
         // path). Kept as whole f16x2 values: bit casts of single elements of
         // an ext_vector read element 0 with this compiler.
-        f16x2 tile01[4], tile23[4];
+        f16x2 tile01[kTiles], tile23[kTiles];
 #pragma unroll
-        for (int rt = 0; rt < 4; ++rt) {
+        for (int rt = 0; rt < kTiles; ++rt) {
             f32x4 acc[2];
 #pragma unroll
             for (int r = 0; r < 2; ++r) {
@@ -250,10 +257,10 @@ __global__ __launch_bounds__(kLseThreads, 3) void lse_kernel(
             // One wave-uniform branch per chunk moves the references of every
             // row tile that needs it (rare); tiles and lanes that do not grow
             // take nr == ref, and den * 2^0 leaves den unchanged.
-            float tmax[4];
+            float tmax[kTiles];
             bool grow_any = false;
 #pragma unroll
-            for (int rt = 0; rt < 4; ++rt) {
+            for (int rt = 0; rt < kTiles; ++rt) {
                 const f16x2 m2 = __builtin_elementwise_max(tile01[rt], tile23[rt]);
                 tmax[rt] = static_cast<float>(m2[0] > m2[1] ? m2[0] : m2[1]);
                 top[rt] = fmaxf(top[rt], tmax[rt]);
@@ -261,7 +268,7 @@ __global__ __launch_bounds__(kLseThreads, 3) void lse_kernel(
             }
             if (__any(grow_any)) {
 #pragma unroll
-                for (int rt = 0; rt < 4; ++rt) {
+                for (int rt = 0; rt < kTiles; ++rt) {
                     const float nr = tmax[rt] > ref[rt] + kLseSlack ? tmax[rt] : ref[rt];
                     den[rt] *= fast_exp2(ref[rt] - nr);
                     ref[rt] = nr;
@@ -270,7 +277,7 @@ __global__ __launch_bounds__(kLseThreads, 3) void lse_kernel(
             // f - ref straight from the fp16 halves with v_fma_mix_f32
             // (f16 -> f32 is exact, so this is the rounded f - ref).
 #pragma unroll
-            for (int rt = 0; rt < 4; ++rt) {
+            for (int rt = 0; rt < kTiles; ++rt) {
                 const uint32_t lo = __builtin_bit_cast(uint32_t, tile01[rt]);
                 const uint32_t hi = __builtin_bit_cast(uint32_t, tile23[rt]);
                 den[rt] += fast_exp2(f16_minus<false>(lo, ref[rt]));
@@ -282,16 +289,18 @@ __global__ __launch_bounds__(kLseThreads, 3) void lse_kernel(
     };
 
     // Whole rows of round j: thread t writes 16 bytes of rows t/8 and t/8 + 32
-    // (blocks past fb land in the row padding, never read). The rows of a
-    // wave belong to query blocks w and w + 4 of the group, so the number of
-    // stores a wave issues (n_st) is uniform.
-    const int n_st = int(qgroup * kLseQBlocks + wave < qb) + int(qgroup * kLseQBlocks + wave + 4 < qb);
+    // (as far as there are rows; blocks past fb land in the row padding, never
+    // read). The rows of a wave belong to query blocks w and w + 4 of the
+    // group, so the number of stores a wave issues (n_st) is uniform.
+    const int n_st = int(wave < kQBlocks && qgroup * kQBlocks + wave < qb) +
+                     int(wave + 4 < kQBlocks && qgroup * kQBlocks + wave + 4 < qb);
     auto store_round = [&](int j) {
-        const unsigned char* ostage = out_stage + (j & 1) * kLseOutBytes;
+        const unsigned char* ostage = out_stage + (j & 1) * kOutBytes;
 #pragma unroll
-        for (int h2 = 0; h2 < 2; ++h2) {
+        for (int h2 = 0; h2 < (kRows + 31) / 32; ++h2) {
             const int R = (tid >> 3) + 32 * h2, U = tid & 7;
-            const int64_t qbk = qgroup * kLseQBlocks + R / kCentroids;
+            if (kRows < 32 && wave >= kQBlocks) break;
+            const int64_t qbk = qgroup * kQBlocks + R / kCentroids;
             const u32x4 val = *reinterpret_cast<const u32x4*>(ostage + R * 128 + 16 * (U ^ ((R >> 1) & 7)));
             // Streaming store: the pair-LSEs are read back only by the next
             // kernel, and allocating them in the caches would evict the
@@ -347,31 +356,31 @@ __global__ __launch_bounds__(kLseThreads, 3) void lse_kernel(
     // Rebase each lane's normaliser on its exact maximum, then merge the four
     // lanes (quads) of each centroid row and the four waves.
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt) den[rt] *= fast_exp2(ref[rt] - top[rt]);
+    for (int rt = 0; rt < kTiles; ++rt) den[rt] *= fast_exp2(ref[rt] - top[rt]);
 #pragma unroll
     for (int off = 16; off < 64; off <<= 1)
 #pragma unroll
-        for (int rt = 0; rt < 4; ++rt) {
+        for (int rt = 0; rt < kTiles; ++rt) {
             const float om = __shfl_xor(top[rt], off);
             const float od = __shfl_xor(den[rt], off);
             combine_pair(top[rt], den[rt], om, od);
         }
     __syncthreads();  // the staging area is reused below
     float* s_max = reinterpret_cast<float*>(smem + kLseInBytes);
-    float* s_den = s_max + 4 * kLseRows;
+    float* s_den = s_max + 4 * kRows;
     if (quad == 0) {
 #pragma unroll
-        for (int rt = 0; rt < 4; ++rt) {
-            s_max[wave * kLseRows + 16 * rt + col] = top[rt];
-            s_den[wave * kLseRows + 16 * rt + col] = den[rt];
+        for (int rt = 0; rt < kTiles; ++rt) {
+            s_max[wave * kRows + 16 * rt + col] = top[rt];
+            s_den[wave * kRows + 16 * rt + col] = den[rt];
         }
     }
     __syncthreads();
-    if (tid < kLseRows) {
+    if (tid < kRows) {
         float m = s_max[tid], d = s_den[tid];
 #pragma unroll
-        for (int w = 1; w < 4; ++w) combine_pair(m, d, s_max[w * kLseRows + tid], s_den[w * kLseRows + tid]);
-        const int64_t qbk = qgroup * kLseQBlocks + tid / kCentroids;
+        for (int w = 1; w < 4; ++w) combine_pair(m, d, s_max[w * kRows + tid], s_den[w * kRows + tid]);
+        const int64_t qbk = qgroup * kQBlocks + tid / kCentroids;
         if (qbk < qb) {
             const int64_t slot = (bh * qb + qbk) * kCentroids + tid % kCentroids;
             lse_max[slot] = m;
@@ -380,22 +389,45 @@ __global__ __launch_bounds__(kLseThreads, 3) void lse_kernel(
     }
 }
 
-}  // namespace
-
-int launch_lse(const void* centroids, const void* pooled, int64_t bh, int64_t n, void* lse,
-               float* lse_max, float* lse_den, hipStream_t stream) {
-    const int64_t qb = (n + kQueryBlock - 1) / kQueryBlock;
-    const int64_t fb = n / kKvBlock;
-    const int groups_per_head = static_cast<int>((qb + kLseQBlocks - 1) / kLseQBlocks);
+template <int kQBlocks>
+int launch(const void* centroids, const void* pooled, int64_t bh, int64_t qb, int64_t fb, void* lse, float* lse_max,
+           float* lse_den, hipStream_t stream) {
+    const int groups_per_head = static_cast<int>((qb + kQBlocks - 1) / kQBlocks);
     const int64_t total = groups_per_head * bh;
     if (total > (int64_t(1) << 30)) return set_error(1, "ibcs: too many query blocks (%lld)", (long long)total);
     const int per_xcd = static_cast<int>((total + 7) / 8);
-    if (int rc = ensure_lds_limit(reinterpret_cast<const void*>(lse_kernel), kLseLdsBytes)) return rc;
-    hipLaunchKernelGGL(lse_kernel, dim3(static_cast<unsigned>(per_xcd * 8)), dim3(kLseThreads), kLseLdsBytes,
+    const auto kernel = lse_kernel<kQBlocks>;
+    if (int rc = ensure_lds_limit(reinterpret_cast<const void*>(kernel), lse_lds_bytes(kQBlocks))) return rc;
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(per_xcd * 8)), dim3(kLseThreads), lse_lds_bytes(kQBlocks),
                        stream, static_cast<const uint16_t*>(centroids), static_cast<const uint16_t*>(pooled),
                        static_cast<_Float16*>(lse), lse_max, lse_den, qb, static_cast<int>(fb), lse_stride(fb),
                        groups_per_head, static_cast<int>(total));
     return check_launch("lse_kernel");
+}
+
+// Query blocks per workgroup: 8, which reads the pooled keys least often, for
+// calls that fill the chip. Below that a smaller workgroup both spreads over
+// more CUs and has less to do per chunk of keys: a round of 64 blocks takes
+// 1.1 us in a lone workgroup of 8, 0.7 in one of 4 and 0.5 in one of 2.
+// Measured at 8 / 4 / 2 (workgroups of 8): 2 heads x 2,048 tokens (4) 13.2 /
+// 8.9 / 7.0 us, 4 x 8,192 (32) 39 / 25 / 19, 5 x 16,384 (80) 71 / 48 / 48, 24 x
+// 8,192 (192) 39 / 32 / 36, 40 x 8,192 (320) 54 / 47 / 60, 5 x 75,600 (370) 434 /
+// 415 / 616, 12 x 32,760 (384) 194 / 190 / 263, 16 x 32,760 (512) 223 / 241 / 348.
+int lse_qblocks(int64_t bh, int64_t qb) {
+    const int64_t groups = (qb + 7) / 8 * bh;
+    return groups <= 80 ? 2 : groups <= 400 ? 4 : 8;
+}
+
+}  // namespace
+
+int launch_lse(const void* centroids, const void* pooled, int64_t bh, int64_t n, void* lse,
+               float* lse_max, float* lse_den, hipStream_t stream) {
+    const int64_t qb = (n + kQueryBlock - 1) / kQueryBlock, fb = n / kKvBlock;
+    switch (lse_qblocks(bh, qb)) {
+        case 2: return launch<2>(centroids, pooled, bh, qb, fb, lse, lse_max, lse_den, stream);
+        case 4: return launch<4>(centroids, pooled, bh, qb, fb, lse, lse_max, lse_den, stream);
+        default: return launch<8>(centroids, pooled, bh, qb, fb, lse, lse_max, lse_den, stream);
+    }
 }
 
 }  // namespace ab
