@@ -22,13 +22,15 @@
 // the last residual, the draws) use all the workgroup's threads, which keeps
 // enough waves per SIMD to hide LDS and fp64 latency.
 //
-// Two storage schemes, same bits:
+// Three storage schemes, same bits:
 //   - sip_lds_kernel (rows whose masses and fp64 prefixes fit in LDS):
 //     persistent workgroups walk rows r, r + grid, ...; while a row is
 //     processed out of LDS, the next row's masses are loaded into registers,
 //     and they are written to LDS as soon as the row's last draw has read it
 //     (before the row's results are stored). Certainty is marked by the sign
 //     bit of the LDS copy, as the reference negates its copy.
+//   - sip_kept_kernel (rows whose masses fit in LDS but not beside all the
+//     prefixes): the same with some of the prefixes kept (coarse_draws);
 //   - sip_global_kernel (larger rows): one row per workgroup, the row is
 //     re-read from L2 by each pass, LDS holds the prefixes and a certainty
 //     bitmask.
@@ -745,6 +747,70 @@ __global__ __launch_bounds__(kSipWorkers) void sip_lds_kernel(
     }
 }
 
+// Persistent kernel for rows whose masses fit in LDS but not beside the full
+// prefix array (c3's 29,700 blocks): masses and coarse_keep(pop) kept prefixes
+// per chunk (coarse_draws), as the fused kernel samples such rows. The next
+// row's first kAhead masses per thread are loaded into registers while a row is
+// sampled; the rest are loaded when it is staged. Bound by the row's ordered
+// phases (one wave per SIMD) and its load: 5,574 rows x 29,700 masses, 2,272
+// samples 802 us with every pass over the row from L2 (sip_global_kernel), 485 us
+// out of LDS.
+template <int kAhead>
+__global__ __launch_bounds__(kSipWorkers) void sip_kept_kernel(
+    const float* __restrict__ masses, const float* __restrict__ offsets, int32_t* __restrict__ ids,
+    float* __restrict__ logw, int population, int samples, int64_t rows) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ SipShared sh;
+    const int t = threadIdx.x;
+    const int pop = population;
+    float* values = reinterpret_cast<float*>(smem);
+    double* kept = reinterpret_cast<double*>(smem + sip_fused_coarse_offset(pop));
+    float next[kAhead];
+    auto prefetch = [&](int64_t r) {
+        const float* in = masses + r * int64_t(pop);
+#pragma unroll
+        for (int k = 0; k < kAhead; ++k) {
+            const float* base = in + k * kSipWorkers;
+            next[k] = t + k * kSipWorkers < pop ? base[t] : 0.0f;
+        }
+    };
+    auto put = [&](int i, float m) {
+        if (i < pop) values[i] = m > 0.0f ? m : 0.0f;  // NaN, negatives -> +0
+    };
+    auto stage = [&](int64_t r) {
+        // The rest of the row first, so that its loads overlap the stores of
+        // what was loaded ahead.
+        const float* in = masses + r * int64_t(pop) + kAhead * kSipWorkers;
+        const int left = pop - kAhead * kSipWorkers;
+        for (int j0 = t; j0 < left; j0 += kUnroll * kSipWorkers) {
+            float m[kUnroll];
+#pragma unroll
+            for (int e = 0; e < kUnroll; ++e) m[e] = in[min(j0 + e * kSipWorkers, left - 1)];
+#pragma unroll
+            for (int e = 0; e < kUnroll; ++e) put(kAhead * kSipWorkers + j0 + e * kSipWorkers, m[e]);
+        }
+#pragma unroll
+        for (int k = 0; k < kAhead; ++k) put(t + k * kSipWorkers, next[k]);
+    };
+    int64_t row = blockIdx.x;
+    if (row < rows) {
+        prefetch(row);
+        stage(row);
+    }
+    for (; row < rows; row += gridDim.x) {
+        const int64_t following = row + gridDim.x;
+        if (following < rows) prefetch(following);
+        lds_barrier();  // this row is staged
+        LdsRow rv{values};
+        double sum = 0.0, mx = 0.0;
+        if (t < kSipThreads) strided_partials<true>(rv, pop, sum, mx);
+        sip_row<kSipWorkers, true>(rv, sum, mx, kept, sh, offsets[row], ids + row * int64_t(samples),
+                                   logw + row * int64_t(samples), pop, samples, [&] {
+                                       if (following < rows) stage(following);
+                                   });
+    }
+}
+
 // Fused masses + SIP for rows whose masses fit in LDS: each persistent
 // workgroup computes its row's masses from the fp16 pair-LSEs [8, ld]
 // straight into LDS (RowMasses: the arithmetic of masses_kernel, so the same
@@ -834,18 +900,19 @@ __global__ __launch_bounds__(kSipWorkers) void sip_global_kernel(
                                 logw + row * int64_t(samples), pop, samples, [] {});
 }
 
-template <int kPer>
-int launch_lds(const float* scores, const float* offsets, int64_t rows, int pop, int samples, int32_t* ids,
-               float* logw, size_t bytes, hipStream_t stream) {
-    const void* fn = reinterpret_cast<const void*>(sip_lds_kernel<kPer>);
+using SipKernel = void (*)(const float*, const float*, int32_t*, float*, int, int, int64_t);
+
+int launch_persistent(SipKernel kernel, const float* scores, const float* offsets, int64_t rows, int pop, int samples,
+                      int32_t* ids, float* logw, size_t bytes, hipStream_t stream) {
+    const void* fn = reinterpret_cast<const void*>(kernel);
     if (int rc = ensure_lds_limit(fn, static_cast<int>(bytes))) return rc;
     int per_cu = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, kSipWorkers, bytes) != hipSuccess || per_cu < 1)
         per_cu = 1;
     const int64_t grid = std::min<int64_t>(rows, int64_t(device_cu_count()) * per_cu);
-    hipLaunchKernelGGL(sip_lds_kernel<kPer>, dim3(static_cast<unsigned>(grid)), dim3(kSipWorkers), bytes, stream,
-                       scores, offsets, ids, logw, pop, samples, rows);
-    return check_launch("sip_lds_kernel");
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(kSipWorkers), bytes, stream, scores, offsets,
+                       ids, logw, pop, samples, rows);
+    return check_launch("sip_kernel");
 }
 
 }  // namespace
@@ -931,12 +998,16 @@ int launch_sip(const float* scores, const float* offsets, int64_t rows, int64_t 
     const int pop = static_cast<int>(population), s = static_cast<int>(samples);
     const size_t lds_bytes = sip_lds_bytes(population, true);
     const int per_thread = (pop + kSipWorkers - 1) / kSipWorkers;
+    auto persistent = [&](SipKernel kernel, size_t bytes) {
+        return launch_persistent(kernel, scores, offsets, rows, pop, s, ids, logw, bytes, stream);
+    };
     if (lds_bytes + kSipStaticLds <= kLdsLimit) {
-        if (per_thread <= 4) return launch_lds<4>(scores, offsets, rows, pop, s, ids, logw, lds_bytes, stream);
-        if (per_thread <= 8) return launch_lds<8>(scores, offsets, rows, pop, s, ids, logw, lds_bytes, stream);
-        if (per_thread <= 16) return launch_lds<16>(scores, offsets, rows, pop, s, ids, logw, lds_bytes, stream);
-        if (per_thread <= 24) return launch_lds<24>(scores, offsets, rows, pop, s, ids, logw, lds_bytes, stream);
+        if (per_thread <= 4) return persistent(sip_lds_kernel<4>, lds_bytes);
+        if (per_thread <= 8) return persistent(sip_lds_kernel<8>, lds_bytes);
+        if (per_thread <= 16) return persistent(sip_lds_kernel<16>, lds_bytes);
+        if (per_thread <= 24) return persistent(sip_lds_kernel<24>, lds_bytes);
     }
+    if (sip_fused_fits(population)) return persistent(sip_kept_kernel<16>, sip_fused_lds_bytes(population, true));
     const size_t bytes = sip_lds_bytes(population, false);
     if (int rc = ensure_lds_limit(reinterpret_cast<const void*>(sip_global_kernel), static_cast<int>(bytes)))
         return rc;

@@ -80,3 +80,16 @@ def test_degenerate_rows(oracle_mod):
     offsets = np.array([0.0, 0.999999, 0.5, 0.25, 0.75], np.float32)
     _assert_bit_exact(scores, offsets, 7, oracle_mod)
     _assert_bit_exact(scores, offsets, 599, oracle_mod)
+
+
+@pytest.mark.parametrize("pop,rows,peak", [(24577, 8, 0.0), (26001, 8, 40.0), (29700, 600, 30.0), (32768, 8, 0.0),
+                                           (39001, 8, 30.0), (41000, 8, 30.0)])
+def test_kept_prefix_rows(pop, rows, peak, oracle_mod):
+    """Rows whose masses fit in LDS without all prefixes, from the smallest to
+    the largest, several per workgroup (600 rows), and one past them (the
+    global-memory path)."""
+    rng = np.random.default_rng(pop)
+    scores = _local_masses(rng, rows, pop, peak)
+    scores[1, pop // 2:] = 0.0  # draws fall in the first half, the last residuals at the floor
+    offsets = rng.random(rows, dtype=np.float32)
+    _assert_bit_exact(scores, offsets, 2272, oracle_mod)
