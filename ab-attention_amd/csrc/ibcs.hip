@@ -41,9 +41,13 @@ namespace {
 // scalar loads instead of being published in LDS, the argmax stays in
 // registers (DPP), and the member sums split the slots between the waves:
 // 80 heads x 75,600 tokens 1,061 -> 887 us, 12 x 32,760 97 -> 81 us, 2 x 2,048
-// 26.8 -> 21.7 us.
+// 26.8 -> 21.7 us (18.3 with two lanes per query, below).
 
-constexpr int kClusterThreads = 128;
+// Calls with few query blocks run the same with kLanes = 2 lanes per query
+// (256 threads): lanes l and l + 32 of a wave hold one query, 16 of its 32
+// chains each (the even and the odd ones: the two halves of the distance's
+// tree).
+
 constexpr int kHalfRows = 64;
 constexpr int kRowWords = kHeadDim / 2 + 1;  // padded bf16 row: 65 dwords
 
@@ -62,59 +66,65 @@ __host__ __device__ constexpr int leaf_chain(int k) {
 // registers that way, and the centre row in LDS (one 16-byte read or write
 // per chain).
 __device__ __forceinline__ int center_pos(int d) { return 4 * leaf_chain(d & 31) + (d >> 5); }
-__device__ __forceinline__ float row_dim(const f32x4 (&x)[32], int d) { return x[leaf_chain(d & 31)][d >> 5]; }
 
-__device__ __forceinline__ float lane_distance(const f32x4 (&x)[32], const float* __restrict__ center) {
-    float pending[6];
+// Sum of the tree over this lane's 32 / kLanes leaves, leaf k being the chain
+// over the differences delta(k, r), r = 0..3. With two lanes the halves meet in
+// the last addition.
+template <int kLanes, class Delta>
+__device__ __forceinline__ float chain_tree(Delta delta) {
+    constexpr int kLeaves = 32 / kLanes, kLevels = kLanes == 1 ? 5 : 4;
+    float pending[kLevels + 1];
 #pragma unroll
-    for (int k = 0; k < 32; ++k) {
-        const f32x4 c = *reinterpret_cast<const f32x4*>(center + 4 * k);
+    for (int k = 0; k < kLeaves; ++k) {
         float acc = 0.0f;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const float delta = x[k][r] - c[r];
-            acc = __builtin_fmaf(delta, delta, acc);
+            const float d = delta(k, r);
+            acc = __builtin_fmaf(d, d, acc);
         }
         float v = acc;
         int level = 0;
 #pragma unroll
-        for (int b = 0; b < 5; ++b)
+        for (int b = 0; b < kLevels; ++b)
             if (((k >> b) & 1) && level == b) {
                 v = pending[b] + v;
                 level = b + 1;
             }
         pending[level] = v;
     }
-    return pending[5];
+    if constexpr (kLanes == 1) return pending[kLevels];
+    const uint32_t half = __float_as_uint(pending[kLevels]);
+    const auto both = __builtin_amdgcn_permlane32_swap(half, half, false, false);
+    return __uint_as_float(both[0]) + __uint_as_float(both[1]);
+}
+
+// Distance of the lane's query to a row in LDS, leaf order (center: this
+// lane's half of it).
+template <int kLanes>
+__device__ __forceinline__ float lane_distance(const f32x4 (&x)[32 / kLanes], const float* __restrict__ center) {
+    f32x4 c;
+    return chain_tree<kLanes>([&](int k, int r) {
+        if (r == 0) c = *reinterpret_cast<const f32x4*>(center + 4 * k);
+        return x[k][r] - c[r];
+    });
 }
 
 // The same to a query row that every lane shares, read through the scalar
 // cache straight into scalar registers (packed: the row's 64 bf16 pairs in
 // global memory, wave-uniform address): no LDS reads, and no store and barrier
-// to publish the row first.
-__device__ __forceinline__ float lane_distance_to_row(const f32x4 (&x)[32], const uint32_t* __restrict__ packed) {
-    float pending[6];
-#pragma unroll
-    for (int k = 0; k < 32; ++k) {
+// to publish the row first. With two lanes per query each picks its half of a
+// pair with one v_perm_b32 (sel).
+template <int kLanes>
+__device__ __forceinline__ float lane_distance_to_row(const f32x4 (&x)[32 / kLanes],
+                                                     const uint32_t* __restrict__ packed, uint32_t sel) {
+    return chain_tree<kLanes>([&](int k, int r) {
         const int dim = leaf_chain(k);
-        float acc = 0.0f;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const uint32_t pair = packed[(dim >> 1) + 16 * r];
-            const float delta = x[k][r] - ((dim & 1) ? bf16_hi(pair) : bf16_lo(pair));
-            acc = __builtin_fmaf(delta, delta, acc);
-        }
-        float v = acc;
-        int level = 0;
-#pragma unroll
-        for (int b = 0; b < 5; ++b)
-            if (((k >> b) & 1) && level == b) {
-                v = pending[b] + v;
-                level = b + 1;
-            }
-        pending[level] = v;
-    }
-    return pending[5];
+        const uint32_t pair = packed[(dim >> 1) + 16 * r];
+        const float c = kLanes == 2 ? __uint_as_float(__builtin_amdgcn_perm(pair, pair, sel))
+                        : (dim & 1) ? bf16_hi(pair)
+                                    : bf16_lo(pair);
+        return x[k][r] - c;
+    });
 }
 
 // Maximum over the wave's lanes, in every lane: DPP row shifts and row
@@ -137,24 +147,39 @@ __device__ __forceinline__ float wave_max(float v) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }
 
-// Block-wide argmax over the 128 threads' values: largest value, lowest
-// thread index on ties (cub::ArgMax semantics, csrc/ibcs.cu:94-102), valid
-// in every thread. Per wave: the maximum (exact, whatever its order), then the
-// lowest lane holding it from a ballot; the two waves meet in LDS. One
-// barrier: the caller places another barrier between this call and the next
-// (the LDS slots are reused).
+// Block-wide argmax over the queries' values: largest value, lowest query on
+// ties (cub::ArgMax semantics, csrc/ibcs.cu:94-102), valid in every thread.
+// Per wave: the maximum (exact, whatever its order), then the lowest lane
+// holding it from a ballot; the waves meet in LDS. One barrier: the caller
+// places another barrier between this call and the next (the LDS slots are
+// reused).
+template <int kLanes>
 __device__ __forceinline__ int block_argmax(float value, float* s_val, int* s_idx) {
     const float m = wave_max(value);
     const uint64_t hit = __ballot(value == m);  // empty only if every value is NaN
     const int wave = threadIdx.x >> 6;
     if ((threadIdx.x & 63) == 0) {
         s_val[wave] = m;
-        s_idx[wave] = 64 * wave + (hit != 0u ? static_cast<int>(__builtin_ctzll(hit)) : 0);
+        s_idx[wave] = 64 / kLanes * wave + (hit != 0u ? static_cast<int>(__builtin_ctzll(hit)) : 0);
     }
     __syncthreads();
-    const float v0 = s_val[0], v1 = s_val[1];
-    const int i0 = s_idx[0], i1 = s_idx[1];
-    return v1 > v0 ? i1 : i0;  // equal values: wave 0 holds the lower index
+    // Queries 0-63 and 64-127; of equal values the first holds the lower index.
+    float v[2];
+    int idx[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        v[h] = s_val[kLanes * h];
+        idx[h] = s_idx[kLanes * h];
+        if constexpr (kLanes == 2) {
+            const float other = s_val[2 * h + 1];
+            // Only NaNs in a wave: any number of the other one wins.
+            if (other > v[h] || (v[h] != v[h] && other == other)) {
+                v[h] = other;
+                idx[h] = s_idx[2 * h + 1];
+            }
+        }
+    }
+    return v[1] > v[0] ? idx[1] : idx[0];
 }
 
 // Byte selector of v_perm_b32 that moves the bf16 of dim `dim` of a packed
@@ -168,17 +193,23 @@ __device__ __forceinline__ float block_elem_sel(const uint32_t* block, int row, 
     return __uint_as_float(__builtin_amdgcn_perm(w, w, sel));
 }
 
-__global__ __launch_bounds__(kClusterThreads) __attribute__((amdgpu_waves_per_eu(3, 3))) void cluster_pool_kernel(
+template <int kLanes>
+__global__ __launch_bounds__(kQueryBlock* kLanes) __attribute__((amdgpu_waves_per_eu(3, 3))) void cluster_pool_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
     QkLayout layout, uint16_t* __restrict__ centroids, float* __restrict__ pops, uint16_t* __restrict__ pooled,
     int64_t n, int64_t qb, float qk_scale_log2, const int32_t* __restrict__ order) {
     __shared__ uint32_t half_block[(kHalfRows + 1) * kRowWords];  // 64 rows and a row of zeros
     __shared__ __align__(16) float center_row[kHeadDim];
-    __shared__ float s_val[2];
-    __shared__ int s_idx[2];
-    __shared__ uint64_t slot_mask[kClusterThreads / 64][kCentroids];
+    constexpr int kWaves = 2 * kLanes, kWaveQueries = 64 / kLanes, kLeaves = 32 / kLanes;
+    __shared__ float s_val[kWaves];
+    __shared__ int s_idx[kWaves];
+    __shared__ uint32_t slot_mask[4][kCentroids];  // members among queries 32i .. 32i + 31
 
-    const int tid = threadIdx.x, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // The lane's query and its half of the dims (kLanes = 2: even or odd).
+    const int query = kWaveQueries * wave + (lane & (kWaveQueries - 1));
+    const int part = kLanes == 2 ? lane >> 5 : 0;
     const int64_t blk = blockIdx.x, bh = blockIdx.y;
     const int64_t base = blk * kQueryBlock;
     const int valid = static_cast<int>(min<int64_t>(kQueryBlock, n - base));
@@ -202,24 +233,26 @@ __global__ __launch_bounds__(kClusterThreads) __attribute__((amdgpu_waves_per_eu
         const int tok = b32 + min(t, valid - 1);
         return uint32_t(__umul24(order ? min(max(order[tok], 0), nm1) : tok, row));
     };
-    u32x4 ka[8], kb[8];
+    constexpr int kPairs = 8 / kLanes;  // key pairs per thread
+    u32x4 ka[kPairs], kb[kPairs];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int p = r0 + 8 * i;
+    for (int i = 0; i < kPairs; ++i) {
+        const int p = r0 + 8 * kLanes * i;
         ka[i] = khead[stored(2 * p, k_row) + c16];
         kb[i] = khead[stored(2 * p + 1, k_row) + c16];
     }
-    f32x4 x[32];
+    const uint32_t part_sel = bf16_select(part);
+    f32x4 x[kLeaves];
     {
-        const uint32_t qoff = stored(tid, q_row);
+        const uint32_t qoff = stored(query, q_row);
         u32x4 qv[16];
 #pragma unroll
         for (int j = 0; j < 16; ++j) qv[j] = qhead[qoff + j];
         // Pool the keys: bf16(0.5 * (k_2r + k_2r+1)) (:244-266).
         u32x4* kdst = reinterpret_cast<u32x4*>(pooled + (bh * (n / 2) + base / 2) * kHeadDim);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int p = r0 + 8 * i;
+        for (int i = 0; i < kPairs; ++i) {
+            const int p = r0 + 8 * kLanes * i;
             if (p < pairs) {
                 u32x4 o;
 #pragma unroll
@@ -232,102 +265,119 @@ __global__ __launch_bounds__(kClusterThreads) __attribute__((amdgpu_waves_per_eu
             }
         }
         // Queries past the sequence end are zero rows.
-        const bool zero_row = tid >= valid;
+        const bool zero_row = query >= valid;
 #pragma unroll
         for (int j = 0; j < 16; ++j)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const uint32_t w = zero_row ? 0u : qv[j][e];
                 const int d = 8 * j + 2 * e;
-                x[leaf_chain(d & 31)][d >> 5] = bf16_lo(w);
-                x[leaf_chain((d + 1) & 31)][(d + 1) >> 5] = bf16_hi(w);
+                if constexpr (kLanes == 1) {
+                    x[leaf_chain(d & 31)][d >> 5] = bf16_lo(w);
+                    x[leaf_chain((d + 1) & 31)][(d + 1) >> 5] = bf16_hi(w);
+                } else {
+                    x[leaf_chain(d & 31)][d >> 5] = __uint_as_float(__builtin_amdgcn_perm(w, w, part_sel));
+                }
             }
     }
 
     if (tid < kRowWords) half_block[kHalfRows * kRowWords + tid] = 0u;  // read after the barriers below
-    // Thread tid owns dim tid in the mean: its word of a packed row and the
-    // selector of its half.
-    const int my_word = tid >> 1;
-    const uint32_t my_sel = bf16_select(tid);
-    // The rows of half h (queries 64h .. 64h+63) into LDS, written by wave h
-    // from its registers: v_perm_b32 takes the high halves of two floats,
-    // which gives back the loaded bf16 pair bit for bit.
+    // The rows of half h (queries 64h .. 64h+63) into LDS, written by the waves
+    // that hold them: v_perm_b32 takes the high halves of two floats, which
+    // gives back the loaded bf16 pair bit for bit. With two lanes per query
+    // they swap halves of words w and w + 32, and write one of them each.
     auto stage_half = [&](int h) {
-        if (wave == h) {
-            uint32_t* dst = half_block + (tid & 63) * kRowWords;
+        if (wave / kLanes == h) {
+            uint32_t* dst = half_block + (query & 63) * kRowWords + 32 * part;
+            auto value = [&](int d) { return __float_as_uint(x[leaf_chain(d & 31)][d >> 5]); };
+            if constexpr (kLanes == 1) {
 #pragma unroll
-            for (int w = 0; w < kHeadDim / 2; ++w)
-                dst[w] = __builtin_amdgcn_perm(__float_as_uint(row_dim(x, 2 * w + 1)),
-                                               __float_as_uint(row_dim(x, 2 * w)), 0x07060302u);
+                for (int w = 0; w < kHeadDim / 2; ++w)
+                    dst[w] = __builtin_amdgcn_perm(value(2 * w + 1), value(2 * w), 0x07060302u);
+            } else {
+#pragma unroll
+                for (int w = 0; w < kHeadDim / 4; ++w) {
+                    const auto s = __builtin_amdgcn_permlane32_swap(value(2 * w), value(2 * w + 64), false, false);
+                    dst[w] = __builtin_amdgcn_perm(s[1], s[0], 0x07060302u);
+                }
+            }
         }
         __syncthreads();
     };
 
-    // Per-dim mean over valid queries in row order (csrc/ibcs.cu:130-140).
+    // Per-dim mean over valid queries in row order (csrc/ibcs.cu:130-140):
+    // thread d < 128 owns dim d, its word of a packed row and its half of that.
     {
+        const int my_word = tid >> 1;
+        const uint32_t my_sel = bf16_select(tid);
         float sum = 0.0f;
         for (int h = 0; h < 2; ++h) {
             stage_half(h);
-            const int end = min(valid - kHalfRows * h, kHalfRows);
+            const int end = tid < kHeadDim ? min(valid - kHalfRows * h, kHalfRows) : 0;
             int i = 0;
-            for (; i + 8 <= end; i += 8) {  // 8 reads in flight, adds in row order
-                float v[8];
+            for (; i + 16 <= end; i += 16) {  // 16 reads in flight, adds in row order
+                float v[16];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) v[e] = block_elem_sel(half_block, i + e, my_word, my_sel);
+                for (int e = 0; e < 16; ++e) v[e] = block_elem_sel(half_block, i + e, my_word, my_sel);
 #pragma unroll
-                for (int e = 0; e < 8; ++e) sum += v[e];
+                for (int e = 0; e < 16; ++e) sum += v[e];
             }
             for (; i < end; ++i) sum += block_elem_sel(half_block, i, my_word, my_sel);
             __syncthreads();
         }
-        center_row[center_pos(tid)] = __fdiv_rn(sum, static_cast<float>(valid));
+        if (tid < kHeadDim) center_row[center_pos(tid)] = __fdiv_rn(sum, static_cast<float>(valid));
     }
     __syncthreads();
 
     // Farthest-first centres with nearest-centre assignment (:158-197). A
     // centre is a query of the block: its row is read from global memory (in
     // the caches since the block's own loads) by scalar loads.
-    const bool live = tid < valid;
-    float min_d = live ? lane_distance(x, center_row) : -INFINITY;
-    int center = block_argmax(min_d, s_val, s_idx);
+    const bool live = query < valid;
+    const float mean_d = lane_distance<kLanes>(x, center_row + 4 * kLeaves * part);
+    float min_d = live ? mean_d : -INFINITY;
+    int center = block_argmax<kLanes>(min_d, s_val, s_idx);
     min_d = INFINITY;
     int assign = 0;
     for (int slot = 0; slot < kCentroids; ++slot) {
         const uint32_t coff = __builtin_amdgcn_readfirstlane(stored(__builtin_amdgcn_readfirstlane(center), q_row));
-        const float dist = lane_distance_to_row(x, reinterpret_cast<const uint32_t*>(qhead + coff));
+        const float dist =
+            lane_distance_to_row<kLanes>(x, reinterpret_cast<const uint32_t*>(qhead + coff), part_sel);
         if (live && dist < min_d) {
             min_d = dist;
             assign = slot;
         }
         if (slot + 1 < kCentroids) {
             __syncthreads();  // every thread has read the last argmax's slots
-            center = block_argmax(live ? min_d : -INFINITY, s_val, s_idx);
+            center = block_argmax<kLanes>(live ? min_d : -INFINITY, s_val, s_idx);
         }
     }
 
     // Members of each slot: per wave, the ballot of the queries assigned to
-    // it. Queries 64w + bit, walked wave by wave and bit by bit, come in
-    // query order (the reference's member order).
+    // it. Queries 32i + bit, walked word by word and bit by bit, come in query
+    // order (the reference's member order).
 #pragma unroll
     for (int s = 0; s < kCentroids; ++s) {
         const uint64_t m = __ballot(live && assign == s);
-        if ((tid & 63) == 0) slot_mask[wave][s] = m;
+        if (lane == 0) {
+            slot_mask[wave * (2 / kLanes)][s] = static_cast<uint32_t>(m);
+            if constexpr (kLanes == 1) slot_mask[2 * wave + 1][s] = static_cast<uint32_t>(m >> 32);
+        }
     }
     __syncthreads();
-    if (tid < kCentroids)
-        pops[row * kCentroids + tid] =
-            static_cast<float>(__popcll(slot_mask[0][tid]) + __popcll(slot_mask[1][tid]));
+    auto members = [&](int s) {
+        return __popc(slot_mask[0][s]) + __popc(slot_mask[1][s]) + __popc(slot_mask[2][s]) + __popc(slot_mask[3][s]);
+    };
+    if (tid < kCentroids) pops[row * kCentroids + tid] = static_cast<float>(members(tid));
 
     // Centroid = bf16(member sum / count), then the LSE pre-scale
     // bf16(centroid * 128^-0.5 * log2 e) (csrc/ibcs.cu:213-237, :293-295).
-    // Wave w sums slots 4w .. 4w + 3, lane l dims 2l and 2l + 1 (one word of a
-    // row), each slot's members in query order (half 0, then half 1) from the
+    // Each wave sums its share of the slots, lane l dims 2l and 2l + 1 (one word
+    // of a row), each slot's members in query order (half 0, then half 1) from the
     // staged half that holds them. Two slots are walked together, four members
     // of each at a time, so eight reads are in flight; a slot that has run out
     // reads the zero row, whose +0.0 leaves a sum (never -0.0) as it is. The
     // member masks are wave-uniform, so finding the next member is scalar work.
-    constexpr int kWaveSlots = kCentroids * 64 / kClusterThreads;
-    const int lane = tid & 63;
+    constexpr int kWaveSlots = kCentroids / kWaves;
     float sum_lo[kWaveSlots], sum_hi[kWaveSlots];
 #pragma unroll
     for (int i = 0; i < kWaveSlots; ++i) sum_lo[i] = sum_hi[i] = 0.0f;
@@ -338,9 +388,9 @@ __global__ __launch_bounds__(kClusterThreads) __attribute__((amdgpu_waves_per_eu
             uint64_t m[2];
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
-                const uint64_t mask = slot_mask[h][kWaveSlots * wave + i + j];
-                m[j] = (uint64_t(__builtin_amdgcn_readfirstlane(uint32_t(mask >> 32))) << 32) |
-                       uint32_t(__builtin_amdgcn_readfirstlane(uint32_t(mask)));
+                const int s = kWaveSlots * wave + i + j;
+                m[j] = (uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(slot_mask[2 * h + 1][s]))) << 32) |
+                       uint32_t(__builtin_amdgcn_readfirstlane(slot_mask[2 * h][s]));
             }
             while ((m[0] | m[1]) != 0u) {
                 uint32_t w[2][4];
@@ -367,7 +417,7 @@ __global__ __launch_bounds__(kClusterThreads) __attribute__((amdgpu_waves_per_eu
 #pragma unroll
     for (int i = 0; i < kWaveSlots; ++i) {
         const int s = kWaveSlots * wave + i;
-        const int cnt = __popcll(slot_mask[0][s]) + __popcll(slot_mask[1][s]);
+        const int cnt = members(s);
         auto scaled = [&](float sum) {
             const uint32_t c = cnt > 0 ? f32_to_bf16(__fdiv_rn(sum, static_cast<float>(cnt))) : 0u;
             return f32_to_bf16(__uint_as_float(c << 16) * qk_scale_log2);
@@ -419,6 +469,12 @@ __global__ __launch_bounds__(kMassThreads) void masses_kernel(
 
 int64_t lse_stride(int64_t fb) { return (fb + 63) / 64 * 64; }
 
+// Lanes per query: two while the blocks leave most SIMDs to one workgroup, where
+// the length of its chain of passes is the time (32 blocks 22.6 -> 18.3 us, 256
+// 23.6 -> 20.1); from about 768 blocks (33.0 us both) the extra v_perm_b32s and
+// waves cost more than they save (1,536 blocks 45 against 54 us).
+int cluster_lanes(int64_t blocks) { return blocks <= 640 ? 2 : 1; }
+
 int launch_cluster_pool(const void* q, const void* k, const QkLayout& layout, int64_t bh, int64_t n, void* centroids,
                         float* pops, void* pooled, float qk_scale_log2, const int32_t* order, hipStream_t stream) {
     // The kernel addresses a head with 32-bit offsets in 16-byte units, made of 24-bit factors.
@@ -428,8 +484,9 @@ int launch_cluster_pool(const void* q, const void* k, const QkLayout& layout, in
             return set_error(1, "ibcs: token stride of %lld is too large", 4 * (long long)t->token);
     const int64_t qb = (n + kQueryBlock - 1) / kQueryBlock;
     dim3 grid(static_cast<unsigned>(qb), static_cast<unsigned>(bh));
-    hipLaunchKernelGGL(cluster_pool_kernel, grid, dim3(kClusterThreads), 0, stream,
-                       static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(k), layout,
+    const int lanes = cluster_lanes(qb * bh);
+    const auto kernel = lanes == 2 ? cluster_pool_kernel<2> : cluster_pool_kernel<1>;
+    hipLaunchKernelGGL(kernel, grid, dim3(kQueryBlock * lanes), 0, stream, static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(k), layout,
                        static_cast<uint16_t*>(centroids), pops, static_cast<uint16_t*>(pooled), n, qb,
                        qk_scale_log2, order);
     return check_launch("cluster_pool_kernel");
