@@ -138,10 +138,11 @@ def ibcs_sip(q: torch.Tensor, k: torch.Tensor, offsets: torch.Tensor, ids: torch
 
 
 def plan_heads(q: torch.Tensor, k: torch.Tensor, start: int, stop: int, offsets: torch.Tensor, ids: torch.Tensor,
-               logs: torch.Tensor, order: torch.Tensor | None = None) -> None:
+               logs: torch.Tensor, samples: int, order: torch.Tensor | None = None) -> None:
     """``ibcs_sip`` of heads start .. stop-1 of the flattened [batch * heads] of
-    q, k (offsets, ids and logs are those heads' rows), reading them where they
-    lie: slices of tokens and transposed projections need no copy (ab_plan)."""
+    q, k (offsets, ids and logs are those heads' rows, contiguous, ``samples``
+    entries each), reading them where they lie: slices of tokens and transposed
+    projections need no copy (ab_plan)."""
     _require(q.is_cuda and k.is_cuda, "q and k must be CUDA tensors")
     _require(q.device == k.device, "q and k must use the same CUDA device")
     _require(q.dtype == torch.bfloat16 and k.dtype == torch.bfloat16, "IBCS requires bfloat16 q/k")
@@ -158,6 +159,6 @@ def plan_heads(q: torch.Tensor, k: torch.Tensor, start: int, stop: int, offsets:
         ws_bytes = lib.ab_ibcs_sip_workspace_bytes(stop - start, tokens)
         workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
         args = _lib.PlanArgs(address(q), address(k), address(order), address(offsets), address(ids), address(logs),
-                             batch, heads, start, stop - start, tokens, ids.shape[1], q_stride, k_stride,
+                             batch, heads, start, stop - start, tokens, samples, q_stride, k_stride,
                              address(workspace), ws_bytes)
         _lib.check(lib.ab_plan(args, _lib.stream(q.device)))

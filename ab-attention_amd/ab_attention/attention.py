@@ -106,21 +106,21 @@ def _build_plan(q, k, sample_pages, seed, order=None):
     offsets = torch.rand(rows, device=q.device, generator=generator)
 
     heads_per_chunk = _heads_per_chunk(batch_heads, q_blocks, tokens)
-    sampled = torch.empty((rows, samples), dtype=torch.int32, device=q.device)
-    log_weights = torch.empty((rows, samples), dtype=torch.float32, device=q.device)
+    plan = SamplePlan(torch.empty((rows, sample_pages, 32), dtype=torch.int32, device=q.device),
+                      torch.empty((rows, sample_pages, 32), dtype=torch.float32, device=q.device))
 
+    # IBCS scores and SIP sampling of each chunk's heads (the reference's _C.ibcs
+    # then _C.sip) in one native call that keeps the scores on chip.
     q, k = _lib.in_place(q)[0], _lib.in_place(k)[0]
+    if 0 < batch_heads <= heads_per_chunk:
+        ops.plan_heads(q, k, 0, batch_heads, offsets, plan.descriptor, plan.log_weights, samples, order)
+        return plan
     for start in range(0, batch_heads, heads_per_chunk):
         stop = min(batch_heads, start + heads_per_chunk)
-        first, last = start * q_blocks, stop * q_blocks
-        # IBCS scores and SIP sampling of the chunk's heads (the reference's
-        # _C.ibcs then _C.sip) in one native call that keeps the scores on chip.
-        ops.plan_heads(q, k, start, stop, offsets[first:last], sampled[first:last], log_weights[first:last], order)
-
-    return SamplePlan(
-        sampled.reshape(rows, sample_pages, 32),
-        log_weights.reshape(rows, sample_pages, 32),
-    )
+        chunk = slice(start * q_blocks, stop * q_blocks)
+        ops.plan_heads(q, k, start, stop, offsets[chunk], plan.descriptor[chunk], plan.log_weights[chunk], samples,
+                       order)
+    return plan
 
 
 @torch.no_grad()
@@ -132,9 +132,9 @@ def apply_plan(q, k, v, plan, *, return_lse=False):
     also returned as float32 [batch, heads, tokens], for merging attention
     partitions. (Reference: attention.py:85-96.)
     """
-    from .paged import paged_attention
+    from .paged import _paged_attention
 
-    return paged_attention(q, k, v, *plan, return_lse=return_lse)
+    return _paged_attention(q, k, v, *plan, return_lse)
 
 
 @torch.no_grad()
@@ -142,4 +142,6 @@ def ab_attention(q, k, v, *, sample_pages=64, seed=42):
     """``build_plan`` then ``apply_plan`` in one call: sparse attention over
     a freshly sampled plan, returned in q's shape and dtype
     (reference: attention.py:99-102)."""
-    return apply_plan(q, k, v, build_plan(q, k, sample_pages=sample_pages, seed=seed))
+    from .paged import _paged_attention
+
+    return _paged_attention(q, k, v, *_build_plan(q, k, sample_pages, seed), False)

@@ -57,14 +57,15 @@ def _run(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, ids, weights, sample
 
 
 def _prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor,
-             order: torch.Tensor | None, return_lse: bool, *, tail=(None, None, 0), out=None):
+             order: torch.Tensor | None, return_lse: bool, *, samples: int | None = None, tail=(None, None, 0), out=None):
     """The weighted prefill, with a query token order when one is given;
-    ids/weights [rows, S]. Shapes are checked by the callers."""
+    ids/weights [rows, S], or any shape of ``samples`` entries per row. Shapes
+    are checked by the callers."""
     if ids.dtype != torch.int32 or not ids.is_contiguous():
         ids = ids.to(torch.int32).contiguous()
     if weights.dtype != torch.float32 or not weights.is_contiguous():
         weights = weights.to(torch.float32).contiguous()
-    return _run(q, k, v, ids, weights, ids.shape[-1], order, return_lse, tail, out)
+    return _run(q, k, v, ids, weights, ids.shape[-1] if samples is None else samples, order, return_lse, tail, out)
 
 
 def check_prefill_inputs(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> None:
@@ -92,19 +93,21 @@ def paged_attention(
     return_lse: bool = False,
 ):
     """Weighted sparse attention over the plan's KV4 blocks; returns o (and base-2 lse)."""
+    return _paged_attention(q, k, v, descriptor, log_weights, return_lse)
+
+
+def _paged_attention(q, k, v, descriptor, log_weights, return_lse):
+    """paged_attention for callers that have turned gradients off (each nested
+    torch.no_grad costs a small call a microsecond)."""
     check_prefill_inputs(q, k, v)
-    batch, heads, tokens, dim = q.shape
-    batch_heads = batch * heads
-    rows = batch_heads * math.ceil(tokens / _QUERY_BLOCK)
+    batch, heads, tokens, _ = q.shape
+    rows = batch * heads * math.ceil(tokens / _QUERY_BLOCK)
     if (descriptor.ndim != 3 or descriptor.shape != log_weights.shape
             or descriptor.shape[0] != rows or descriptor.shape[-1] != 32):
         raise ValueError(f"descriptor and log_weights must share [{rows}, pages, 32] shape")
     if descriptor.device != q.device or log_weights.device != q.device:
         raise ValueError("descriptor and log_weights must be on the Q device")
-
-    samples = descriptor.shape[1] * 32
-    return _prefill(q, k, v, descriptor.reshape(rows, samples), log_weights.reshape(rows, samples), None,
-                    return_lse)
+    return _prefill(q, k, v, descriptor, log_weights, None, return_lse, samples=descriptor.shape[1] * 32)
 
 
 def _prefill_kv(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor,

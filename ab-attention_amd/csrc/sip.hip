@@ -900,16 +900,34 @@ __global__ __launch_bounds__(kSipWorkers) void sip_global_kernel(
                                 logw + row * int64_t(samples), pop, samples, [] {});
 }
 
+// Workgroups of a persistent kernel that the device holds at once. The last
+// answer of each thread is kept (the query costs a small call about a
+// microsecond).
+int64_t resident_workgroups(const void* fn, int threads, size_t bytes) {
+    struct Last {
+        const void* fn;
+        int device, per_cu;
+        size_t bytes;
+    };
+    static thread_local Last last{nullptr, -1, 0, 0};
+    int device = 0;
+    (void)hipGetDevice(&device);
+    if (last.fn != fn || last.device != device || last.bytes != bytes) {
+        int per_cu = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, threads, bytes) != hipSuccess || per_cu < 1)
+            per_cu = 1;
+        last = Last{fn, device, per_cu, bytes};
+    }
+    return int64_t(device_cu_count()) * last.per_cu;
+}
+
 using SipKernel = void (*)(const float*, const float*, int32_t*, float*, int, int, int64_t);
 
 int launch_persistent(SipKernel kernel, const float* scores, const float* offsets, int64_t rows, int pop, int samples,
                       int32_t* ids, float* logw, size_t bytes, hipStream_t stream) {
     const void* fn = reinterpret_cast<const void*>(kernel);
     if (int rc = ensure_lds_limit(fn, static_cast<int>(bytes))) return rc;
-    int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, kSipWorkers, bytes) != hipSuccess || per_cu < 1)
-        per_cu = 1;
-    const int64_t grid = std::min<int64_t>(rows, int64_t(device_cu_count()) * per_cu);
+    const int64_t grid = std::min<int64_t>(rows, resident_workgroups(fn, kSipWorkers, bytes));
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(kSipWorkers), bytes, stream, scores, offsets,
                        ids, logw, pop, samples, rows);
     return check_launch("sip_kernel");
@@ -952,10 +970,7 @@ int launch_fused(const _Float16* lse, const float* pops, const float* lse_max, c
     const size_t bytes = sip_fused_lds_bytes(pop, kCoarse);
     const void* fn = reinterpret_cast<const void*>(sip_fused_kernel<kWorkers, kCoarse>);
     if (int rc = ensure_lds_limit(fn, static_cast<int>(bytes))) return rc;
-    int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, kWorkers, bytes) != hipSuccess || per_cu < 1)
-        per_cu = 1;
-    const int64_t grid = std::min<int64_t>(rows, int64_t(device_cu_count()) * per_cu);
+    const int64_t grid = std::min<int64_t>(rows, resident_workgroups(fn, kWorkers, bytes));
     hipLaunchKernelGGL((sip_fused_kernel<kWorkers, kCoarse>), dim3(static_cast<unsigned>(grid)), dim3(kWorkers), bytes,
                        stream, lse, pops, lse_max, lse_den, ld, offsets, ids, logw, pop, samples, rows,
                        force_exact);
