@@ -58,7 +58,9 @@
 // v_mfma_f32_16x16x32_bf16 tiles (see there).
 // Calls with too few rows to fill the chip split each row's tiles over several
 // workgroups (kSplit, prefill_parts), whose float32 partial results
-// combine_kernel adds up.
+// combine_kernel adds up. All parts of a row share its reference, so a split
+// row differs from an unsplit one by the order of its float32 sums only, unless
+// it leaves the fast pass (then P rounds to bf16 against other references).
 #include <algorithm>
 #include <type_traits>
 
@@ -248,11 +250,16 @@ __device__ __forceinline__ bool unit_slot(const RowGrid& g, const Divisor& heads
     us.part = static_cast<int>(head_part - flat * parts);
     return true;
 }
-// Tiles [first, first + count) of part `part` of `parts` (parts <= tiles, so
-// none is empty).
-__device__ __forceinline__ void part_tiles(int tiles, int parts, int part, int& first, int& count) {
-    first = static_cast<int>(int64_t(tiles) * part / parts);
-    count = static_cast<int>(int64_t(tiles) * (part + 1) / parts) - first;
+// Tiles of part `part` of `parts` (parts <= tiles, so none is empty). Every part
+// but the first leads with the row's tile 0: it sets the fast pass's reference,
+// as in the unsplit pass, so that every p = 2^(z - m) has the same bf16 bits
+// however a row is split, and adds nothing itself. `lead` is 1 for these parts;
+// tile 0 of the unit is the row's tile 0 and tile u > 0 the row's u + skip.
+__device__ __forceinline__ void part_tiles(int tiles, int parts, int part, int& lead, int& skip, int& count) {
+    const int first = static_cast<int>(int64_t(tiles) * part / parts);
+    lead = part > 0 ? 1 : 0;
+    skip = first - lead;
+    count = static_cast<int>(int64_t(tiles) * (part + 1) / parts) - skip;
 }
 
 // Partial results of the split kernels, in the caller's workspace: per unit
@@ -284,10 +291,10 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_kernel(
     extern __shared__ __align__(16) unsigned char smem[];
 
     UnitSlot rs;
-    int tile0 = 0, tiles = (lists.samples + (kTail ? lists.tail : 0)) / kTilePages;
+    int lead = 0, skip = 0, tiles = (lists.samples + (kTail ? lists.tail : 0)) / kTilePages;
     if constexpr (kSplit) {
         if (!unit_slot(grid, layout.heads, partials.parts, rs)) return;
-        part_tiles(tiles, partials.parts, rs.part, tile0, tiles);
+        part_tiles(tiles, partials.parts, rs.part, lead, skip, tiles);
     } else {
         if (!row_slot(grid, layout.heads, rs)) return;
     }
@@ -315,9 +322,8 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_kernel(
     }
 
     const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_u8*)smem));
-    const int first = kTail ? 0 : tile0 * kTilePages;
-    const int32_t* row_ids = lists.ids + row * int64_t(lists.samples) + first;
-    const float* row_w = lists.logw + row * int64_t(lists.samples) + first;
+    const int32_t* row_ids = lists.ids + row * int64_t(lists.samples);
+    const float* row_w = lists.logw + row * int64_t(lists.samples);
     const uint16_t* kbase = k + layout.k.at(rs.b, rs.h, 0);
     const uint16_t* vbase = v + layout.v.at(rs.b, rs.h, 0);
     const uint32_t k_token = token_bytes<kPacked>(layout.k), v_token = token_bytes<kPacked>(layout.v);
@@ -330,18 +336,18 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_kernel(
     auto issue_batch = [&](int b) {
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-            const uint32_t src = min(uint32_t(b) * kBatchBytes + i * 1024u + 16u * lane, unit_bytes - 16u);
+            uint32_t at = min(uint32_t(b) * kBatchBytes + i * 1024u + 16u * lane, unit_bytes - 16u);
+            if constexpr (kSplit) at += at >= kTilePages * 4u ? static_cast<uint32_t>(skip) * (kTilePages * 4u) : 0u;
             const uint32_t dst = (b & 1) * kBatchBytes + i * 1024u;
             if constexpr (kTail) {
-                const uint32_t at = src + static_cast<uint32_t>(tile0) * (kTilePages * 4u);
                 const uint32_t row_bytes = static_cast<uint32_t>(lists.samples) * 4u;
                 const bool tail = at >= row_bytes;
                 const uint32_t off = at - (tail ? row_bytes : 0u);
                 dma16(reinterpret_cast<const char*>(tail ? lists.tail_ids : row_ids) + off, lds0 + kIdsOffset + dst);
                 dma16(reinterpret_cast<const char*>(tail ? lists.tail_logw : row_w) + off, lds0 + kWeightsOffset + dst);
             } else {
-                dma16(row_ids, src, lds0 + kIdsOffset + dst);
-                dma16(row_w, src, lds0 + kWeightsOffset + dst);
+                dma16(row_ids, at, lds0 + kIdsOffset + dst);
+                dma16(row_w, at, lds0 + kWeightsOffset + dst);
             }
         }
     };
@@ -604,6 +610,13 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_kernel(
             for (int r = 0; r < 16; ++r) s0[r] -= m_run;
             mx = started ? -INFINITY : INFINITY;
         }
+        if constexpr (kSplit) {
+            if (lead) {  // tile 0 belongs to the first part
+#pragma unroll
+                for (int r = 0; r < 16; ++r) s0[r] = -INFINITY;
+                if constexpr (kSafe) mx = -INFINITY;
+            }
+        }
         // Four steps per iteration: t is a multiple of 4 there, so every ring
         // stage (u & 3) is a compile-time constant and the LDS addresses fold
         // into the instructions' offsets.
@@ -697,10 +710,10 @@ __global__ __launch_bounds__(kPfThreads, 2) void dense_kernel(
     int samples, float scale_log2, PartialsArg<kSplit> partials) {
     extern __shared__ __align__(16) unsigned char smem[];
     UnitSlot rs;
-    int tile0 = 0, tiles = samples / kTilePages;
+    int lead = 0, skip = 0, tiles = samples / kTilePages;
     if constexpr (kSplit) {
         if (!unit_slot(grid, layout.heads, partials.parts, rs)) return;
-        part_tiles(samples / kTilePages, partials.parts, rs.part, tile0, tiles);
+        part_tiles(samples / kTilePages, partials.parts, rs.part, lead, skip, tiles);
     } else {
         if (!row_slot(grid, layout.heads, rs)) return;
     }
@@ -744,11 +757,13 @@ __global__ __launch_bounds__(kPfThreads, 2) void dense_kernel(
         const int P = lane >> 3, sl = (lane >> 1) & 3, h = lane & 1;
         v_src[e] = uint32_t(sl) * v_token + uint32_t(2 * (P ^ e) + h) * 16u;
     }
+    // The row's tile of the unit's tile u; past the end, the last one.
+    auto row_tile = [&](int u) { return kSplit && u == 0 ? 0 : skip + min(u, tiles - 1); };
     // This wave's two pages of tile u, clamped into the head; tiles past the
     // row's end read its last tile (their transfers only keep the per-step
     // count uniform).
     auto load_ids = [&](int u) {
-        const int id = (tile0 + min(u, tiles - 1)) * kTilePages + 2 * wave;
+        const int id = row_tile(u) * kTilePages + 2 * wave;
         const u32x2 c = {uint32_t(min(id, fb - 1)), uint32_t(min(id + 1, fb - 1))};
         return c;
     };
@@ -762,7 +777,7 @@ __global__ __launch_bounds__(kPfThreads, 2) void dense_kernel(
     // The weights of this lane's keys in tile u: pages lg and 4 + lg, 0 inside
     // K/V and -inf past its end.
     auto load_weights = [&](int u, float (&wv)[2]) {
-        const int uc = tile0 + min(u, tiles - 1);
+        const int uc = row_tile(u);
 #pragma unroll
         for (int kt = 0; kt < 2; ++kt) wv[kt] = uc * kTilePages + 4 * kt + lg < fb ? 0.f : -INFINITY;
     };
@@ -992,6 +1007,15 @@ __global__ __launch_bounds__(kPfThreads, 2) void dense_kernel(
                     for (int r = 0; r < 4; ++r) s0[2 * kt + j][r] -= m_run[j];
             }
             mx[0] = all_started ? -INFINITY : INFINITY;
+        }
+        if constexpr (kSplit) {
+            if (lead) {  // tile 0 belongs to the first part
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) s0[c][r] = -INFINITY;
+                if constexpr (kSafe) mx[0] = mx[1] = -INFINITY;
+            }
         }
         int t = 0;
         for (; t + 3 < tiles; t += 4) {
@@ -1227,20 +1251,22 @@ int64_t prefill_launch_slots(int64_t bh, int64_t n) {
 // 512 (two workgroups per CU); the time of a tile step then grows from 0.49 us
 // (a few lone workgroups) over 0.58 (one on every CU) to 0.88 (two), measured
 // on dense calls of 24 to 3,072 rows, and a unit costs its tiles plus a
-// prologue and epilogue worth about 8. Splitting adds combine_kernel (6 us)
+// prologue and epilogue worth about 8, and its leading tile where the row is
+// split (0.1 to 0.6 us of the times below). Splitting adds combine_kernel (6 us)
 // and its 128 KiB of traffic per unit (0.03 us); dense units cannot run faster
 // than their K/V arrive (5.5 TB/s). More units than 512 lose: their rounds do
 // not start together and share less of what they read (640 dense rows of 512
 // tiles: 680 us, in 2 parts 618, but 640 sparse rows of 128: 211 and 238), so
 // calls of more than 256 rows never split. Measured, unsplit and at the parts
-// this picks: dense 24 rows x 3,715 tiles 1,866 -> 269 us, 48 x 3,721 1,855 ->
-// 376, 4 x 1,024 498 -> 35, 256 x 512 275 -> 240; sparse 64 x 64 42 -> 26.
+// this picks: dense 24 rows x 3,715 tiles 1,862 -> 278 us, 48 x 3,721 1,819 ->
+// 384, 4 x 1,024 504 -> 37, 256 x 512 264 -> 240; sparse 64 x 64 38.8 -> 24.4,
+// 16 x 128 69.2 -> 22.5.
 int prefill_parts(int64_t rows, int64_t tiles, int64_t kv_bytes) {
     constexpr double kSetupSteps = 8, kCombine = 6, kUnitTraffic = 0.03, kBytesPerUs = 5.5e6, kGain = 0.95;
     auto cost = [&](int64_t parts) {
         const double units = double(rows * parts), wide = double(kPartUnits);
         const double step = units <= wide ? 0.49 + 0.09 * units / wide : 0.58 + 0.30 * (units / wide - 1.0);
-        const double run = step * (double((tiles + parts - 1) / parts) + kSetupSteps);
+        const double run = step * (double((tiles + parts - 1) / parts) + kSetupSteps + (parts > 1 ? 1.0 : 0.0));
         return std::max(run, double(kv_bytes) / kBytesPerUs) + (parts > 1 ? kCombine + kUnitTraffic * units : 0.0);
     };
     int best = 1;

@@ -163,9 +163,12 @@ int ab_dense_prefill(const void *q, const void *k, const void *v, int64_t batch_
  * video row's sampled ones. ab_prefill_workspace_bytes counts them in samples. With a workspace, a call whose rows would
  * leave much of the GPU idle (a prompt's few query blocks over a whole video,
  * a short clip) splits each row's keys over several workgroups and adds up
- * their float32 partial results; the result is the same up to float32
- * rounding. ab_prefill_workspace_bytes gives the bytes (0: this size is not
- * split and needs none), 16-byte aligned. workspace NULL never splits. */
+ * their float32 partial results. That reorders float32 sums: bf16 outputs
+ * differ in their last bit here and there (about 1e-4 of their norm). Rows
+ * whose first 32 listed keys have no finite logit, or one more than 64 (base 2)
+ * below a later one, also round their probabilities to bf16 against other
+ * references (3e-3). ab_prefill_workspace_bytes gives the bytes (0: this size
+ * is not split and needs none), 16-byte aligned. workspace NULL never splits. */
 #define AB_PREFILL_DENSE (-1)
 typedef struct ab_prefill_args {
     const void *q, *k, *v;
