@@ -278,6 +278,15 @@ struct NoPartials {};
 template <bool kSplit>
 using PartialsArg = std::conditional_t<kSplit, Partials, NoPartials>;
 
+// The first thing each prefill kernel does: values from all three 64-byte lines
+// of its arguments (in host memory) in scalar registers at once, so that the
+// lines arrive together. Left to itself the compiler reads the last one, waits,
+// then reads the others: 35.2 us against 35.7 at 24 heads x 3,496 tokens and 96
+// blocks, 42.3 against 42.9 at 8 x 8,192 and 256.
+__device__ __forceinline__ void touch_arguments(const void* q, const PrefillLayout& layout, const RowGrid& grid) {
+    asm volatile("" ::"s"(q), "s"(layout.q.batch), "s"(grid.bh));
+}
+
 // The sparse prefill: the row's listed KV4 blocks, with their log weights.
 // kSplit: one part of the row's tiles, its result left in `partials`. kTail:
 // the shared blocks behind the row's own (at compile time: with the choice of
@@ -289,6 +298,7 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_kernel(
     float* __restrict__ lse, PrefillLayout layout, int n, RowGrid grid, int fb, float scale_log2,
     const int32_t* __restrict__ order, PartialsArg<kSplit> partials) {
     extern __shared__ __align__(16) unsigned char smem[];
+    touch_arguments(q, layout, grid);
 
     UnitSlot rs;
     int lead = 0, skip = 0, tiles = (lists.samples + (kTail ? lists.tail : 0)) / kTilePages;
@@ -709,6 +719,7 @@ __global__ __launch_bounds__(kPfThreads, 2) void dense_kernel(
     uint16_t* __restrict__ out, float* __restrict__ lse, PrefillLayout layout, int n, RowGrid grid, int fb,
     int samples, float scale_log2, PartialsArg<kSplit> partials) {
     extern __shared__ __align__(16) unsigned char smem[];
+    touch_arguments(q, layout, grid);
     UnitSlot rs;
     int lead = 0, skip = 0, tiles = samples / kTilePages;
     if constexpr (kSplit) {
