@@ -1164,35 +1164,29 @@ __global__ __launch_bounds__(kPfThreads) void combine_kernel(Partials partials, 
 }
 
 // Plan ids of a permuted token layout -> KV4 pages of the stored layout:
-// out[i] = map[clamp(ids[i])]. Bound by the ids' read and write; each thread
-// takes kRemapPer groups of 4 ids, a workgroup apart, with 16-byte loads and
-// stores where ids and out lie on 16 bytes, so that all its gathers (the map
-// stays in the caches) are in flight together: 12.6 million ids 43 -> 26 us.
-constexpr int kRemapPer = 4;
+// out[i] = map[clamp(ids[i])]. Bound by the ids' read and write (12.6 million
+// ids, out of the caches: 34.0 us one id per thread, 20.5 four, at 4.9 TB/s) and,
+// below about a million, by the launch and one load after another (14,336 ids
+// 2.5 -> 1.9 us, 400,000 3.0 -> 2.0). Each thread takes 4 ids with 16-byte loads
+// and stores where ids and out lie on 16 bytes; four such groups per thread left
+// small calls with few workgroups (14,336 ids 2.4 us) and gained nothing on large
+// ones (22.8).
 template <bool kAligned>
 __global__ __launch_bounds__(256) void remap_ids_kernel(const int32_t* __restrict__ ids, int64_t count,
                                                         const int32_t* __restrict__ map, int map_len,
                                                         int32_t* __restrict__ out) {
     typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
-    const int64_t first = (int64_t(blockIdx.x) * (256 * kRemapPer) + threadIdx.x) * 4;
+    const int64_t first = (int64_t(blockIdx.x) * 256 + threadIdx.x) * 4;
     auto mapped = [&](int32_t id) { return map[min(max(id, 0), map_len - 1)]; };
-    if (kAligned && (int64_t(blockIdx.x) + 1) * (256 * kRemapPer * 4) <= count) {
-        i32x4 v[kRemapPer];
-#pragma unroll
-        for (int p = 0; p < kRemapPer; ++p) v[p] = *reinterpret_cast<const i32x4*>(ids + first + p * 1024);
-#pragma unroll
-        for (int p = 0; p < kRemapPer; ++p) {
-            const i32x4 r = {mapped(v[p][0]), mapped(v[p][1]), mapped(v[p][2]), mapped(v[p][3])};
-            *reinterpret_cast<i32x4*>(out + first + p * 1024) = r;
-        }
+    if (kAligned && first + 4 <= count) {
+        const i32x4 v = *reinterpret_cast<const i32x4*>(ids + first);
+        const i32x4 r = {mapped(v[0]), mapped(v[1]), mapped(v[2]), mapped(v[3])};
+        *reinterpret_cast<i32x4*>(out + first) = r;
         return;
     }
-    for (int p = 0; p < kRemapPer; ++p)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int64_t i = first + p * 1024 + e;
-            if (i < count) out[i] = mapped(ids[i]);
-        }
+    for (int e = 0; e < 4; ++e)
+        if (first + e < count) out[first + e] = mapped(ids[first + e]);
 }
 
 // Merge of two attention states over disjoint key sets (base-2 LSEs), as
@@ -1238,7 +1232,7 @@ int launch_merge(const void* oa, const float* sa, const void* ob, const float* s
 int launch_remap_ids(const int32_t* ids, int64_t count, const int32_t* map, int64_t map_len, int32_t* out,
                      hipStream_t stream) {
     if (count == 0) return 0;
-    constexpr int64_t kPerBlock = 256 * kRemapPer * 4;
+    constexpr int64_t kPerBlock = 256 * 4;
     const bool aligned = ((reinterpret_cast<uintptr_t>(ids) | reinterpret_cast<uintptr_t>(out)) & 15u) == 0;
     hipLaunchKernelGGL(aligned ? remap_ids_kernel<true> : remap_ids_kernel<false>,
                        dim3(static_cast<unsigned>((count + kPerBlock - 1) / kPerBlock)), dim3(256), 0, stream, ids,

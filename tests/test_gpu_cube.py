@@ -60,7 +60,7 @@ def test_cube_attention_c4_head():
 @pytest.mark.parametrize("count", [1, 4095, 4096, 4097, 12291])
 @pytest.mark.parametrize("skip", [0, 1])
 def test_remap_ids(count, skip):
-    """Whole workgroups of 4,096 ids, ragged ends and (skip 1) ids that do not lie
+    """Whole workgroups of 1,024 ids, ragged ends and (skip 1) ids that do not lie
     on 16 bytes; ids outside the map are clamped into it."""
     from ab_attention import _lib
 
