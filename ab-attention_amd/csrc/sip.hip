@@ -210,7 +210,9 @@ __device__ __forceinline__ void strided_partials(const R& rv, int pop, double& s
 // whatever its probes: the draw then finds it with a binary search over the
 // kept prefixes and a walk of fewer than `step` buckets. Each chunk checks
 // its boundary; a row where some threshold lands in a drop (sh.exact) makes
-// the reference's probes instead, each prefix rebuilt from the kept ones.
+// the reference's probes instead, each prefix rebuilt from the kept ones. So
+// does a row for which none of this holds: an infinite mass (the scale is 0, the
+// prefixes from it on NaN) or an offset outside [0, 1).
 template <int kWorkers, class R, class StageNext>
 __device__ __forceinline__ void coarse_draws(R& rv, double* coarse, SipShared& sh, float offset_u,
                                              int32_t* __restrict__ out_ids, float* __restrict__ out_w, int pop,
@@ -224,6 +226,7 @@ __device__ __forceinline__ void coarse_draws(R& rv, double* coarse, SipShared& s
     const int step = (cb + keep - 1) / keep;  // buckets between kept prefixes
     const double rd = static_cast<double>(residuals);
     const double offset = static_cast<double>(offset_u);
+    const bool regular = scale > 0.0 && offset >= 0.0 && offset < 1.0;
     double* kept = coarse;  // [256][keep]: chunk c's prefixes at buckets c*cb + j*step
     auto chunk_end = [&](int c) { return min((c + 1) * cb, buckets); };
     // prefix[c * cb]: the chunk's scan value, or R past the last residual
@@ -295,9 +298,10 @@ __device__ __forceinline__ void coarse_draws(R& rv, double* coarse, SipShared& s
                 }
             }
             // A drop at the boundary with the next chunk: does some threshold
-            // offset + s (0 <= s < residuals, exact in fp64) lie in it?
+            // offset + s (0 <= s < residuals, exact in fp64) lie in it? (Each
+            // loop ends within two steps: s is at most a few thousand.)
             const double next = first_prefix(t + 1);
-            if (vlast > next) {
+            if (regular && vlast > next) {
                 double s = ceil(next - offset);
                 while (s > 0.0 && offset + (s - 1.0) >= next) s -= 1.0;
                 while (offset + s < next) s += 1.0;
@@ -326,7 +330,7 @@ __device__ __forceinline__ void coarse_draws(R& rv, double* coarse, SipShared& s
         for (int bb = c * cb + j * step; bb < b; ++bb) cum = add_bucket(bb, cum);
         return cum;
     };
-    const bool exact = sh.exact != 0;
+    const bool exact = !regular || sh.exact != 0;
     const int per_round = kWorkers * kDraws;
     const int rounds = (residuals + per_round - 1) / per_round;
     for (int round = 0; round < rounds; ++round) {

@@ -93,3 +93,25 @@ def test_kept_prefix_rows(pop, rows, peak, oracle_mod):
     scores[1, pop // 2:] = 0.0  # draws fall in the first half, the last residuals at the floor
     offsets = rng.random(rows, dtype=np.float32)
     _assert_bit_exact(scores, offsets, 2272, oracle_mod)
+
+
+@pytest.mark.parametrize("pop", [8190, 24577, 29700, 41000])
+@pytest.mark.parametrize("case", ["infinite masses", "offsets outside [0, 1)"])
+def test_irregular_rows(pop, case, oracle_mod):
+    """Rows whose prefixes are not finite or whose thresholds do not start in
+    [0, 1) are answered as the reference's probes answer them in every storage
+    scheme: LDS, kept prefixes (24,577 and 29,700 blocks) and global memory.
+    Weights of infinite masses are NaN, of either sign."""
+    rng = np.random.default_rng(pop)
+    if case == "infinite masses":
+        scores, offsets = _local_masses(rng, 5, pop, 30.0), rng.random(5, dtype=np.float32)
+        for row, at in ((0, [0]), (1, [pop // 2]), (2, [pop - 1]), (3, [100, 101, pop // 3])):
+            scores[row, at] = np.inf
+    else:
+        offsets = np.array([1.0, 1.75, 600.0, -0.5, -3.25, 1e17, -1e17, np.inf, -np.inf, np.nan], np.float32)
+        scores = _local_masses(rng, len(offsets), pop, 30.0)
+    print(f"sip irregular rows pop={pop} {case}", flush=True)
+    ids_g, w_g = _run_gpu(scores, offsets, 500)
+    ids_o, w_o = oracle_mod.sip(scores, offsets, 500)
+    assert np.array_equal(ids_g, ids_o)
+    assert np.array_equal(w_g, w_o, equal_nan=True)
