@@ -154,6 +154,8 @@ def plan_heads(q: torch.Tensor, k: torch.Tensor, start: int, stop: int, offsets:
         _require(order.dtype == torch.int32 and order.is_contiguous() and order.device == q.device
                  and order.shape == (tokens,), "order must be int32 [tokens] on the q device")
     (q, q_stride), (k, k_stride) = _lib.in_place(q), _lib.in_place(k)
+    if batch > 1 and max(q_stride[0], k_stride[0]) >= _lib.MAX_STRIDE:
+        (q, q_stride), (k, k_stride) = _lib.in_one_batch(q, k)
     lib, address = _lib.load(), _lib.address
     with _lib.on(q.device):
         ws_bytes = lib.ab_ibcs_sip_workspace_bytes(stop - start, tokens)

@@ -181,3 +181,15 @@ def in_place(t: torch.Tensor):
         t = t.contiguous()
     _, heads, tokens, dim = t.shape  # not t.stride(): it may be anything where a size is 1
     return t, (heads * tokens * dim, tokens * dim, dim)
+
+
+MAX_STRIDE = 1 << 34
+
+
+def in_one_batch(*tensors):
+    """``in_place`` of tensors of which some (contiguous) one has a batch stride
+    of MAX_STRIDE elements or more: the library takes that only where every
+    tensor's batch items follow its heads at the head stride, so the others are
+    copied if need be."""
+    return tuple((t, stride) if stride[0] == t.shape[1] * stride[1] else in_place(t.contiguous())
+                 for t, stride in map(in_place, tensors))

@@ -41,6 +41,8 @@ def _run(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, ids, weights, sample
     kv_tokens, device = k.shape[2], q.device
     (q, q_stride), (k, k_stride), (v, v_stride) = _lib.in_place(q), _lib.in_place(k), _lib.in_place(v)
     out_stride = (heads * tokens * dim, tokens * dim, dim) if out is None else out.stride()[:3]
+    if batch > 1 and max(q_stride[0], k_stride[0], v_stride[0], out_stride[0]) >= _lib.MAX_STRIDE:
+        (q, q_stride), (k, k_stride), (v, v_stride) = _lib.in_one_batch(q, k, v)
     output = torch.empty_like(q, memory_format=torch.contiguous_format) if out is None else out
     lse = torch.empty((batch, heads, tokens), dtype=torch.float32, device=device) if return_lse else None
     lib, address = _lib.load(), _lib.address

@@ -88,16 +88,36 @@ int check_qk_shape(const char* what, int64_t bh, int64_t n) {
     return AB_OK;
 }
 
-// Strides (batch, head, token) in elements of a tensor whose rows start at
-// multiples of `align` elements.
-int tensor_layout(const char* what, const int64_t (&stride)[3], int64_t align, TensorLayout& out) {
-    for (int64_t s : stride)
-        if (s < 0 || s % align || s / 4 > int64_t(0xffffffff))
+bool stride_fits(int64_t s) { return s >= 0 && s / 4 <= int64_t(0xffffffff); }
+
+// Strides (batch, head, token) in elements of a [batch, heads, ...] tensor
+// whose rows start at multiples of `align` elements. The stride of one batch
+// item or head is not used, so it may be of any size.
+int tensor_layout(const char* what, const int64_t (&stride)[3], int64_t batch, int64_t heads, int64_t align,
+                  TensorLayout& out) {
+    const int64_t extent[3] = {batch, heads, 2};
+    uint32_t units[3];
+    for (int i = 0; i < 3; ++i) {
+        const int64_t s = stride[i];
+        if (s < 0 || s % align || (extent[i] > 1 && !stride_fits(s)))
             return set_error(AB_ERR_INVALID, "%s: strides must be multiples of %d elements from 0 to 2^34", what,
                              (int)align);
-    out = {static_cast<uint32_t>(stride[0] / 4), static_cast<uint32_t>(stride[1] / 4),
-           static_cast<uint32_t>(stride[2] / 4)};
+        units[i] = extent[i] > 1 ? static_cast<uint32_t>(s / 4) : 0u;
+    }
+    out = {units[0], units[1], units[2]};
     return AB_OK;
+}
+
+// A call whose batch stride is too large for a layout, in which every tensor's
+// batch items follow its heads at the head stride, has all its heads in one
+// batch item.
+template <class... Strides>
+void fold_batch(int64_t& batch, int64_t& heads, const Strides&... stride) {
+    if (batch <= 1 || heads <= 0 || batch > 65535 || heads > 65535 || (stride_fits(stride[0]) && ...)) return;
+    if (((stride_fits(stride[1]) && stride[0] == heads * stride[1]) && ...)) {
+        heads *= batch;
+        batch = 1;
+    }
 }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -325,9 +345,11 @@ int ab_plan(const ab_plan_args* a, void* stream) {
         a->head_count > a->batch * a->heads - a->first_head)
         return set_error(AB_ERR_INVALID, "ibcs_sip: head range outside the tensors");
     QkLayout layout;
-    if (int rc = tensor_layout("ibcs_sip", a->q_stride, 8, layout.q)) return rc;
-    if (int rc = tensor_layout("ibcs_sip", a->k_stride, 8, layout.k)) return rc;
-    layout.heads = divisor(static_cast<uint32_t>(a->heads));
+    int64_t batch = a->batch, heads = a->heads;
+    fold_batch(batch, heads, a->q_stride, a->k_stride);
+    if (int rc = tensor_layout("ibcs_sip", a->q_stride, batch, heads, 8, layout.q)) return rc;
+    if (int rc = tensor_layout("ibcs_sip", a->k_stride, batch, heads, 8, layout.k)) return rc;
+    layout.heads = divisor(static_cast<uint32_t>(heads));
     layout.first_head = static_cast<uint32_t>(a->first_head);
     return ibcs_sip_impl(a->q, a->k, layout, a->order, a->head_count, a->tokens, a->offsets, a->samples, a->workspace,
                          a->workspace_bytes, a->ids, a->log_weights, 0, stream);
@@ -448,12 +470,14 @@ size_t ab_prefill_workspace_bytes(int64_t batch_heads, int64_t q_tokens, int64_t
 int ab_prefill(const ab_prefill_args* a, void* stream) {
     if (!a) return set_error(AB_ERR_INVALID, "paged_prefill: null pointer");
     PrefillCall c{};
-    if (int rc = tensor_layout("paged_prefill", a->q_stride, 8, c.layout.q)) return rc;
-    if (int rc = tensor_layout("paged_prefill", a->k_stride, 8, c.layout.k)) return rc;
-    if (int rc = tensor_layout("paged_prefill", a->v_stride, 8, c.layout.v)) return rc;
-    if (int rc = tensor_layout("paged_prefill", a->out_stride, 4, c.layout.out)) return rc;
-    c.layout.heads = divisor(std::clamp<int64_t>(a->heads, 0, 65536));  // 65,536: rejected
-    c.batch = a->batch;
+    int64_t batch = a->batch, heads = a->heads;
+    fold_batch(batch, heads, a->q_stride, a->k_stride, a->v_stride, a->out_stride);
+    if (int rc = tensor_layout("paged_prefill", a->q_stride, batch, heads, 8, c.layout.q)) return rc;
+    if (int rc = tensor_layout("paged_prefill", a->k_stride, batch, heads, 8, c.layout.k)) return rc;
+    if (int rc = tensor_layout("paged_prefill", a->v_stride, batch, heads, 8, c.layout.v)) return rc;
+    if (int rc = tensor_layout("paged_prefill", a->out_stride, batch, heads, 4, c.layout.out)) return rc;
+    c.layout.heads = divisor(std::clamp<int64_t>(heads, 0, 65536));  // 65,536: rejected
+    c.batch = batch;
     c.q = a->q;
     c.k = a->k;
     c.v = a->v;

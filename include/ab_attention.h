@@ -92,7 +92,9 @@ int ab_ibcs_sip(const void *q, const void *k, const int32_t *order, int64_t batc
 /* ab_ibcs_sip of heads first_head .. first_head + head_count - 1 (of the
  * flattened batch * heads) of q, k [batch, heads, tokens, 128] with strides of
  * their own (batch, head, token; in elements, multiples of 8): only the heads'
- * rows, offsets and workspace are passed. */
+ * rows, offsets and workspace are passed. Limits: a batch or head stride that
+ * is used lies under 2^34 elements, unless every batch stride is heads * the
+ * head stride; a token stride under 2^27, and a head's extent under 64 GiB. */
 typedef struct ab_plan_args {
     const void *q, *k;
     const int32_t *order;
@@ -160,8 +162,11 @@ int ab_dense_prefill(const void *q, const void *k, const void *v, int64_t batch_
  * tokens, heads, 128] are read in place. lse is contiguous. A sparse call may
  * list tail_samples blocks (a multiple of 8) once for all rows, as if they
  * followed every row's own list: a prompt's blocks at weight 0 behind each
- * video row's sampled ones. ab_prefill_workspace_bytes counts them in samples. With a workspace, a call whose rows would
- * leave much of the GPU idle (a prompt's few query blocks over a whole video,
+ * video row's sampled ones. ab_prefill_workspace_bytes counts them in samples.
+ * Limits: a batch or head stride that is used lies under 2^34 elements, unless
+ * every tensor's batch stride is heads * its head stride; K's and V's token
+ * strides under 2^21 elements, and the extent of one of their heads under 4 GiB.
+ * With a workspace, a call whose rows would leave much of the GPU idle (a prompt's few query blocks over a whole video,
  * a short clip) splits each row's keys over several workgroups and adds up
  * their float32 partial results. That reorders float32 sums: bf16 outputs
  * differ in their last bit here and there (about 1e-4 of their norm). Rows

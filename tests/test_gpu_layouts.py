@@ -1,10 +1,12 @@
 """Q, K and V that are not contiguous are read where they lie (or copied where
 their rows cannot be): every public call equals the same call on contiguous
 tensors bit for bit, for each form of strides the dispatch distinguishes."""
+import contextlib
+
 import pytest
 import torch
 
-from ab_attention import _lib, apply_plan, attention, build_plan
+from ab_attention import _C, _lib, apply_plan, attention, build_plan, paged
 from ab_attention.video import apply_cube_plan, cube_plan, exact_attention
 
 B, H, N, GRID = 2, 3, 1920, (6, 16, 20)
@@ -42,6 +44,42 @@ def test_forms_read_in_place():
     assert _lib.in_place(still)[0].is_contiguous()  # a token stride of 0 is copied
 
 
+@pytest.mark.parametrize("batch,heads,tokens,q_tokens", [(1, 1024, 131072, 131072), (2, 1024, 131072, 131072),
+                                                         (2, 2048, 65536, 64), (1, 2048, 131072, 128)])
+def test_long_batch_strides(batch, heads, tokens, q_tokens, monkeypatch):
+    """Tensors of 2^27 tokens and more per batch item (their batch stride does
+    not fit 32 bits) pass the library's checks of strides: it stops at the
+    stand-in addresses put in here. A token-major q is copied beside them."""
+    lib, seen = _lib.load(), []
+
+    class Library:
+        ab_ibcs_sip_workspace_bytes = lib.ab_ibcs_sip_workspace_bytes
+        ab_prefill_workspace_bytes = lib.ab_prefill_workspace_bytes
+
+        @staticmethod
+        def ab_prefill(args, stream):
+            args.q = args.k = args.v = args.out = 4097
+            return seen.append((lib.ab_prefill(args, None), lib.ab_last_error())) or 0
+
+        @staticmethod
+        def ab_plan(args, stream):
+            args.q = args.k = args.offsets = args.ids = args.log_weights = 4097
+            return seen.append((lib.ab_plan(args, None), lib.ab_last_error())) or 0
+
+    monkeypatch.setattr(_lib, "load", lambda: Library)
+    monkeypatch.setattr(_lib, "on", lambda device: contextlib.nullcontext())
+    monkeypatch.setattr(_lib, "stream", lambda device: None)
+    like = dict(dtype=torch.bfloat16, device="meta")
+    k = torch.empty(batch, heads, tokens, 128, **like)
+    for q in (torch.empty(batch, heads, q_tokens, 128, **like),
+              torch.empty(batch, q_tokens, heads, 128, **like).transpose(1, 2)):
+        paged._run(q, k, k, None, None, _lib.PREFILL_DENSE, None, False)
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True)
+    rows = torch.empty(0, **like)
+    _C.plan_heads(k, k, 0, 1, rows, rows, rows, 32)
+    assert [rc for rc, _ in seen] == [1, 1, 1] and all(b"aligned" in message for _, message in seen), seen
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("form", ["token major", "token slice", "batch inside", "packed", "misaligned rows",
                                   "dims outside", "shared heads"])
@@ -67,3 +105,26 @@ def test_layouts_equal_contiguous(form, monkeypatch):
         for got, ref in zip(call(qs, ks, vs), call(q, k, v)):
             assert got.is_contiguous() and torch.equal(got, ref)
     torch.cuda.synchronize()
+
+
+@pytest.mark.gpu
+def test_folded_batch():
+    """K and V whose batch stride does not fit 32 bits, read where they lie as
+    heads of one batch item (51.5 GB of untouched memory around them)."""
+    print("folded batch", flush=True)
+    b, h, n, far = 2, 2, 256, 1 << 34
+    g = torch.Generator(device="cuda").manual_seed(5)
+    q, k, v = (torch.randn(b, h, n, 128, device="cuda", generator=g).to(torch.bfloat16) for _ in range(3))
+    memory = torch.empty(far + far // 2 + 2 * n * 128, dtype=torch.bfloat16, device="cuda")
+    views = [memory[i * n * 128:].as_strided((b, h, n, 128), (far, far // 2, 128, 1)) for i in range(2)]
+    for view, t in zip(views, (k, v)):
+        view.copy_(t)
+    want, out = exact_attention(q, k, v), torch.empty_like(q)
+    ws = torch.empty(_lib.load().ab_prefill_workspace_bytes(b * h, n, n, _lib.PREFILL_DENSE) + 16, dtype=torch.uint8,
+                     device="cuda")
+    near, wide = (h * n * 128, n * 128, 128), (far, far // 2, 128)
+    args = _lib.PrefillArgs(*(_lib.address(t) for t in (q, *views, None, None, None, out, None)), b, h, n, n,
+                            _lib.PREFILL_DENSE, near, wide, wide, near, None, None, 0, _lib.address(ws), ws.numel())
+    _lib.check(_lib.load().ab_prefill(args, _lib.stream(q.device)))
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)
