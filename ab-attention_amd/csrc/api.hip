@@ -396,9 +396,11 @@ int prefill_checked(PrefillCall call, size_t workspace_bytes, void* stream) {
     if (call.dense) call.samples = (call.kv_tokens / kKvBlock + 7) / 8 * 8;
     if (call.samples <= 0 || call.samples % 8)
         return set_error(AB_ERR_INVALID, "paged_prefill: samples must be a positive multiple of 8");
-    if (call.tail_samples < 0 || call.tail_samples % 8 || (call.dense && call.tail_samples) ||
-        call.samples + call.tail_samples > INT32_MAX / 4)
+    if (call.tail_samples < 0 || call.tail_samples % 8 || (call.dense && call.tail_samples))
         return set_error(AB_ERR_INVALID, "paged_prefill: the shared list must be a multiple of 8 blocks of a sparse call");
+    // The kernels address a row's list with 32-bit byte offsets.
+    if (call.samples >= (int64_t(1) << 30) || call.tail_samples >= (int64_t(1) << 30) - call.samples)
+        return set_error(AB_ERR_INVALID, "paged_prefill: a row lists fewer than 2^30 blocks");
     if (call.tail_samples && (!call.tail_ids || !call.tail_log_weights))
         return set_error(AB_ERR_INVALID, "paged_prefill: null pointer");
     if (!call.q || !call.k || !call.v || !call.out || (!call.dense && (!call.ids || !call.log_weights)))

@@ -152,3 +152,15 @@ def test_split_rounds_as_unsplit(heads, nq, nk, samples):
     (o, lse), (ref, ref_lse) = (_run(q, k, v, ids, w, None, split) for split in (True, False))
     assert np.linalg.norm(o - ref) / np.linalg.norm(ref) <= 4e-4
     assert np.abs(lse - ref_lse).max() <= 2e-5
+
+
+def test_longest_lists():
+    """Rows of up to 2^30 - 8 listed blocks are taken (these calls stop at the
+    misaligned output behind the check of the list), longer ones refused."""
+    lib, a, stride = _lib.load(), 4096, (1 << 20, 1 << 14, 128)
+    for samples, tail, message in ((1 << 29, 0, b"aligned"), ((1 << 30) - 8, 0, b"aligned"),
+                                   ((1 << 30) - 16, 8, b"aligned"), (1 << 30, 0, b"2^30"), ((1 << 30) - 8, 8, b"2^30"),
+                                   (8, (1 << 62), b"2^30")):
+        args = _lib.PrefillArgs(a, a, a, None, a, a, a + 1, None, 1, 1, 128, 128, samples, *4 * [stride], a, a, tail,
+                                None, 0)
+        assert lib.ab_prefill(args, None) == 1 and message in lib.ab_last_error(), (samples, tail)
