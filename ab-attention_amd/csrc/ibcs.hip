@@ -109,6 +109,9 @@ __device__ __forceinline__ float lane_distance(const f32x4 (&x)[32 / kLanes], co
     });
 }
 
+// v_perm_b32 selector of four zero bytes.
+constexpr uint32_t kZeroSelect = 0x0c0c0c0cu;
+
 // The same to a query row that every lane shares, read through the scalar
 // cache straight into scalar registers (packed: the row's 64 bf16 pairs in
 // global memory, wave-uniform address): no LDS reads, and no store and barrier
@@ -339,9 +342,15 @@ __global__ __launch_bounds__(kQueryBlock* kLanes) __attribute__((amdgpu_waves_pe
     min_d = INFINITY;
     int assign = 0;
     for (int slot = 0; slot < kCentroids; ++slot) {
-        const uint32_t coff = __builtin_amdgcn_readfirstlane(stored(__builtin_amdgcn_readfirstlane(center), q_row));
+        center = __builtin_amdgcn_readfirstlane(center);
+        const uint32_t coff = __builtin_amdgcn_readfirstlane(stored(center, q_row));
+        // A query past the end (only if NaNs leave no other maximum) is a zero row.
+        const bool inside = center < valid;
+        const uint32_t* center_words = reinterpret_cast<const uint32_t*>(qhead + coff);
         const float dist =
-            lane_distance_to_row<kLanes>(x, reinterpret_cast<const uint32_t*>(qhead + coff), part_sel);
+            inside || kLanes == 2
+                ? lane_distance_to_row<kLanes>(x, center_words, inside ? part_sel : kZeroSelect)
+                : chain_tree<kLanes>([&](int k, int r) { return x[k][r]; });
         if (live && dist < min_d) {
             min_d = dist;
             assign = slot;

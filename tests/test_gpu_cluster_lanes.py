@@ -46,3 +46,30 @@ def test_lanes_agree(n, ordered):
     torch.cuda.synchronize()
     for a, b in zip(few, whole):
         assert torch.equal(a, b[:len(a)])
+
+
+@pytest.mark.parametrize("valid", [4, 28, 36, 60])
+@pytest.mark.parametrize("heads", [5, 700])
+def test_nan_in_a_short_last_block(heads, valid):
+    """A NaN among fewer than 64 queries leaves no distance to the mean that is
+    a number: the farthest query is then a padding one, a zero row, and every
+    query falls to it (two lanes per query for 5 heads, one for 700)."""
+    n, lib = 128 + valid, _lib.load()
+    g = torch.Generator(device="cuda").manual_seed(valid)
+    q, k = (torch.randn(1, heads, n, 128, device="cuda", generator=g).to(torch.bfloat16) for _ in range(2))
+    q[0, 1, n - 1, 5] = float("nan")  # the last query
+    q[0, 2, n - 1] = float("nan")
+    q[0, 3, 128, 7] = float("nan")  # the block's first
+    cent = torch.empty(2 * heads, 8, 128, dtype=torch.bfloat16, device="cuda")
+    pops = torch.empty(2 * heads, 8, device="cuda")
+    pooled = torch.empty(heads, n // 4, 2, 128, dtype=torch.bfloat16, device="cuda")
+    print(f"cluster NaN heads={heads} valid={valid}", flush=True)
+    _lib.check(lib.ab_ibcs_cluster_pool(_lib.ptr(q), _lib.ptr(k), heads, n, _lib.ptr(cent), _lib.ptr(pops),
+                                        _lib.ptr(pooled), _lib.stream(q.device)))
+    torch.cuda.synchronize()
+    for head in (1, 2, 3):
+        row = 2 * head + 1
+        assert pops[row].tolist() == [valid] + 7 * [0]
+        assert bool((torch.isnan(cent[row, 0]) == torch.isnan(q[0, head, 128:]).any(0)).all())
+        assert not bool(cent[row, 1:].any())
+    assert bool((pops.sum(1) == torch.tensor([128, valid], device="cuda").repeat(heads)).all())
