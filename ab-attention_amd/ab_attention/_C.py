@@ -96,13 +96,13 @@ def sip(scores: torch.Tensor, offsets: torch.Tensor, ids: torch.Tensor, logs: to
 
 def ibcs_sip(q: torch.Tensor, k: torch.Tensor, offsets: torch.Tensor, ids: torch.Tensor, logs: torch.Tensor,
              order: torch.Tensor | None = None) -> None:
-    """``sip(ibcs(q, k), offsets, ids, logs)`` in one native call (ab_ibcs_sip).
+    """``sip(ibcs(q, k), offsets, ids, logs)`` in one native call (ab_plan).
 
     The same ids and weights bit for bit, without materialising the scores:
     one kernel computes each row's masses into LDS and samples the row. With
     ``order`` (int32 [tokens]) the tokens are read through that permutation,
-    as ``ibcs_ordered``. This is build_plan's per-chunk work
-    (reference: attention.py:65-75).
+    as ``ibcs_ordered``. ``plan_heads``, which this calls, is build_plan's
+    per-chunk work (reference: attention.py:65-75).
     """
     _require(q.is_cuda and k.is_cuda, "q and k must be CUDA tensors")
     _require(q.device == k.device, "q and k must use the same CUDA device")
@@ -128,13 +128,7 @@ def ibcs_sip(q: torch.Tensor, k: torch.Tensor, offsets: torch.Tensor, ids: torch
     if order is not None:
         _require(order.dtype == torch.int32 and order.is_contiguous() and order.device == q.device
                  and order.shape == (tokens,), "order must be int32 [tokens] on the q device")
-    lib = _lib.load()
-    with _lib.on(q.device):
-        ws_bytes = lib.ab_ibcs_sip_workspace_bytes(batch_heads, tokens)
-        workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
-        _lib.check(lib.ab_ibcs_sip(_lib.ptr(q), _lib.ptr(k), _lib.ptr(order), batch_heads, tokens,
-                                   _lib.ptr(offsets), samples, _lib.ptr(workspace), ws_bytes, _lib.ptr(ids),
-                                   _lib.ptr(logs), _lib.stream(q.device)))
+    plan_heads(q, k, 0, batch_heads, offsets, ids, logs, samples, order)
 
 
 def plan_heads(q: torch.Tensor, k: torch.Tensor, start: int, stop: int, offsets: torch.Tensor, ids: torch.Tensor,
@@ -145,11 +139,20 @@ def plan_heads(q: torch.Tensor, k: torch.Tensor, start: int, stop: int, offsets:
     projections need no copy (ab_plan)."""
     _require(q.is_cuda and k.is_cuda, "q and k must be CUDA tensors")
     _require(q.device == k.device, "q and k must use the same CUDA device")
+    _require(q.dim() == 4 and q.shape == k.shape, "q and k must have matching [batch, heads, tokens, 128] shapes")
     _require(q.dtype == torch.bfloat16 and k.dtype == torch.bfloat16, "IBCS requires bfloat16 q/k")
     _require(q.shape[3] == HEAD_DIM, "IBCS requires head_dim=128")
     batch, heads, tokens, _ = q.shape
     fine_blocks = tokens // KV_BLOCK
     _require(0 < fine_blocks <= MAX_KV_BLOCKS, "KV4 block count must be in [1, 32768]")
+    rows = (stop - start) * -(-tokens // QUERY_BLOCK)
+    _require(offsets.dtype == torch.float32 and ids.dtype == torch.int32 and logs.dtype == torch.float32,
+             "SIP requires float32 offsets/weights and int32 ids")
+    _require(offsets.numel() == rows and ids.numel() == rows * samples and logs.numel() == rows * samples,
+             "expected offsets [rows], ids/weights [rows,samples]")
+    _require(offsets.device == q.device and ids.device == q.device and logs.device == q.device
+             and offsets.is_contiguous() and ids.is_contiguous() and logs.is_contiguous(),
+             "SIP tensors must be contiguous and on the q device")
     if order is not None:
         _require(order.dtype == torch.int32 and order.is_contiguous() and order.device == q.device
                  and order.shape == (tokens,), "order must be int32 [tokens] on the q device")

@@ -75,8 +75,9 @@ def test_long_batch_strides(batch, heads, tokens, q_tokens, monkeypatch):
               torch.empty(batch, q_tokens, heads, 128, **like).transpose(1, 2)):
         paged._run(q, k, k, None, None, _lib.PREFILL_DENSE, None, False)
     monkeypatch.setattr(torch.Tensor, "is_cuda", True)
-    rows = torch.empty(0, **like)
-    _C.plan_heads(k, k, 0, 1, rows, rows, rows, 32)
+    rows = tokens // 128
+    _C.plan_heads(k, k, 0, 1, torch.empty(rows, device="meta"), torch.empty(rows, 32, device="meta", dtype=torch.int32),
+                  torch.empty(rows, 32, device="meta"), 32)
     assert [rc for rc, _ in seen] == [1, 1, 1] and all(b"aligned" in message for _, message in seen), seen
 
 
@@ -128,3 +129,28 @@ def test_folded_batch():
     _lib.check(_lib.load().ab_prefill(args, _lib.stream(q.device)))
     torch.cuda.synchronize()
     assert torch.equal(out, want)
+
+
+def test_plan_heads_checks(monkeypatch):
+    """Tensors that do not match each other never reach the library, which reads
+    and writes them by their strides and row counts."""
+    class Library:
+        ab_ibcs_sip_workspace_bytes = staticmethod(lambda *_: 16)
+        ab_plan = staticmethod(lambda *_: pytest.fail("reached the library"))
+
+    monkeypatch.setattr(_lib, "load", lambda: Library)
+    monkeypatch.setattr(_lib, "on", lambda device: contextlib.nullcontext())
+    monkeypatch.setattr(_lib, "stream", lambda device: None)
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True)
+    q = torch.empty(2, 3, 1000, 128, dtype=torch.bfloat16)
+    rows = 4 * 8  # heads 1 .. 4
+    good = dict(q=q, k=q, offsets=torch.empty(rows), ids=torch.empty(rows, 32, dtype=torch.int32),
+                logs=torch.empty(rows, 32))
+    for name, bad in (("k", q[:, :, :996]), ("k", q[:, :2]), ("k", q[0]), ("offsets", torch.empty(rows - 1)),
+                      ("offsets", torch.empty(2 * rows)[::2]), ("ids", torch.empty(rows - 1, 32, dtype=torch.int32)),
+                      ("ids", torch.empty(rows, 32)), ("logs", torch.empty(rows, 31)),
+                      ("logs", torch.empty(rows, 32, dtype=torch.float64)),
+                      ("logs", torch.empty(rows, 64)[:, ::2]), ("ids", torch.empty(rows, 32, device="meta"))):
+        a = dict(good, **{name: bad})
+        with pytest.raises(RuntimeError):
+            _C.plan_heads(a["q"], a["k"], 1, 5, a["offsets"], a["ids"], a["logs"], 32)
