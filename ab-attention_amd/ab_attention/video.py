@@ -118,6 +118,8 @@ def apply_cube_plan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, plan: Sam
     if descriptor.ndim != 3 or descriptor.shape != log_weights.shape or descriptor.shape[0] != rows \
             or descriptor.shape[-1] != 32:
         raise ValueError(f"descriptor and log_weights must share [{rows}, pages, 32] shape")
+    if descriptor.device != q.device or log_weights.device != q.device:
+        raise ValueError("descriptor and log_weights must be on the Q device")
     order, page_map = _cube_maps(grid, q.device)
     ids = _remap_ids(descriptor.reshape(rows, -1), page_map)
     return _prefill_ordered(q, k, v, order, ids, log_weights.reshape(rows, -1), return_lse=return_lse)
@@ -300,7 +302,11 @@ def hunyuan_attention(schedule: VideoAttention, layer: int, q: torch.Tensor, k: 
         q_video, k_video = q[:, :, video], k[:, :, video]
         if fused:
             plan = schedule.plan(layer, q_video, k_video)
-            rows = plan.descriptor.shape[0]
+            rows = q.shape[0] * q.shape[1] * math.ceil(video_tokens / _QUERY_BLOCK)
+            if plan.descriptor.shape != plan.log_weights.shape or plan.descriptor.shape[0] != rows:
+                raise ValueError(f"descriptor and log_weights must share a shape of {rows} rows")
+            if plan.descriptor.device != q.device or plan.log_weights.device != q.device:
+                raise ValueError("descriptor and log_weights must be on the Q device")
             text_ids, text_w = _dense_pages(1, prompt_tokens // _PAGE, q.device, offset=video_tokens // _PAGE)
             _prefill_kv(q_video, k[:, :, seen], v[:, :, seen], plan.descriptor.reshape(rows, -1),
                         plan.log_weights.reshape(rows, -1), tail=(text_ids, text_w, text_ids.shape[1]),

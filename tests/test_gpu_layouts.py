@@ -6,7 +6,7 @@ import contextlib
 import pytest
 import torch
 
-from ab_attention import _C, _lib, apply_plan, attention, build_plan, paged
+from ab_attention import _C, _lib, apply_plan, attention, build_plan, paged, video
 from ab_attention.video import apply_cube_plan, cube_plan, exact_attention
 
 B, H, N, GRID = 2, 3, 1920, (6, 16, 20)
@@ -154,3 +154,28 @@ def test_plan_heads_checks(monkeypatch):
         a = dict(good, **{name: bad})
         with pytest.raises(RuntimeError):
             _C.plan_heads(a["q"], a["k"], 1, 5, a["offsets"], a["ids"], a["logs"], 32)
+
+
+def test_plans_are_checked(monkeypatch):
+    """A plan on another device, or with other rows than the queries', never
+    reaches the library (a kept plan can be another video's)."""
+    class Library:
+        ab_prefill_workspace_bytes = staticmethod(lambda *_: 0)
+        ab_prefill = ab_remap_ids = staticmethod(lambda *_: pytest.fail("reached the library"))
+
+    monkeypatch.setattr(_lib, "load", lambda: Library)
+    monkeypatch.setattr(_lib, "on", lambda device: contextlib.nullcontext())
+    monkeypatch.setattr(_lib, "stream", lambda device: None)
+    monkeypatch.setattr(video, "_check_qkv", lambda *_: None)
+    monkeypatch.setattr(paged, "check_prefill_inputs", lambda *_: None)
+    q = torch.empty(2, 3, 4 * 16 * 16 + 32, 128, dtype=torch.bfloat16)
+    cube = q[:, :, :1024]
+    for device, rows, weight_rows in (("meta", 48, 48), ("cpu", 40, 40), ("cpu", 48, 40), ("cpu", 96, 96)):
+        plan = attention.SamplePlan(torch.zeros(rows, 2, 32, dtype=torch.int32, device=device),
+                                    torch.zeros(weight_rows, 2, 32))
+        schedule = video.VideoAttention(2)
+        schedule.step, schedule.plan = 12, lambda *_: plan
+        with pytest.raises(ValueError):
+            video.hunyuan_attention(schedule, 1, q, q, q, 1024, 32)
+        with pytest.raises(ValueError):
+            apply_cube_plan(cube, cube, cube, plan, (4, 16, 16))
