@@ -179,3 +179,83 @@ def test_plans_are_checked(monkeypatch):
             video.hunyuan_attention(schedule, 1, q, q, q, 1024, 32)
         with pytest.raises(ValueError):
             apply_cube_plan(cube, cube, cube, plan, (4, 16, 16))
+
+
+def _token_major(*tensors):
+    return tuple(t.transpose(1, 2).contiguous().transpose(1, 2) for t in tensors)
+
+
+def _split_parts(heads, nq, nk, samples):
+    return _lib.load().ab_prefill_workspace_bytes(heads, nq, nk, samples) > 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,n,samples,tail,split", [
+    (2, 2048, 512, 0, True), (1, 1000, 520, 24, True), (2, 1000, 504, 520, True),
+    (40, 1000, 128, 0, False), (40, 1000, 64, 16, False), (3, 12000, 2000, 8, False),
+])
+def test_strided_lists(heads, n, samples, tail, split):
+    """The sparse kernels on token-major K/V, with and without shared blocks, in
+    split calls (lists that end inside and beyond a batch of 512 blocks) and
+    unsplit ones."""
+    print(f"strided lists heads={heads} n={n} samples={samples} tail={tail}", flush=True)
+    assert _split_parts(heads, n, n, samples + tail) == split
+    g = torch.Generator(device="cuda").manual_seed(samples)
+    q, k, v = (torch.randn(1, heads, n, 128, device="cuda", generator=g).to(torch.bfloat16) for _ in range(3))
+    rows = heads * -(-n // 128)
+    ids = torch.randint(n // 4, (rows, samples), device="cuda", generator=g, dtype=torch.int32)
+    w = torch.rand(rows, samples, device="cuda", generator=g) * 3
+    shared = (None, None, 0)
+    if tail:
+        shared = (torch.randint(n // 4, (1, tail), device="cuda", generator=g, dtype=torch.int32),
+                  torch.zeros(1, tail, device="cuda"), tail)
+    want = paged._prefill_kv(q, k, v, ids, w, return_lse=True, tail=shared)
+    for form in (_token_major(q, k, v), (q, *_token_major(k), v)):
+        got = paged._prefill_kv(*form, ids, w, return_lse=True, tail=shared)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,nq,nk,split", [(40, 1000, 2000, False), (3, 12000, 1000, False), (2, 200, 4100, True)])
+def test_strided_dense(heads, nq, nk, split):
+    """The dense kernels on token-major tensors, split and not."""
+    print(f"strided dense heads={heads} nq={nq} nk={nk}", flush=True)
+    assert _split_parts(heads, nq, nk, _lib.PREFILL_DENSE) == split
+    g = torch.Generator(device="cuda").manual_seed(nk)
+    q = torch.randn(1, heads, nq, 128, device="cuda", generator=g).to(torch.bfloat16)
+    k, v = (torch.randn(1, heads, nk, 128, device="cuda", generator=g).to(torch.bfloat16) for _ in range(2))
+    want = exact_attention(q, k, v, return_lse=True)
+    for form in (_token_major(q, k, v), (q, k, *_token_major(v))):
+        for got, ref in zip(exact_attention(*form, return_lse=True), want):
+            assert torch.equal(got, ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads", [2, 24])
+@pytest.mark.parametrize("layout", ["contiguous", "token major"])
+def test_hunyuan_batches(heads, layout):
+    """Every part of the partition at two batch items, written into its slice of
+    the output, against the same parts computed from contiguous copies and
+    concatenated (2 heads split the video's rows, 24 do not)."""
+    n_video, prompt, padding, pages = 2560, 40, 24, 16
+    n, end = n_video + prompt + padding, n_video + prompt
+    print(f"hunyuan batches heads={heads} {layout}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(heads)
+    q, k, v = (torch.randn(2, heads, n, 128, device="cuda", generator=g).to(torch.bfloat16) for _ in range(3))
+    part = lambda t, *s: t[:, :, slice(*s)].contiguous()
+    plan = build_plan(part(q, n_video), part(k, n_video), sample_pages=pages)
+    rows = plan.descriptor.shape[0]
+    assert _split_parts(2 * heads, n_video, end, 32 * pages + 16) == (heads == 2)
+    text = [t.expand(rows, -1) for t in video._dense_pages(1, prompt // 4, "cuda", offset=n_video // 4)]
+    ids, w = (torch.cat([p.reshape(rows, -1), t], 1) for p, t in zip(plan, text))
+    seen = part(k, end), part(v, end)
+    rest = exact_attention(part(q, end, n), part(k, end, n), part(v, end, n))
+    sparse = torch.cat([paged._prefill_kv(part(q, n_video), *seen, ids, w),
+                        exact_attention(part(q, n_video, end), *seen), rest], 2)
+    dense = torch.cat([exact_attention(part(q, end), *seen), rest], 2)
+    given = (q, k, v) if layout == "contiguous" else _token_major(q, k, v)
+    schedule = video.VideoAttention(pages)
+    assert torch.equal(video.hunyuan_attention(schedule, 1, *given, n_video, prompt), dense)
+    schedule.step, schedule.plan = 12, lambda *_: plan
+    assert torch.equal(video.hunyuan_attention(schedule, 1, *given, n_video, prompt), sparse)
+    torch.cuda.synchronize()
