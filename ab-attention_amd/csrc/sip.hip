@@ -30,8 +30,9 @@
 //     (before the row's results are stored). Certainty is marked by the sign
 //     bit of the LDS copy, as the reference negates its copy.
 //   - sip_kept_kernel (rows whose masses fit in LDS but not beside all the
-//     prefixes): the same with some of the prefixes kept (coarse_draws);
-//   - sip_global_kernel (larger rows): one row per workgroup, the row is
+//     prefixes, where sip_kept_pays): the same with some of the prefixes kept
+//     (coarse_draws);
+//   - sip_global_kernel (the others): one row per workgroup, the row is
 //     re-read from L2 by each pass, LDS holds the prefixes and a certainty
 //     bitmask.
 // The fused plan (sip_fused_kernel, below) computes each row's masses into
@@ -1009,6 +1010,21 @@ int launch_sip_fused(const void* lse, const float* pops, const float* lse_max, c
                                            force_exact, stream);
 }
 
+// Whether rows that fit sip_kept_kernel are faster there than in
+// sip_global_kernel, which holds two rows per CU at once. With at least 8 kept
+// prefixes per chunk (rows of up to 36,000 blocks, draws that walk at most 5
+// buckets) they are while each CU has one row, or draws few samples: many leave
+// blocks with certainty, whose passes over the row wait on barriers that a second
+// row per CU would fill. Global / kept in us, 1,500 rows of 32,768 blocks: 239 / 187
+// with 4,096 samples, 254 / 233 with 6,000, 577 / 651 with 8,000 (256 rows: 153 /
+// 119); of 24,600: 178 / 147 and 414 / 435 with 4,096 and 6,000. With 4 or 2 of them
+// the draws walk 10 or 20 buckets: 8 rows of 39,000 blocks 33 / 33 with 1,024
+// samples, 36 / 50 with 2,272; of 37,000 31 / 26 and 34 / 36.
+bool sip_kept_pays(int64_t rows, int64_t population, int64_t samples) {
+    if (coarse_keep(population) < 8) return samples <= 1024;
+    return rows <= device_cu_count() || 5 * samples <= population;
+}
+
 int launch_sip(const float* scores, const float* offsets, int64_t rows, int64_t population, int64_t samples,
                int32_t* ids, float* logw, hipStream_t stream) {
     if (!sip_fits(population))
@@ -1026,7 +1042,8 @@ int launch_sip(const float* scores, const float* offsets, int64_t rows, int64_t 
         if (per_thread <= 16) return persistent(sip_lds_kernel<16>, lds_bytes);
         if (per_thread <= 24) return persistent(sip_lds_kernel<24>, lds_bytes);
     }
-    if (sip_fused_fits(population)) return persistent(sip_kept_kernel<16>, sip_fused_lds_bytes(population, true));
+    if (sip_fused_fits(population) && sip_kept_pays(rows, population, samples))
+        return persistent(sip_kept_kernel<16>, sip_fused_lds_bytes(population, true));
     const size_t bytes = sip_lds_bytes(population, false);
     if (int rc = ensure_lds_limit(reinterpret_cast<const void*>(sip_global_kernel), static_cast<int>(bytes)))
         return rc;

@@ -115,3 +115,14 @@ def test_irregular_rows(pop, case, oracle_mod):
     ids_o, w_o = oracle_mod.sip(scores, offsets, 500)
     assert np.array_equal(ids_g, ids_o)
     assert np.array_equal(w_g, w_o, equal_nan=True)
+
+
+@pytest.mark.parametrize("pop,rows,samples", [(37001, 8, 1000), (39001, 8, 1024), (39001, 8, 1025), (24577, 8, 6000),
+                                              (24577, 300, 6000), (32768, 300, 6553), (32768, 300, 6554)])
+def test_kept_prefix_rule(pop, rows, samples, oracle_mod):
+    """Both sides of the rule that gives long rows to kept prefixes or to global
+    memory: few kept prefixes per chunk, and many samples with more rows than
+    CUs."""
+    rng = np.random.default_rng(pop + samples)
+    scores = _local_masses(rng, 16, pop, 3.0)[np.arange(rows) % 16]
+    _assert_bit_exact(scores, rng.random(rows, dtype=np.float32), samples, oracle_mod)
