@@ -33,7 +33,7 @@ namespace {
 // key tokens. One workgroup of 128 threads per (query block, head): thread i
 // owns query i (its row kept in 128 VGPRs as f32); thread d owns dim d in the
 // mean, which reads the block from LDS one 64-row half at a time (17 KB of LDS
-// and 150 VGPRs: three waves per SIMD).
+// and 164 VGPRs: three waves per SIMD).
 //
 // Bound by VALU issue on a full chip (nine distance passes of 256 sub/fma per
 // query are over half of it) and by the chain of passes, reductions and
@@ -116,16 +116,20 @@ constexpr uint32_t kZeroSelect = 0x0c0c0c0cu;
 // cache straight into scalar registers (packed: the row's 64 bf16 pairs in
 // global memory, wave-uniform address): no LDS reads, and no store and barrier
 // to publish the row first. With two lanes per query each picks its half of a
-// pair with one v_perm_b32 (sel).
+// pair with one v_perm_b32 (sel). Not inside: a zero row in its place, by the
+// same instructions with zeros as their selector, mask and factor (a branch to
+// code of its own took plans of 1,300 blocks from 112.3 to 112.9 us).
 template <int kLanes>
 __device__ __forceinline__ float lane_distance_to_row(const f32x4 (&x)[32 / kLanes],
-                                                     const uint32_t* __restrict__ packed, uint32_t sel) {
+                                                     const uint32_t* __restrict__ packed, uint32_t sel, bool inside) {
+    const uint32_t hi_mask = inside ? 0xffff0000u : 0u, lo_factor = inside ? 0x10000u : 0u;
+    if (!inside) sel = kZeroSelect;
     return chain_tree<kLanes>([&](int k, int r) {
         const int dim = leaf_chain(k);
         const uint32_t pair = packed[(dim >> 1) + 16 * r];
         const float c = kLanes == 2 ? __uint_as_float(__builtin_amdgcn_perm(pair, pair, sel))
-                        : (dim & 1) ? bf16_hi(pair)
-                                    : bf16_lo(pair);
+                        : (dim & 1) ? __uint_as_float(pair & hi_mask)
+                                    : __uint_as_float(pair * lo_factor);
         return x[k][r] - c;
     });
 }
@@ -345,12 +349,8 @@ __global__ __launch_bounds__(kQueryBlock* kLanes) __attribute__((amdgpu_waves_pe
         center = __builtin_amdgcn_readfirstlane(center);
         const uint32_t coff = __builtin_amdgcn_readfirstlane(stored(center, q_row));
         // A query past the end (only if NaNs leave no other maximum) is a zero row.
-        const bool inside = center < valid;
-        const uint32_t* center_words = reinterpret_cast<const uint32_t*>(qhead + coff);
-        const float dist =
-            inside || kLanes == 2
-                ? lane_distance_to_row<kLanes>(x, center_words, inside ? part_sel : kZeroSelect)
-                : chain_tree<kLanes>([&](int k, int r) { return x[k][r]; });
+        const float dist = lane_distance_to_row<kLanes>(x, reinterpret_cast<const uint32_t*>(qhead + coff), part_sel,
+                                                        center < valid);
         if (live && dist < min_d) {
             min_d = dist;
             assign = slot;
