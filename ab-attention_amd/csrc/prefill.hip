@@ -58,9 +58,11 @@
 // v_mfma_f32_16x16x32_bf16 tiles (see there).
 // Calls with too few rows to fill the chip split each row's tiles over several
 // workgroups (kSplit, prefill_parts), whose float32 partial results
-// combine_kernel adds up. All parts of a row share its reference, so a split
-// row differs from an unsplit one by the order of its float32 sums only, unless
-// it leaves the fast pass (then P rounds to bf16 against other references).
+// combine_kernel adds up. In the fast pass the parts after the first take the
+// row's reference, from the logits of its first tile (`lead` in the kernels), so
+// that every p has the same bf16 bits however a row is split, and a split row
+// differs from an unsplit one by the order of its float32 sums only. Rows that
+// leave the fast pass round P against other references.
 #include <algorithm>
 #include <type_traits>
 
@@ -83,6 +85,12 @@ constexpr int kIdsOffset = 2 * kRing * kTileBytes;             // 2 batch buffer
 constexpr int kWeightsOffset = kIdsOffset + 2 * kBatchBytes;   // 2 batch buffers of weights
 constexpr int kVoteOffset = kWeightsOffset + 2 * kBatchBytes;  // 4 words: fast-pass votes
 constexpr int kLdsBytes = kVoteOffset + 16;                    // 72 KiB + 16 B
+// Split rows: ids and weights (32 bytes each) of the row's first tile, in a
+// transfer's 1 KiB, and the stage that its K takes before the loop: V's last,
+// which V(3) fills in step 0.
+constexpr int kLeadOffset = kLdsBytes;
+constexpr int kSplitLdsBytes = kLeadOffset + 1024;
+constexpr int kLeadStage = 2 * kRing - 1;
 constexpr int kGroupOps = 4;                                   // transfers per wave per step
 constexpr int64_t kRowsPerLaunch = 11000;                      // see launch_prefill
 // Limits of a split (prefill_parts): units that give each CU one workgroup (at
@@ -101,7 +109,7 @@ constexpr float kFastRange = 64.0f;
 constexpr int kDenseVoteOffset = 2 * kRing * kTileBytes;
 constexpr int kDenseLdsBytes = kDenseVoteOffset + 16;          // 64 KiB + 16 B
 
-static_assert(kLdsBytes * 2 <= 160 * 1024, "two workgroups per CU must fit in LDS");
+static_assert(kSplitLdsBytes * 2 <= 160 * 1024, "two workgroups per CU must fit in LDS");
 static_assert(kDenseLdsBytes * 2 <= 160 * 1024, "two dense workgroups per CU must fit in LDS");
 
 typedef short i16x4 __attribute__((ext_vector_type(4)));
@@ -250,16 +258,11 @@ __device__ __forceinline__ bool unit_slot(const RowGrid& g, const Divisor& heads
     us.part = static_cast<int>(head_part - flat * parts);
     return true;
 }
-// Tiles of part `part` of `parts` (parts <= tiles, so none is empty). Every part
-// but the first leads with the row's tile 0: it sets the fast pass's reference,
-// as in the unsplit pass, so that every p = 2^(z - m) has the same bf16 bits
-// however a row is split, and adds nothing itself. `lead` is 1 for these parts;
-// tile 0 of the unit is the row's tile 0 and tile u > 0 the row's u + skip.
-__device__ __forceinline__ void part_tiles(int tiles, int parts, int part, int& lead, int& skip, int& count) {
-    const int first = static_cast<int>(int64_t(tiles) * part / parts);
-    lead = part > 0 ? 1 : 0;
-    skip = first - lead;
-    count = static_cast<int>(int64_t(tiles) * (part + 1) / parts) - skip;
+// Tiles [first, first + count) of part `part` of `parts` (parts <= tiles, so
+// none is empty).
+__device__ __forceinline__ void part_tiles(int tiles, int parts, int part, int& first, int& count) {
+    first = static_cast<int>(int64_t(tiles) * part / parts);
+    count = static_cast<int>(int64_t(tiles) * (part + 1) / parts) - first;
 }
 
 // Partial results of the split kernels, in the caller's workspace: per unit
@@ -301,10 +304,10 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_kernel(
     touch_arguments(q, layout, grid);
 
     UnitSlot rs;
-    int lead = 0, skip = 0, tiles = (lists.samples + (kTail ? lists.tail : 0)) / kTilePages;
+    int tile0 = 0, tiles = (lists.samples + (kTail ? lists.tail : 0)) / kTilePages;
     if constexpr (kSplit) {
         if (!unit_slot(grid, layout.heads, partials.parts, rs)) return;
-        part_tiles(tiles, partials.parts, rs.part, lead, skip, tiles);
+        part_tiles(tiles, partials.parts, rs.part, tile0, tiles);
     } else {
         if (!row_slot(grid, layout.heads, rs)) return;
     }
@@ -347,7 +350,7 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_kernel(
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             uint32_t at = min(uint32_t(b) * kBatchBytes + i * 1024u + 16u * lane, unit_bytes - 16u);
-            if constexpr (kSplit) at += at >= kTilePages * 4u ? static_cast<uint32_t>(skip) * (kTilePages * 4u) : 0u;
+            if constexpr (kSplit) at += static_cast<uint32_t>(tile0) * (kTilePages * 4u);
             const uint32_t dst = (b & 1) * kBatchBytes + i * 1024u;
             if constexpr (kTail) {
                 const uint32_t row_bytes = static_cast<uint32_t>(lists.samples) * 4u;
@@ -560,8 +563,21 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_kernel(
         // are in; K(4) goes into K(0)'s stage only after every wave has read
         // it. The last eight transfers before step 0 are then K(3), V(1), V(2),
         // K(4), as step 0's wait expects.
-        if (wave == 0) issue_batch(0);
+        const bool lead = kSplit && !kSafe && tile0 > 0;
+        if (wave == 0) {
+            if (lead)
+                dma16(reinterpret_cast<const char*>(lane & 2 ? static_cast<const void*>(row_w) : row_ids) + 16 * (lane & 1),
+                      lds0 + kLeadOffset);
+            issue_batch(0);
+        }
         wait_and_barrier<0>();
+        if (lead) {
+            const u32x2 raw = *reinterpret_cast<const u32x2*>(smem + kLeadOffset + 8 * wave);
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+                dma16(kbase, page_offset<kPacked>(uint32_t(min(max(static_cast<int>(raw[e]), 0), fb - 1)), k_page) + k_src[e],
+                      lds0 + kLeadStage * kTileBytes + (2 * wave + e) * kPageBytes);
+        }
         {
 #pragma unroll
             for (int u = 0; u < 3; ++u) {
@@ -581,51 +597,65 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_kernel(
             dma_v(2, iv2[0], 0);
             dma_v(2, iv2[1], 1);
         }
-        const u32x2 ik4 = load_ids(4);
-        u32x2 idk = load_ids(5), idv = load_ids(3);
-        wait_and_barrier<10>();  // K(0), K(1) in; 10 newer transfers may be in flight
         f32x16 s0, s1;
         u32x4 ka[8];
-        {
+        // S of the tile in a stage of K's ring (or, from kRing on, V's).
+        auto compute_s = [&](int stage) {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) ka[j] = read_k(0, j);
+            for (int j = 0; j < 8; ++j)
+                ka[j] = *reinterpret_cast<const lds_u32x4*>(static_cast<uintptr_t>(k_abs[j] + stage * kTileBytes));
 #pragma unroll
             for (int r = 0; r < 16; ++r) s0[r] = 0.f;
 #pragma unroll
             for (int j = 0; j < 8; ++j)
                 s0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, ka[j]), bq[j], s0, 0, 0, 0);
+        };
+        // The query's reference from its largest logit, over both lane halves; a
+        // query without a finite one fails the pass.
+        auto set_reference = [&](float mx) {
+            const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+            mx = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+            started = mx > -INFINITY;
+            m_run = started ? mx : 0.f;
+        };
+        if (lead) {
+            wait_and_barrier<14>();  // the leading tile is in; the 14 transfers after it may be in flight
+            compute_s(kLeadStage);
+            const float* ws = reinterpret_cast<const float*>(smem + kLeadOffset + 4 * kTilePages);
+            float mx = -INFINITY;
 #pragma unroll
-            for (int j = 0; j < 8; ++j) ka[j] = read_k(1, j);
+            for (int r = 0; r < 16; ++r) mx = fmaxf(mx, __builtin_fmaf(s0[r], scale_log2, ws[2 * (r >> 2) + half]));
+            set_reference(mx);
         }
+        const u32x2 ik4 = load_ids(4);
+        u32x2 idk = load_ids(5), idv = load_ids(3);
+        wait_and_barrier<10>();  // K(0), K(1) in; 10 newer transfers may be in flight
+        compute_s(0);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) ka[j] = read_k(1, j);
         wait_and_barrier<63>();  // every wave's reads of K(0) are done (no transfer wait)
         dma_k(4, ik4[0], 0);
         dma_k(4, ik4[1], 1);
-        // Logits of S(0) (against reference 0).
+        // Logits of S(0), against reference 0 or the leading tile's.
         float w0[4], mx = -INFINITY;
         load_weights(0, w0);
+        if (lead) {
+#pragma unroll
+            for (int g = 0; g < 4; ++g) w0[g] -= m_run;
+        }
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             s0[r] = __builtin_fmaf(s0[r], scale_log2, w0[r >> 2]);
             mx = fmaxf(mx, s0[r]);
         }
         if constexpr (!kSafe) {
-            // The query's reference is the maximum of its first tile, over
-            // both lane halves; a query without a finite logit there fails the
-            // pass.
-            const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
-            mx = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
-            started = mx > -INFINITY;
-            m_run = started ? mx : 0.f;
+            if (!lead) {
+                set_reference(mx);
 #pragma unroll
-            for (int r = 0; r < 16; ++r) s0[r] -= m_run;
-            mx = started ? -INFINITY : INFINITY;
-        }
-        if constexpr (kSplit) {
-            if (lead) {  // tile 0 belongs to the first part
-#pragma unroll
-                for (int r = 0; r < 16; ++r) s0[r] = -INFINITY;
-                if constexpr (kSafe) mx = -INFINITY;
+                for (int r = 0; r < 16; ++r) s0[r] -= m_run;
+                mx = -INFINITY;
             }
+            if (!started) mx = INFINITY;
         }
         // Four steps per iteration: t is a multiple of 4 there, so every ring
         // stage (u & 3) is a compile-time constant and the LDS addresses fold
@@ -721,10 +751,10 @@ __global__ __launch_bounds__(kPfThreads, 2) void dense_kernel(
     extern __shared__ __align__(16) unsigned char smem[];
     touch_arguments(q, layout, grid);
     UnitSlot rs;
-    int lead = 0, skip = 0, tiles = samples / kTilePages;
+    int tile0 = 0, tiles = samples / kTilePages;
     if constexpr (kSplit) {
         if (!unit_slot(grid, layout.heads, partials.parts, rs)) return;
-        part_tiles(samples / kTilePages, partials.parts, rs.part, lead, skip, tiles);
+        part_tiles(samples / kTilePages, partials.parts, rs.part, tile0, tiles);
     } else {
         if (!row_slot(grid, layout.heads, rs)) return;
     }
@@ -768,13 +798,11 @@ __global__ __launch_bounds__(kPfThreads, 2) void dense_kernel(
         const int P = lane >> 3, sl = (lane >> 1) & 3, h = lane & 1;
         v_src[e] = uint32_t(sl) * v_token + uint32_t(2 * (P ^ e) + h) * 16u;
     }
-    // The row's tile of the unit's tile u; past the end, the last one.
-    auto row_tile = [&](int u) { return kSplit && u == 0 ? 0 : skip + min(u, tiles - 1); };
     // This wave's two pages of tile u, clamped into the head; tiles past the
     // row's end read its last tile (their transfers only keep the per-step
     // count uniform).
     auto load_ids = [&](int u) {
-        const int id = row_tile(u) * kTilePages + 2 * wave;
+        const int id = (tile0 + min(u, tiles - 1)) * kTilePages + 2 * wave;
         const u32x2 c = {uint32_t(min(id, fb - 1)), uint32_t(min(id + 1, fb - 1))};
         return c;
     };
@@ -788,7 +816,7 @@ __global__ __launch_bounds__(kPfThreads, 2) void dense_kernel(
     // The weights of this lane's keys in tile u: pages lg and 4 + lg, 0 inside
     // K/V and -inf past its end.
     auto load_weights = [&](int u, float (&wv)[2]) {
-        const int uc = row_tile(u);
+        const int uc = tile0 + min(u, tiles - 1);
 #pragma unroll
         for (int kt = 0; kt < 2; ++kt) wv[kt] = uc * kTilePages + 4 * kt + lg < fb ? 0.f : -INFINITY;
     };
@@ -946,7 +974,14 @@ __global__ __launch_bounds__(kPfThreads, 2) void dense_kernel(
         // K(0) and K(1) are in; K(4) goes into K(0)'s stage only after every
         // wave has read it. The last eight transfers before step 0 are then
         // K(3), V(1), V(2), K(4), as step 0's wait expects.
+        const bool lead = kSplit && !kSafe && tile0 > 0;
         wait_and_barrier<0>();
+        if (lead) {
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+                dma16(kbase, page_offset<kPacked>(uint32_t(min(2 * wave + e, fb - 1)), k_page) + k_src[e],
+                      lds0 + kLeadStage * kTileBytes + (2 * wave + e) * kPageBytes);
+        }
         {
 #pragma unroll
             for (int u = 0; u < 3; ++u) {
@@ -966,14 +1001,14 @@ __global__ __launch_bounds__(kPfThreads, 2) void dense_kernel(
             dma_v(2, iv2[0], 0);
             dma_v(2, iv2[1], 1);
         }
-        const u32x2 ik4 = load_ids(4);
-        u32x2 idk = load_ids(5), idv = load_ids(3);
-        wait_and_barrier<10>();  // K(0), K(1) in; 10 newer transfers may be in flight
         f32x4 s0[4], s1[4];
         u32x4 ka[8];
-        {
+        // S of the tile in a stage of K's ring (or, from kRing on, V's).
+        auto compute_s = [&](int stage) {
 #pragma unroll
-            for (int f = 0; f < 8; ++f) ka[f] = read_k(0, f);
+            for (int f = 0; f < 8; ++f)
+                ka[f] = *reinterpret_cast<const lds_u32x4*>(
+                    static_cast<uintptr_t>(k_abs[f & 3] + stage * kTileBytes + (f >> 2) * 4096));
 #pragma unroll
             for (int c = 0; c < 4; ++c)
 #pragma unroll
@@ -984,49 +1019,63 @@ __global__ __launch_bounds__(kPfThreads, 2) void dense_kernel(
                 s0[2 * kt + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, ka[4 * kt + ks]),
                                                                          bq[j][ks], s0[2 * kt + j], 0, 0, 0);
             }
+        };
+        // Each query's reference from its largest logit, over its four lanes; a
+        // query without a finite one fails the pass.
+        auto set_reference = [&](float (&mx)[2]) {
+            max_over_rows(mx[0], mx[1]);
 #pragma unroll
-            for (int f = 0; f < 8; ++f) ka[f] = read_k(1, f);
+            for (int j = 0; j < 2; ++j) {
+                const bool started = mx[j] > -INFINITY;
+                m_run[j] = started ? mx[j] : 0.f;
+                thr[j] = started ? kSlack : -INFINITY;
+            }
+        };
+        if (lead) {
+            wait_and_barrier<14>();  // the leading tile is in; the 14 transfers after it may be in flight
+            compute_s(kLeadStage);
+            float mx[2] = {-INFINITY, -INFINITY};
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const float w = 4 * (c >> 1) + lg < fb ? 0.f : -INFINITY;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) mx[c & 1] = fmaxf(mx[c & 1], __builtin_fmaf(s0[c][r], scale_log2, w));
+            }
+            set_reference(mx);
         }
+        const u32x2 ik4 = load_ids(4);
+        u32x2 idk = load_ids(5), idv = load_ids(3);
+        wait_and_barrier<10>();  // K(0), K(1) in; 10 newer transfers may be in flight
+        compute_s(0);
+#pragma unroll
+        for (int f = 0; f < 8; ++f) ka[f] = read_k(1, f);
         wait_and_barrier<63>();  // every wave's reads of K(0) are done (no transfer wait)
         dma_k(4, ik4[0], 0);
         dma_k(4, ik4[1], 1);
-        // Logits of S(0) (against reference 0).
+        // Logits of S(0), against reference 0 or the leading tile's.
         float w0[2], mx[2] = {-INFINITY, -INFINITY};
         load_weights(0, w0);
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
+            const float w = lead ? w0[c >> 1] - m_run[c & 1] : w0[c >> 1];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                s0[c][r] = __builtin_fmaf(s0[c][r], scale_log2, w0[c >> 1]);
+                s0[c][r] = __builtin_fmaf(s0[c][r], scale_log2, w);
                 mx[c & 1] = fmaxf(mx[c & 1], s0[c][r]);
             }
         }
         if constexpr (!kSafe) {
-            // Each query's reference is the maximum of its first tile, over its
-            // four lanes; a query without a finite logit there fails the pass.
-            max_over_rows(mx[0], mx[1]);
-            bool all_started = true;
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                const bool started = mx[j] > -INFINITY;
-                all_started = all_started && started;
-                m_run[j] = started ? mx[j] : 0.f;
-                thr[j] = started ? kSlack : -INFINITY;
-#pragma unroll
-                for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) s0[2 * kt + j][r] -= m_run[j];
-            }
-            mx[0] = all_started ? -INFINITY : INFINITY;
-        }
-        if constexpr (kSplit) {
-            if (lead) {  // tile 0 belongs to the first part
+            if (lead) {
+                mx[0] = fmaxf(mx[0], mx[1]);
+            } else {
+                set_reference(mx);
 #pragma unroll
                 for (int c = 0; c < 4; ++c)
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) s0[c][r] = -INFINITY;
-                if constexpr (kSafe) mx[0] = mx[1] = -INFINITY;
+                    for (int r = 0; r < 4; ++r) s0[c][r] -= m_run[c & 1];
+                mx[0] = -INFINITY;
             }
+            if (thr[0] != kSlack || thr[1] != kSlack) mx[0] = INFINITY;
         }
         int t = 0;
         for (; t + 3 < tiles; t += 4) {
@@ -1256,22 +1305,22 @@ int64_t prefill_launch_slots(int64_t bh, int64_t n) {
 // 512 (two workgroups per CU); the time of a tile step then grows from 0.49 us
 // (a few lone workgroups) over 0.58 (one on every CU) to 0.88 (two), measured
 // on dense calls of 24 to 3,072 rows, and a unit costs its tiles plus a
-// prologue and epilogue worth about 8, and its leading tile where the row is
-// split (0.1 to 0.6 us of the times below). Splitting adds combine_kernel (6 us)
+// prologue and epilogue worth about 8, with the row's reference where it is
+// split (0.1 to 0.3 us). Splitting adds combine_kernel (6 us)
 // and its 128 KiB of traffic per unit (0.03 us); dense units cannot run faster
 // than their K/V arrive (5.5 TB/s). More units than 512 lose: their rounds do
 // not start together and share less of what they read (640 dense rows of 512
 // tiles: 680 us, in 2 parts 618, but 640 sparse rows of 128: 211 and 238), so
 // calls of more than 256 rows never split. Measured, unsplit and at the parts
-// this picks: dense 24 rows x 3,715 tiles 1,862 -> 278 us, 48 x 3,721 1,819 ->
-// 384, 4 x 1,024 504 -> 37, 256 x 512 264 -> 240; sparse 64 x 64 38.8 -> 24.4,
-// 16 x 128 69.2 -> 22.5.
+// this picks: dense 24 rows x 3,715 tiles 1,874 -> 299 us, 48 x 3,721 1,815 ->
+// 415, 4 x 1,024 504 -> 37, 256 x 512 282 -> 251; sparse 64 x 64 37.9 -> 24.7,
+// 16 x 128 68.9 -> 21.7.
 int prefill_parts(int64_t rows, int64_t tiles, int64_t kv_bytes) {
     constexpr double kSetupSteps = 8, kCombine = 6, kUnitTraffic = 0.03, kBytesPerUs = 5.5e6, kGain = 0.95;
     auto cost = [&](int64_t parts) {
         const double units = double(rows * parts), wide = double(kPartUnits);
         const double step = units <= wide ? 0.49 + 0.09 * units / wide : 0.58 + 0.30 * (units / wide - 1.0);
-        const double run = step * (double((tiles + parts - 1) / parts) + kSetupSteps + (parts > 1 ? 1.0 : 0.0));
+        const double run = step * (double((tiles + parts - 1) / parts) + kSetupSteps);
         return std::max(run, double(kv_bytes) / kBytesPerUs) + (parts > 1 ? kCombine + kUnitTraffic * units : 0.0);
     };
     int best = 1;
@@ -1319,7 +1368,7 @@ int launch_prefill(const PrefillCall& c, hipStream_t stream) {
     const int64_t per_xcd = (qb + 7) / 8;
     if (rows == 0) return 0;
     const int parts = c.workspace ? call_parts(dense, bh, n, n_kv, samples + c.tail_samples) : 1;
-    const int lds_bytes = dense ? kDenseLdsBytes : kLdsBytes;
+    const int lds_bytes = dense ? kDenseLdsBytes : parts > 1 ? kSplitLdsBytes : kLdsBytes;
     const int fb = static_cast<int>(n_kv / kKvBlock), s = static_cast<int>(samples);
     const dim3 block(kPfThreads);
     uint16_t* out = static_cast<uint16_t*>(c.out);
