@@ -125,7 +125,7 @@ def _prefill_kv(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, ids: torch.Te
 
 def _prefill_dense(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, return_lse: bool = False, out=None):
     """Dense attention of q bf16 [B,H,Nq,128] over every key of k/v bf16
-    [B,H,Nk,128] (Nk % 4 == 0) on the dense kernel (ab_dense_prefill); the
+    [B,H,Nk,128] (Nk % 4 == 0) on the dense kernel (ab_prefill); the
     page list is implicit, so nothing of size rows x blocks is built. Shapes
     are checked by the callers."""
     return _run(q, k, v, None, None, _lib.PREFILL_DENSE, None, return_lse, out=out)

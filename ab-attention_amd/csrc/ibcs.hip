@@ -63,7 +63,7 @@ __host__ __device__ constexpr int leaf_chain(int k) {
 }
 // Rows are held in leaf order, the four dims of a chain together: element
 // [k][r] of a row is dim leaf_chain(k) + 32r. A query's row sits in 32 f32x4
-// registers that way, and the centre row in LDS (one 16-byte read or write
+// registers that way, and the mean's row in LDS (one 16-byte read or write
 // per chain).
 __device__ __forceinline__ int center_pos(int d) { return 4 * leaf_chain(d & 31) + (d >> 5); }
 

@@ -86,8 +86,8 @@ def test_degenerate_rows(oracle_mod):
                                            (39001, 8, 30.0), (41000, 8, 30.0)])
 def test_kept_prefix_rows(pop, rows, peak, oracle_mod):
     """Rows whose masses fit in LDS without all prefixes, from the smallest to
-    the largest, several per workgroup (600 rows), and one past them (the
-    global-memory path)."""
+    the largest, several per workgroup (600 rows), and one past them; 39,001 and
+    41,000 blocks take this many samples from global memory."""
     rng = np.random.default_rng(pop)
     scores = _local_masses(rng, rows, pop, peak)
     scores[1, pop // 2:] = 0.0  # draws fall in the first half, the last residuals at the floor
