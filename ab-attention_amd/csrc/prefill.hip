@@ -973,15 +973,18 @@ __global__ __launch_bounds__(kPfThreads, 2) void dense_kernel(
         // Prologue: K(0..3) and V(0..2); S(0) and K(1) into registers once
         // K(0) and K(1) are in; K(4) goes into K(0)'s stage only after every
         // wave has read it. The last eight transfers before step 0 are then
-        // K(3), V(1), V(2), K(4), as step 0's wait expects.
+        // K(3), V(1), V(2), K(4), as step 0's wait expects. A leading tile comes
+        // with Q, before them, so that its logits are computed while they are in
+        // flight (4 heads x 256 queries over 4,000 keys: 18.25 us with its
+        // transfers just before theirs, 18.15 now, 17.9 without the tile).
         const bool lead = kSplit && !kSafe && tile0 > 0;
-        wait_and_barrier<0>();
         if (lead) {
 #pragma unroll
             for (int e = 0; e < 2; ++e)
                 dma16(kbase, page_offset<kPacked>(uint32_t(min(2 * wave + e, fb - 1)), k_page) + k_src[e],
                       lds0 + kLeadStage * kTileBytes + (2 * wave + e) * kPageBytes);
         }
+        wait_and_barrier<0>();
         {
 #pragma unroll
             for (int u = 0; u < 3; ++u) {
@@ -1032,7 +1035,6 @@ __global__ __launch_bounds__(kPfThreads, 2) void dense_kernel(
             }
         };
         if (lead) {
-            wait_and_barrier<14>();  // the leading tile is in; the 14 transfers after it may be in flight
             compute_s(kLeadStage);
             float mx[2] = {-INFINITY, -INFINITY};
 #pragma unroll
